@@ -87,7 +87,7 @@ def sampler_params(state):
 def build(force: bool = False) -> None:
     """Compile the oracle (and the reference build when its sources exist)."""
     subprocess.run(["make", "-s", "-C", HERE] + (["-B"] if force else []), check=True)
-    if os.path.isdir(REFERENCE_ROOT):
+    if os.path.isdir(os.path.join(REFERENCE_ROOT, "projects")):  # an empty mount holds no sources
         subprocess.run(["make", "-s", "-j8", "-C", os.path.join(HERE, "ref")] + (["-B"] if force else []), check=True)
 
 
