@@ -59,23 +59,24 @@ IFX_HD float u2f(uint32_t u) { return __builtin_bit_cast(float, u); }
 // (AMD) mantissa bits, exact exponent scaling, sub-normal results flushed to
 // signed zero, zero and sub-normal inputs give signed infinity, infinities
 // give signed zero, NaNs come back quieted.
+// Without branches: the table's entry for the mantissa with 127 - e added to its
+// exponent, replaced where that leaves the normal range.
 IFX_HD float rcp_ps(float x, int model) {
-    uint32_t b = f2u(x);
-    uint32_t sign = b & 0x80000000u;
-    uint32_t e = (b >> 23) & 0xffu;
-    if (e == 0u) return u2f(sign | 0x7f800000u);
-    if (e == 255u) return (b & 0x7fffffu) ? u2f(b | 0x400000u) : u2f(sign);
+    const uint32_t b = f2u(x);
+    const uint32_t sign = b & 0x80000000u;
+    const int32_t e = (int32_t)((b >> 23) & 0xffu);
     const bool amd = model == kRcpAmd;
-    const uint32_t idx = amd ? (b >> 11) & 0xfffu : (b >> 12) & 0x7ffu;
+    const uint32_t idx = (b >> (amd ? 11 : 12)) & (amd ? 0xfffu : 0x7ffu);
 #if defined(__HIP_DEVICE_COMPILE__)
     const uint32_t* tab = amd ? kRcpTableAmd : kRcpTable;
 #else
     const uint32_t* tab = amd ? kRcpTableAmdHost : kRcpTableHost;
 #endif
-    uint32_t t = tab[idx];
-    int re = (int)((t >> 23) & 0xffu) + 127 - (int)e;
-    if (re <= 0) return u2f(sign);
-    return u2f(sign | (t & 0x7fffffu) | ((uint32_t)re << 23));
+    const int32_t t = (int32_t)tab[idx] + ((127 - e) * 0x800000);  // exponents 126 or 127 in the table
+    uint32_t r = t < 0x800000 ? 0u : (uint32_t)t;                  // sub-normal results flush to zero
+    r = e == 0 ? 0x7f800000u : r;
+    r = e == 255 ? ((b & 0x7fffffu) ? (b & 0x7fffffffu) | 0x400000u : 0u) : r;
+    return u2f(sign | r);
 }
 
 // ApproxReciprocalNR256: r = rcp(x); (r + r) - x * (r * r).

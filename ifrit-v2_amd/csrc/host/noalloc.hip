@@ -113,11 +113,11 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     if (!base) return setError(err);
 
     // everything the draw reads from the renderer's own buffers and sizes, restored on every exit
-    DevBuf* const bufs[] = {&vtx_, &idx_, &clip_, &recs_[0], &recs_[1], &recs_[2], &recs_[3], &recs_[4], &recs_[5],
-                            &bary_, &binQueue_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_, &bigList_,
-                            &ctr_, &groupBounds_, &groupOut_, &clipList_, &statPart_, &items_, &tilePartial_,
+    DevBuf* const bufs[] = {&vtx_, &idx_, &recs_[0], &recs_[1], &recs_[2], &recs_[3], &recs_[4], &recs_[5],
+                            &bary_, &binFront_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_,
+                            &ctr_, &groupBounds_, &clipList_, &statPart_, &items_, &tilePartial_,
                             &multiList_, &partials_, &visDepth_, &visSlot_, &visClass_, &rgba8_, &rgba32f_,
-                            &texDesc_, &viewDev_, &tileView_, &shadeView_, &viewCtr_, &planSums_, &swapped_};
+                            &texDesc_, &viewDev_, &tileView_, &shadeView_, &viewCtr_, &swapped_};
     constexpr size_t kBufs = sizeof(bufs) / sizeof(bufs[0]);
     struct Restore {
         TileRasterRenderer& r;
@@ -206,32 +206,34 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
         b.ptr = A.take(n);
         b.bytes = n;
     };
+    // first what starts at zero: counters, the tile maps (all view 0), the tile counts
     put(ctr_, sizeof(DeviceCounters));
-    put(viewDev_, sizeof(ViewDesc));
     put(viewCtr_, sizeof(ViewCounters));
     put(tileView_, std::max<size_t>(1, tiles) * 2);
     put(shadeView_, std::max<size_t>(1, shadeTiles_) * 2);
+    put(binCount_, tiles * 8);
+    const size_t zeroed = A.used;
+    put(viewDev_, sizeof(ViewDesc));
     put(texDesc_, std::max<size_t>(1, textures_.size()) * sizeof(TexDesc));
     put(groupBounds_, std::max<size_t>(1, groups) * 32);
-    put(groupOut_, std::max<size_t>(1, groups));
-    put(clip_, (size_t)nverts_ * 16);
     for (int k = 0; k < 6; k++) put(recs_[k], slots * 16);
-    put(bary_, slots * 32);
-    put(binQueue_, slots * 16);
+    // 16 bytes a vertex and 48 a record slot are set aside for the fans' vertex weights and the
+    // geometry kernel's outputs, which never need more: what a draw may hold does not depend on how
+    // they are laid out
+    const size_t weights = ((size_t)clipCap_ * 32 + 255) & ~(size_t)255;
+    put(bary_, weights);
+    put(binFront_, std::max(frontBytes(), (size_t)nverts_ * 16 + slots * 48 + std::max<size_t>(1, groups) - weights));
     put(slotOf_, (size_t)std::max(1, ntri) * 4);
     if (needSwapFlags()) put(swapped_, slots);
     put(clipList_, (size_t)clipCap_ * 4);
-    put(statPart_, ((size_t)(ntri + 1023) / 1024 + 2 * (size_t)rasterGrid() + 2) * 8);
+    put(statPart_, (2 * (size_t)rasterGrid() + 2) * 8);
     put(items_, (size_t)itemCap_ * 16);
     put(tilePartial_, tiles * 4);
-    put(planSums_, ((tiles + kPlanTiles - 1) / kPlanTiles + 1) * 6 * 4);
-    put(multiList_, tiles * 8);
+    put(multiList_, tiles * 4);
     put(partials_, (size_t)partialCap_ * 256 * samples_ * 8);
-    put(binCount_, tiles * 4);
     put(binStart_, tiles * 4);
     put(binCursor_, tiles * 4);
     put(binList_, (size_t)binCap_ * 4);
-    put(bigList_, (size_t)bigCap_ * 4);
     put(visSlot_, px * samples_ * 4);
     put(visClass_, px);
     if (!A.fits())
@@ -266,8 +268,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     if (!ok(hipMemcpy(viewDev_.ptr, &vd, sizeof(vd), hipMemcpyHostToDevice), "iftrDrawNoAlloc view table") ||
         !ok(hipMemcpy(texDesc_.ptr, td.data(), td.size() * sizeof(TexDesc), hipMemcpyHostToDevice),
             "iftrDrawNoAlloc texture table") ||
-        !ok(hipMemsetAsync(tileView_.ptr, 0, tileView_.bytes, stream_), "iftrDrawNoAlloc tile map") ||
-        !ok(hipMemsetAsync(shadeView_.ptr, 0, shadeView_.bytes, stream_), "iftrDrawNoAlloc shading map"))
+        !ok(hipMemsetAsync(base, 0, zeroed, stream_), "iftrDrawNoAlloc counters and tile maps"))
         return;
     if (boundsTris_ > 0)
         launch_group_bounds(vtx_.as<float>(), stride_, nverts_, idx_.as<int>(), ntri, groupBounds_.as<float4>(), stream_);

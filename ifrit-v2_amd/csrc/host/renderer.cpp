@@ -51,17 +51,24 @@ void DevBuf::release() {
     bytes = 0;
 }
 
+bool TileRasterRenderer::ensureZeroed(DevBuf& b, size_t n) {
+    const void* had = b.ptr;
+    const size_t bytes = b.bytes;
+    if (!b.ensure(n)) return false;
+    return (b.ptr == had && b.bytes == bytes) || hipMemsetAsync(b.ptr, 0, b.bytes, stream_) == hipSuccess;
+}
+
 TileRasterRenderer::TileRasterRenderer() {}
 
 TileRasterRenderer::~TileRasterRenderer() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     dropGraph();
-    for (DevBuf* b : {&vtx_, &idx_, &clip_, &recs_[0], &recs_[1], &recs_[2], &recs_[3], &recs_[4], &recs_[5], &bary_, &binQueue_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_,
-                      &bigList_, &ctr_, &clipList_, &statPart_, &items_, &tilePartial_, &multiList_, &partials_, &visId_, &visDepth_, &visSlot_, &visClass_, &rgba8_, &rgba32f_, &texDesc_, &nnParams_, &nnGrads_, &nnM_, &nnV_,
+    for (DevBuf* b : {&vtx_, &idx_, &clip_, &recs_[0], &recs_[1], &recs_[2], &recs_[3], &recs_[4], &recs_[5], &bary_, &binFront_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_,
+                      &ctr_, &clipList_, &statPart_, &items_, &tilePartial_, &multiList_, &partials_, &visId_, &visDepth_, &visSlot_, &visClass_, &rgba8_, &rgba32f_, &texDesc_, &nnParams_, &nnGrads_, &nnM_, &nnV_,
                       &nnPacked_, &nnQinfo_, &lat32_, &latGrad_, &latM_, &latV_, &lat16_, &nnData_, &nnFeat_, &nnCount_,
                       &nnLoss_, &nnEvalIn_, &nnEvalOut_, &nnGradPart_, &viewDev_, &tileView_, &shadeView_,
-                      &groupBounds_, &groupOut_, &swapped_, &scissorDev_,
-                      &viewCtr_, &digest_, &planSums_, &polyKeys_, &meshVtx_, &meshIdx_})
+                      &groupBounds_, &swapped_, &scissorDev_,
+                      &viewCtr_, &digest_, &polyKeys_, &meshVtx_, &meshIdx_})
         b->release();
     for (DevBuf& b : bufSlots_) b.release();
     for (auto& t : textures_)
@@ -99,7 +106,7 @@ void TileRasterRenderer::Init() {
     if (!ok(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate")) return;
     for (auto& e : ev_)
         if (!ok(hipEventCreate(&e), "hipEventCreate")) return;
-    if (!ctr_.ensure(sizeof(DeviceCounters))) setError("hipMalloc counters");
+    if (!ensureZeroed(ctr_, sizeof(DeviceCounters))) setError("hipMalloc counters");
     std::string err;
     if (!noalloc_register_device(&err)) setError(err);
     int dev = 0, cus = 0;
@@ -785,28 +792,36 @@ bool TileRasterRenderer::prepare(int indexCount) {
     partialCap_ = std::max<unsigned>(partialCap_, std::max(256u, binCap_ / (8u * part)));
     // point and line records take one slot per index (3 per triangle)
     const size_t slots = std::max(((size_t)ntri + clipCap_) * nv, polygonMode_ != 0 ? (size_t)indexCount : 0);
+    // vertex weights: of the clip fans, or of every point and line
+    const size_t fans = std::max((size_t)clipCap_ * nv, polygonMode_ != 0 ? (size_t)indexCount : 0);
     const bool wantFloat = batch_.empty() && ((fb_ && !fb_->color.empty() && fb_->color[0]) || floatOut_ ||
                                               blend_.blendEnable);
-    bool okAll = clip_.ensure((size_t)nverts_ * 16 * nv) &&
-                 groupOut_.ensure(std::max<size_t>(1, (size_t)(boundsTris_ + kGroupTris - 1) / kGroupTris) * nv) &&
+    // clip positions are kept for the point and line modes only (a host vertex shader uploaded its own)
+    bool okAll = (polygonMode_ == 0 || clip_.ensure((size_t)nverts_ * 16 * nv)) &&
                  recs_[0].ensure(slots * 16) &&
                  recs_[1].ensure(slots * 16) && recs_[2].ensure(slots * 16) && recs_[3].ensure(slots * 16) &&
-                 recs_[4].ensure(slots * 16) && recs_[5].ensure(slots * 16) && bary_.ensure(slots * 32) &&
-                 binQueue_.ensure(slots * 16) && slotOf_.ensure((size_t)std::max(1, ntri) * 4 * nv) &&
+                 recs_[4].ensure(slots * 16) && recs_[5].ensure(slots * 16) && bary_.ensure(fans * 32) &&
+                 binFront_.ensure(frontBytes()) && slotOf_.ensure((size_t)std::max(1, ntri) * 4 * nv) &&
                  (!needSwapFlags() || swapped_.ensure(slots)) &&
                  clipList_.ensure((size_t)clipCap_ * 4 * nv) &&
-                 statPart_.ensure(((size_t)(ntri + 255) / 256 * nv + 2 * (size_t)rasterGrid() + 2) * 8) &&
+                 statPart_.ensure((2 * (size_t)rasterGrid() + 2) * 8) &&
                  items_.ensure((size_t)itemCap_ * 16) && tilePartial_.ensure(tiles * 4) &&
-                 planSums_.ensure(((tiles + kPlanTiles - 1) / kPlanTiles + 1) * 6 * 4) &&
-                 multiList_.ensure(tiles * 8) && partials_.ensure((size_t)partialCap_ * 256 * samples_ * 8) &&
-                 binCount_.ensure(tiles * 4) && binStart_.ensure(tiles * 4) && binCursor_.ensure(tiles * 4) &&
-                 binList_.ensure((size_t)binCap_ * 4) && bigList_.ensure((size_t)bigCap_ * 4) &&
+                 multiList_.ensure(tiles * 4) && partials_.ensure((size_t)partialCap_ * 256 * samples_ * 8) &&
+                 ensureZeroed(binCount_, tiles * 8) && binStart_.ensure(tiles * 4) && binCursor_.ensure(tiles * 4) &&
+                 binList_.ensure((size_t)binCap_ * 4) &&
                  visId_.ensure(ps * 4) && visDepth_.ensure(ps * 4) && visSlot_.ensure(ps * 4) &&
                  visClass_.ensure(px) && rgba8_.ensure(px * 4) && (!wantFloat || rgba32f_.ensure(px * 16)) &&
                  (polygonMode_ == 0 || polyKeys_.ensure(px * 8));
     if (!okAll) {
         setError("device allocation failed");
         return false;
+    }
+    if (countersDirty_) {
+        if (!ok(hipMemsetAsync(binCount_.ptr, 0, binCount_.bytes, stream_), "tile counts") ||
+            !ok(hipMemsetAsync(ctr_.ptr, 0, sizeof(DeviceCounters), stream_), "counters") ||
+            !ok(hipMemsetAsync(viewCtr_.ptr, 0, viewCtr_.bytes, stream_), "view counters"))
+            return false;
+        countersDirty_ = false;
     }
     if (texDescDirty_) {
         // the pool pointer the kernels offset is the lowest texture allocation, so that every texture's
@@ -895,7 +910,7 @@ bool TileRasterRenderer::layoutViews(int ntri) {
     const bool descChanged = d.size() != viewDesc_.size() ||
                              std::memcmp(d.data(), viewDesc_.data(), d.size() * sizeof(ViewDesc)) != 0;
     if (descChanged) {
-        if (!viewDev_.ensure(d.size() * sizeof(ViewDesc)) || !viewCtr_.ensure(d.size() * sizeof(ViewCounters)))
+        if (!viewDev_.ensure(d.size() * sizeof(ViewDesc)) || !ensureZeroed(viewCtr_, d.size() * sizeof(ViewCounters)))
             return setError("hipMalloc views"), false;
         // the previous draw may still read the table
         if (!ok(hipStreamSynchronize(stream_), "view table") ||
@@ -933,7 +948,57 @@ Views TileRasterRenderer::deviceViews() const {
     V.ctr = viewCtr_.as<ViewCounters>();
     V.count = (int)viewDesc_.size();
     V.slotsPerView = (unsigned)curTris_ + clipCap_;
+    V.waves = geom_waves(curTris_);
     return V;
+}
+
+VertexInput TileRasterRenderer::vertexInput() const {
+    // a host vertex shader's clip positions were uploaded to clip_; an emitted list holds its own
+    if (hostVs_) return VertexInput{clip_.as<float>(), 4, 0};
+    return VertexInput{vtx_.as<float>(), stride_,
+                       clipAt_ >= 0 ? clipAt_ : vs_.desc.kind == IFHIP_VS_CLIP_PASSTHROUGH ? 0 : -1};
+}
+
+// Scatter workgroups: four waves each, a wave per geometry wave up to 16384
+// (64 per compute unit), then several geometry waves per wave; 64 workgroups
+// at least, for the clip fans and deferred triangles.
+void TileRasterRenderer::scatterShape(int* grid, int* regions) const {
+    const size_t R = (size_t)geom_waves(curTris_) * std::max<size_t>(1, viewDesc_.size());
+    *regions = (int)std::min<size_t>(64, std::max<size_t>(1, R / 16384));
+    *grid = (int)std::min<size_t>(65536, std::max<size_t>(64, (R + 4 * *regions - 1) / (4 * *regions)));
+}
+
+namespace {
+constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+}  // namespace
+
+size_t TileRasterRenderer::frontBytes() const {
+    const size_t nv = std::max<size_t>(1, viewDesc_.size()), W = (size_t)geom_waves(curTris_) * nv;
+    int grid, regions;
+    scatterShape(&grid, &regions);
+    return align256(W * 64 * sizeof(uint2)) + align256(W * 64 * sizeof(uint4)) + align256(W * sizeof(WaveInfo)) +
+           align256((size_t)clipCap_ * nv * sizeof(uint2)) + align256((size_t)bigCap_ * sizeof(uint4)) +
+           align256((size_t)grid * 8);
+}
+
+BinBufs TileRasterRenderer::binBufs() const {
+    const size_t nv = std::max<size_t>(1, viewDesc_.size()), W = (size_t)geom_waves(curTris_) * nv;
+    uint8_t* p = binFront_.as<uint8_t>();
+    BinBufs b{};
+    b.entry = reinterpret_cast<uint2*>(p);
+    p += align256(W * 64 * sizeof(uint2));
+    b.entry1 = reinterpret_cast<uint4*>(p);
+    p += align256(W * 64 * sizeof(uint4));
+    b.waves = reinterpret_cast<WaveInfo*>(p);
+    p += align256(W * sizeof(WaveInfo));
+    b.fanBox = reinterpret_cast<uint2*>(p);
+    p += align256((size_t)clipCap_ * nv * sizeof(uint2));
+    b.big = reinterpret_cast<uint4*>(p);
+    b.cnt = binCount_.as<unsigned>();
+    b.start = binStart_.as<unsigned>();
+    b.cursor = binCursor_.as<unsigned>();
+    b.list = binList_.as<unsigned>();
+    return b;
 }
 
 TriRecs TileRasterRenderer::recPtrs() const {
@@ -943,14 +1008,14 @@ TriRecs TileRasterRenderer::recPtrs() const {
 
 StatPartials TileRasterRenderer::statPtrs() const {
     StatPartials st{};
-    // setup workgroups: 1024 threads for up to four views, 256 beyond
-    const int nv = (int)std::max<size_t>(1, viewDesc_.size()), per = nv <= 4 ? 1024 : 256;
-    st.setupBlocks = (curTris_ + per - 1) / per * nv;
+    int regions;
+    scatterShape(&st.setupBlocks, &regions);
     st.rasterBlocks = rasterGrid();
     unsigned long long* base = statPart_.as<unsigned long long>();
-    st.setupAssembled = base;
-    st.rasterFrags = base + st.setupBlocks;
-    st.rasterCovs = base + st.setupBlocks + st.rasterBlocks;
+    st.setupAssembled = reinterpret_cast<unsigned long long*>(
+        reinterpret_cast<uint8_t*>(binBufs().big) + align256((size_t)bigCap_ * sizeof(uint4)));
+    st.rasterFrags = base;
+    st.rasterCovs = base + st.rasterBlocks;
     return st;
 }
 
@@ -1017,22 +1082,17 @@ void TileRasterRenderer::enqueue(bool clear) {
         if (stageTiming_ && !capturing_) (void)hipEventRecord(ev_[i], s);
     };
     mark(0);
-    // triangle groups outside a view are marked by the vertex launch and skipped by setup
-    const bool cullGroups = !hostVs_ && vs_.desc.kind == IFHIP_VS_TRANSFORM && groupOut_.ptr;
-    const int groups = (boundsTris_ + kGroupTris - 1) / kGroupTris;
-    if (hostVs_)
-        launch_reset(binCount_.as<unsigned>(), binCursor_.as<unsigned>(), tiles, V, ctr_.as<DeviceCounters>(), s);
-    else  // the vertex launch also clears the counters
-        launch_vertex(vtx_.as<float>(), stride_, nverts_, V,
-                      clipAt_ >= 0 ? clipAt_ : vs_.desc.kind == IFHIP_VS_CLIP_PASSTHROUGH ? 0 : -1,
-                      clip_.as<float4>(), binCount_.as<unsigned>(), binCursor_.as<unsigned>(), tiles,
-                      ctr_.as<DeviceCounters>(), groupBounds_.as<float4>(), groups,
-                      cullGroups ? groupOut_.as<unsigned char>() : nullptr, s);
-    mark(1);
+    const VertexInput vin = vertexInput();
     if (polygonMode_ != 0) {
+        if (hostVs_)
+            launch_reset(V, ctr_.as<DeviceCounters>(), s);
+        else
+            launch_vertex(vin, nverts_, V, clip_.as<float4>(), ctr_.as<DeviceCounters>(), s);
+        mark(1);
         enqueuePolygons(clear, V);
         return;
     }
+    mark(1);
     SetupParams sp{};
     sp.ntri = curTris_;
     sp.nverts = nverts_;
@@ -1042,21 +1102,26 @@ void TileRasterRenderer::enqueue(bool clear) {
     sp.clipCap = clipCap_;
     sp.invTileWidth = ifx::rcp_nr_ss(16.0f, rcpModel_);
     sp.rcpModel = rcpModel_;
-    sp.groupOut = cullGroups ? groupOut_.as<unsigned char>() : nullptr;
-    sp.groups = groups;
-    launch_setup(sp, V, clip_.as<float4>(), idx_.as<int>(), recPtrs(), bary_.as<float4>(), binQueue_.as<uint4>(),
-                 slotOf_.as<unsigned>(), clipList_.as<unsigned>(), statPtrs(), ctr_.as<DeviceCounters>(), s);
+    // triangle groups outside a view are skipped whole
+    sp.groupBounds = vin.clipAt < 0 ? groupBounds_.as<float4>() : nullptr;
+    sp.groups = (boundsTris_ + kGroupTris - 1) / kGroupTris;
+    sp.bigCap = bigCap_;
+    sp.bigThreshold = bigThreshold_;
+    const BinBufs bins = binBufs();
+    launch_geometry(sp, V, vin, idx_.as<int>(), recPtrs(), bary_.as<float4>(), bins, slotOf_.as<unsigned>(),
+                    clipList_.as<unsigned>(), ctr_.as<DeviceCounters>(), s);
     mark(2);
     RasterQueue q{items_.as<uint4>(), tilePartial_.as<int>(), multiList_.as<unsigned>(),
-                  partials_.as<unsigned long long>(), planSums_.as<unsigned>(), itemCap_, partialCap_, rasterGrid(),
+                  partials_.as<unsigned long long>(), itemCap_, partialCap_, binCap_, rasterGrid(),
                   numCUs_ * rasterGroupsPerCU_, partShift_, samples_ == 1 ? tileThreads_ : 256};
-    // enough workgroups for every view's queue, at most 16 per compute unit
-    const size_t queueChunks = ((size_t)curTris_ + clipCap_ + 255) / 256 * viewDesc_.size();
-    BinParams bp{tiles, (int)std::max<size_t>(1, std::min<size_t>(queueChunks, (size_t)numCUs_ * 16)), curTris_,
-                 clipCap_, binCap_, bigCap_, bigThreshold_};
-    launch_bin(bp, V, recPtrs(), binQueue_.as<uint4>(), binCount_.as<unsigned>(), binStart_.as<unsigned>(),
-               binCursor_.as<unsigned>(), binList_.as<unsigned>(), bigList_.as<unsigned>(), q,
-               ctr_.as<DeviceCounters>(), s);
+    BinParams bp{};
+    bp.tiles = tiles;
+    scatterShape(&bp.grid, &bp.regions);
+    bp.ntri = curTris_;
+    bp.clipCap = clipCap_;
+    bp.binCap = binCap_;
+    bp.bigCap = bigCap_;
+    launch_bin(bp, V, recPtrs(), bins, q, statPtrs(), ctr_.as<DeviceCounters>(), s);
     mark(3);
     RasterParams rp{};
     rp.depthFunc = depthFunc_;
@@ -1082,23 +1147,19 @@ void TileRasterRenderer::enqueue(bool clear) {
         // blending: fragments shaded and blended in primitive order (the shade stage is part of it)
         launch_blend_ordered(shadeParams(true), blendCoefs_, depthFunc_, clear ? 1 : 0, binCap_, V, recPtrs(),
                              bary_.as<float4>(), vtx_.as<float>(), idx_.as<int>(), texDesc_.as<TexDesc>(), texPool_,
-                             binStart_.as<unsigned>(), binCount_.as<unsigned>(), binList_.as<unsigned>(), tiles,
-                             rasterGrid(), visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, rgba8_.as<uchar4>(),
+                             bins, tiles, rasterGrid(), visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, rgba8_.as<uchar4>(),
                              rgba32f_.as<float4>(), statPtrs(), s);
         mark(4);
     } else if (depthFunc_ == IF_COMPARE_OP_LESS && !rp.depthWrite) {
         // order-independent: the lexicographic minimum of (depth, primitive)
-        launch_raster(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), binStart_.as<unsigned>(),
-                      binCount_.as<unsigned>(), binList_.as<unsigned>(), q, tiles, visDepth_.as<float>(),
+        launch_raster(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), bins, q, tiles, visDepth_.as<float>(),
                       visSlot_.as<uint32_t>(), cls, statPtrs(), ctr_.as<DeviceCounters>(), s);
         mark(4);
-        launch_raster_merge(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), binStart_.as<unsigned>(),
-                            binCount_.as<unsigned>(), q, visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, tiles,
-                            ctr_.as<DeviceCounters>(), s);
+        launch_raster_merge(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), bins, q, visDepth_.as<float>(),
+                            visSlot_.as<uint32_t>(), cls, tiles, ctr_.as<DeviceCounters>(), s);
     } else {
         // every other depth function folds each pixel's fragments in primitive order
-        launch_raster_ordered(rp, V, samples_, recPtrs(), binStart_.as<unsigned>(), binCount_.as<unsigned>(),
-                              binList_.as<unsigned>(), tiles, rasterGrid(), visDepth_.as<float>(),
+        launch_raster_ordered(rp, V, samples_, recPtrs(), bins, tiles, rasterGrid(), visDepth_.as<float>(),
                               visSlot_.as<uint32_t>(), cls, statPtrs(), s);
         mark(4);
     }
@@ -1232,7 +1293,7 @@ bool TileRasterRenderer::finish(bool clear, int indexCount) {
     stats_.inputTriangles = (int64_t)curTris_ * (int64_t)viewDesc_.size();
     stats_.assembledTriangles = (int64_t)c.assembled;
     stats_.clippedTriangles = (int64_t)c.clipCount;
-    stats_.binEntries = c.binTotal;
+    stats_.binEntries = c.tot[kTotEntries];
     stats_.fragments = (int64_t)c.fragments;
     stats_.coveredSamples = (int64_t)c.coveredSamples;
     stats_.status = c.status;
@@ -1250,11 +1311,11 @@ bool TileRasterRenderer::finish(bool clear, int indexCount) {
     };
     if (c.status & kStatusClipOverflow) clipCap_ = grow(clipCap_, c.clipMax + 1024u);
     if (c.status & kStatusBinOverflow) binCap_ = grow(binCap_, (unsigned)std::min<unsigned long long>(
-                                                                   (unsigned long long)c.binTotal + (1u << 20), 0xFFFFFFF0ull));
+                                                                   (unsigned long long)c.tot[kTotEntries] + (1u << 20), 0xFFFFFFF0ull));
     if (c.status & kStatusBigOverflow) bigCap_ = grow(bigCap_, c.bigCount + 1024u);
     if (c.status & kStatusRasterOverflow) {
-        itemCap_ = grow(itemCap_, c.numItems + 1024u);
-        partialCap_ = grow(partialCap_, c.numPartials + 256u);
+        itemCap_ = grow(itemCap_, c.tot[kTotLong] + c.tot[kTotShort] + 1024u);
+        partialCap_ = grow(partialCap_, c.tot[kTotPartials] + 256u);
     }
     if (c.status & kStatusBadIndex) setError("index buffer references a vertex beyond the vertex buffer");
     return (c.status & (kStatusClipOverflow | kStatusBinOverflow | kStatusBigOverflow | kStatusRasterOverflow)) == 0;
@@ -1267,7 +1328,10 @@ void TileRasterRenderer::drawElements(int indexCount, bool clear) {
     for (int attempt = 0; attempt < kAttempts; attempt++) {
         if (!prepare(indexCount)) return;
         submit(clear);
-        if (!ok(hipGetLastError(), "kernel launch")) return;
+        if (!ok(hipGetLastError(), "kernel launch")) {
+            countersDirty_ = true;
+            return;
+        }
         if (finish(clear, indexCount)) break;
         stats_.retries++;
         if (!clear) {
@@ -1285,7 +1349,7 @@ void TileRasterRenderer::drawAsync(int indexCount, bool clear) {
     if (gsBound_ && clipAt_ < 0) return drawGeometry(indexCount, clear, true);
     if (!prepare(indexCount)) return;
     submit(clear);
-    ok(hipGetLastError(), "kernel launch");
+    if (!ok(hipGetLastError(), "kernel launch")) countersDirty_ = true;
 }
 
 void TileRasterRenderer::synchronize() {

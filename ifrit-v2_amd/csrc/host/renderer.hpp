@@ -262,7 +262,7 @@ private:
     std::vector<int> viewLayout_;           // (width, height, shade) per view + shading tile
     unsigned totalTiles_ = 0, shadeTiles_ = 0;
     size_t totalPixels_ = 0;
-    DevBuf viewDev_, tileView_, shadeView_, viewCtr_, digest_, planSums_;
+    DevBuf viewDev_, tileView_, shadeView_, viewCtr_, digest_;
 
     // launch parameters (IfritTuning) and graph replay
     int partShift_ = kRasterPartShift;
@@ -278,8 +278,12 @@ private:
     std::vector<uint8_t> graphKey_;
 
     // device buffers
-    DevBuf vtx_, idx_, clip_, recs_[6], bary_, binQueue_, slotOf_, binCount_, binStart_, binCursor_, binList_, bigList_, ctr_;
-    DevBuf groupBounds_, groupOut_;  // per triangle group: bounds; per view and group: outside flag
+    DevBuf vtx_, idx_, clip_, recs_[6], bary_, binFront_, slotOf_, binCount_, binStart_, binCursor_, binList_, ctr_;
+    // the tile counts and live counters, zero between draws (the tile plan leaves them so), were
+    // left behind by a draw that failed to launch
+    bool countersDirty_ = false;
+    bool ensureZeroed(DevBuf& b, size_t n);
+    DevBuf groupBounds_;             // per triangle group: bounds
     DevBuf swapped_;                 // per record slot: set up with vertices 0 and 2 exchanged
     DevBuf polyKeys_;                // point and line modes: per pixel the nearest candidate's key
     static constexpr int kBufferSlots = 64;
@@ -302,6 +306,11 @@ private:
     int curTris_ = 0;
     int curIdx_ = 0;  // indices of the current draw (the point mode draws every index)
     TriRecs recPtrs() const;
+    VertexInput vertexInput() const;
+    // The geometry kernel's outputs (BinBufs and the assembled counts) in binFront_.
+    size_t frontBytes() const;
+    BinBufs binBufs() const;
+    void scatterShape(int* grid, int* regions) const;
     StatPartials statPtrs() const;
     int rasterGrid() const;
     std::vector<TextureSlot> textures_;

@@ -5,11 +5,15 @@
 // receives the triangle, flagged as fully covered when the trivial-accept
 // corner is inside too.
 //
-// Two passes over the triangles (count, then scatter after an exclusive scan
-// of the per-tile counts) build contiguous per-tile lists.  Lanes of a wave
-// that hit the same tile share one atomic (wave_inc).  Triangles spanning
-// more than bigThreshold tiles are deferred to a workgroup-per-triangle pass
-// so that a few screen-sized triangles do not serialise one lane.
+// The geometry and clip kernels counted the entries of every tile, triangles of
+// up to four tiles and others apart.  Here the tile plan turns the counts into list
+// ranges and raster work, and the scatter writes the contiguous per-tile
+// lists: the place of a triangle of up to four tiles is the list's start plus
+// the rank its count returned (no atomic, and its record is not read), the
+// others follow them through a cursor per tile.  Lanes of a wave that hit the same tile
+// share one atomic (wave_inc).  Triangles spanning more than bigThreshold
+// tiles go through a workgroup each, so that a few screen-sized triangles do
+// not serialise one lane.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -20,148 +24,23 @@ namespace {
 
 using dev::Edges;
 using dev::load_edges;
-using dev::tile_class;
-
-__device__ __forceinline__ int4 unpack_box(const uint4& e) {
-    return make_int4((int)(e.y & 0xFFFFu), (int)(e.y >> 16), (int)(e.z & 0xFFFFu), (int)(e.z >> 16));
-}
-
-// Shared traversal of the small triangles over the bin queues of all views.
-// Triangles deferred by the small-triangle pass (more tiles than the
-// threshold): one workgroup per triangle from `first` in steps of `stride`,
-// its threads over the tile rectangle.
-template <bool SCATTER>
-__device__ __forceinline__ void bin_big(const BinParams& P, const Views& V, const TriRecs& recs,
-                                        const uint4* __restrict__ queueAll, unsigned* __restrict__ binCount,
-                                        const unsigned* __restrict__ binStart, unsigned* __restrict__ binCursor,
-                                        unsigned* __restrict__ binList, const unsigned* __restrict__ bigList,
-                                        const DeviceCounters* ctr, unsigned first, unsigned stride) {
-    const unsigned nbig = min(ctr->bigCount, P.bigCap);
-    for (unsigned i = first; i < nbig; i += stride) {
-        const unsigned qi = bigList[i];
-        const ViewDesc& D = V.desc[qi / V.slotsPerView];
-        const unsigned tileBase = D.tileBase;
-        const int tilesX = D.tilesX;
-        const uint4 e = queueAll[qi];
-        const unsigned s = e.x;
-        const int4 b = unpack_box(e);
-        const Edges E = load_edges(recs, s);
-        const int w = b.z - b.x + 1;
-        const int area = w * (b.w - b.y + 1);
-        for (int q = threadIdx.x; q < area; q += blockDim.x) {
-            const int tx = b.x + q % w, ty = b.y + q / w;
-            const int c = tile_class(E, tx, ty);
-            if (!c) continue;
-            const int t = (int)tileBase + ty * tilesX + tx;
-            if (!SCATTER) {
-                atomicAdd(&binCount[t], 1u);
-            } else {
-                const unsigned at = binStart[t] + atomicAdd(&binCursor[t], 1u);
-                if (at < P.binCap) binList[at] = s | (c == 2 ? 0x80000000u : 0u);
-            }
-        }
-    }
-}
-
-// The queue entries of view v are numbered in chunks of 256 that continue
-// from the previous view's, and chunk c goes to workgroup c mod gridDim.x, so
-// the work spreads evenly whatever the views' sizes.  SCATTER = false counts
-// (and defers the big triangles), SCATTER = true writes the lists.
-template <bool SCATTER>
-__global__ void __launch_bounds__(256) k_bin_small(BinParams P, Views V, TriRecs recs,
-                                                   const uint4* __restrict__ queueAll, unsigned* __restrict__ binCount,
-                                                   const unsigned* __restrict__ binStart,
-                                                   unsigned* __restrict__ binCursor, unsigned* __restrict__ binList,
-                                                   unsigned* __restrict__ bigList, DeviceCounters* ctr) {
-    const unsigned G = gridDim.x;
-    unsigned chunkBase = 0;
-    for (int v = 0; v < V.count; v++) {
-        const unsigned nq = min(V.ctr[v].queued, V.slotsPerView);
-        const unsigned nch = (nq + 255u) / 256u;
-        const unsigned c0 = (blockIdx.x + G - chunkBase % G) % G;
-        chunkBase += nch;
-        if (c0 >= nch) continue;
-        const ViewDesc& D = V.desc[v];
-        const unsigned tileBase = D.tileBase;
-        const int tilesX = D.tilesX;
-        const uint4* queue = queueAll + (size_t)v * V.slotsPerView;
-        for (unsigned c = c0; c < nch; c += G) {
-            const unsigned qi = c * 256u + threadIdx.x;
-            const bool valid = qi < nq;
-            uint4 e = make_uint4(0u, 0u, 0u, 0u);
-            if (valid) e = queue[qi];
-            const unsigned s = e.x;
-            const int4 b = unpack_box(e);
-            const int w = b.z - b.x + 1;
-            const int area = valid ? w * (b.w - b.y + 1) : 0;
-            const bool big = valid && area > P.bigThreshold;
-            if (!SCATTER) {
-                // deferred triangles go to the per-workgroup pass (as their queue position)
-                const unsigned k = dev::wave_inc(&ctr->bigCount, 0, big);
-                if (big) {
-                    if (k < P.bigCap)
-                        bigList[k] = (unsigned)v * V.slotsPerView + qi;
-                    else
-                        atomicOr(&ctr->status, kStatusBigOverflow);
-                }
-            }
-            const int n = (valid && !big) ? area : 0;
-            Edges E;
-            if (n) E = load_edges(recs, s);
-            const int iters = dev::wave_max(n);
-            for (int i = 0; i < iters; i++) {
-                const bool active = i < n;
-                int t = 0, cls = 0;
-                if (active) {
-                    const int tx = b.x + i % w, ty = b.y + i / w;
-                    t = (int)tileBase + ty * tilesX + tx;
-                    cls = tile_class(E, tx, ty);
-                }
-                const bool hit = active && cls != 0;
-                if (!SCATTER) {
-                    (void)dev::wave_inc(binCount, t, hit);
-                } else {
-                    // the list start is loaded before the atomic, so that the two round trips overlap
-                    const unsigned st0 = hit ? binStart[t] : 0u;
-                    const unsigned pos = dev::wave_inc(binCursor, t, hit);
-                    if (hit) {
-                        const unsigned at = st0 + pos;
-                        if (at < P.binCap) binList[at] = s | (cls == 2 ? 0x80000000u : 0u);
-                    }
-                }
-            }
-        }
-    }
-    // the scatter pass also takes the deferred triangles, whose list the count pass completed
-    if constexpr (SCATTER)
-        bin_big<true>(P, V, recs, queueAll, binCount, binStart, binCursor, binList, bigList, ctr, blockIdx.x, G);
-}
-
-// The count pass's deferred triangles (the scatter pass takes its own at the
-// end of k_bin_small: the list is complete by then).
-__global__ void __launch_bounds__(256) k_bin_big_count(BinParams P, Views V, TriRecs recs,
-                                                       const uint4* __restrict__ queueAll,
-                                                       unsigned* __restrict__ binCount,
-                                                       const unsigned* __restrict__ bigList, const DeviceCounters* ctr) {
-    bin_big<false>(P, V, recs, queueAll, binCount, nullptr, nullptr, nullptr, bigList, ctr, blockIdx.x, gridDim.x);
-}
 
 // ---------------------------------------------------------------------------
-// Raster planning over the tiles of all views, in three launches so that
-// every phase is spread over the chip: (A) per block of 2048 tiles the sums
-// of six per-tile quantities, (B) one workgroup's exclusive scan of the block
-// sums and the totals, (C) per block the list starts and the work lists.
-// A tile's list is cut into items of at most 1 << partShift entries; items
-// of more than kRasterPass entries are listed from the front of the item
-// array and the others from its back, so that the queue hands out the long
-// ones first.  Tiles with several items get a partial key block per item and
-// go to multiList[0, numMulti); empty tiles go to multiList[tiles, ...).
-// Lists need not be in tile order: every tile's range is contiguous and the
-// ranges are disjoint.
+// Raster planning over the tiles of all views, in one launch: each workgroup
+// scans six quantities of its 256 tiles and takes its range of each with one
+// atomic on the draw's totals.  The workgroups' ranges come in any order, but
+// every tile's list is contiguous, the lists are disjoint, and a workgroup's
+// tiles stay together.  A tile's list is cut into items of at most 1 <<
+// partShift entries; items of more than kRasterPass entries are listed from
+// the front of the item array and the others from its back, so that the queue
+// hands out the long ones first.  Tiles with several items get a partial key
+// block per item and go to the front of multiList; empty tiles go to its back.
+//
+// The plan is also where a draw's live counters end: it publishes the draw's
+// own and leaves the tile counts and the live counters at zero, so that the
+// next draw needs no clearing launch.
 // ---------------------------------------------------------------------------
-constexpr int kPlanBlock = kPlanTiles;       // tiles per block
-constexpr int kPlanPer = kPlanBlock / 256;  // tiles per thread
-constexpr int kPlanQ = 6;                   // entries, long items, short items, partial blocks, multi, empty
+constexpr int kPlanQ = kTotCount;
 
 struct TilePlan {
     unsigned q[kPlanQ];
@@ -173,19 +52,14 @@ __device__ __forceinline__ TilePlan tile_plan(unsigned c, bool valid, int sh) {
     const unsigned p = valid ? (c + part - 1u) >> sh : 0u;
     const unsigned last = c - (p ? p - 1u : 0u) * part;  // entries of the last item
     const unsigned shortItems = p && last <= (unsigned)kRasterPass ? 1u : 0u;
-    w.q[0] = valid ? c : 0u;
-    w.q[1] = p - shortItems;
-    w.q[2] = shortItems;
-    w.q[3] = p > 1u ? p : 0u;
-    w.q[4] = p > 1u ? 1u : 0u;
-    w.q[5] = valid && p == 0u ? 1u : 0u;
+    w.q[kTotEntries] = valid ? c : 0u;
+    w.q[kTotLong] = p - shortItems;
+    w.q[kTotShort] = shortItems;
+    w.q[kTotPartials] = p > 1u ? p : 0u;
+    w.q[kTotMulti] = p > 1u ? 1u : 0u;
+    w.q[kTotEmpty] = valid && p == 0u ? 1u : 0u;
     return w;
 }
-
-// Tile of thread t's i-th slot in block b: a thread takes kPlanPer
-// consecutive tiles, so the work lists follow the tile order (neighbouring
-// tiles share triangles, and the raster runs neighbouring items together).
-__device__ __forceinline__ int plan_tile(int b, int i, int t) { return b * kPlanBlock + t * kPlanPer + i; }
 
 // Exclusive scan of kPlanQ values over a 256-thread workgroup; every thread must call it.
 __device__ __forceinline__ void scan256x6(unsigned* v, unsigned (*sWave)[4], unsigned* total) {
@@ -203,168 +77,199 @@ __device__ __forceinline__ void scan256x6(unsigned* v, unsigned (*sWave)[4], uns
 #pragma unroll
         for (int i = 0; i < 4; i++) base += i < w ? sWave[k][i] : 0u;
         v[k] += base;
-        if (total) total[k] = sWave[k][0] + sWave[k][1] + sWave[k][2] + sWave[k][3];
+        total[k] = sWave[k][0] + sWave[k][1] + sWave[k][2] + sWave[k][3];
     }
+}
+
+__global__ void __launch_bounds__(kPlanTiles) k_plan(uint2* __restrict__ cnt, unsigned* __restrict__ start,
+                                                     unsigned* __restrict__ cursor, int n, Views V, RasterQueue q,
+                                                     DeviceCounters* ctr) {
+    static_assert(kPlanTiles == 256, "one tile per thread");
+    __shared__ unsigned sWave[kPlanQ][4];
+    __shared__ unsigned sBase[kPlanQ];
+    const int t = threadIdx.x, tile = blockIdx.x * kPlanTiles + t;
+    if (blockIdx.x == 0) {
+        // publish the draw's counters and clear the live ones
+        for (int v = t; v < V.count; v += kPlanTiles) {
+            ViewCounters& c = V.ctr[v];
+            c.fans = c.fanLive;
+            c.clipIn = c.clipLive;
+            c.fanLive = 0u;
+            c.clipLive = 0u;
+        }
+        if (t == 0) {
+            ctr->status = ctr->live.status;
+            ctr->bigCount = ctr->live.bigCount;
+            ctr->clipMax = ctr->live.clipMax;
+            ctr->assembled = ctr->live.fans;
+            ctr->clipCount = 0u;
+            ctr->live.status = 0u;
+            ctr->live.bigCount = 0u;
+            ctr->live.clipMax = 0u;
+            ctr->live.fans = 0u;
+        }
+    }
+    uint2 c = make_uint2(0u, 0u);
+    if (tile < n) {
+        c = cnt[tile];
+        cnt[tile] = make_uint2(0u, 0u);
+    }
+    const unsigned total = c.x + c.y;
+    const TilePlan w = tile_plan(total, tile < n, q.partShift);
+    unsigned v[kPlanQ], sum[kPlanQ];
+#pragma unroll
+    for (int k = 0; k < kPlanQ; k++) v[k] = w.q[k];
+    scan256x6(v, sWave, sum);
+    // one lane per quantity, so that the atomics' round trips overlap
+#pragma unroll
+    for (int k = 0; k < kPlanQ; k++)
+        if (t == k) sBase[k] = sum[k] ? atomicAdd(&ctr->tot[k], sum[k]) : 0u;
     __syncthreads();
-}
-
-__global__ void __launch_bounds__(256) k_plan_sums(const unsigned* __restrict__ cnt, int n, int sh,
-                                                   unsigned* __restrict__ blockSums) {
-    __shared__ unsigned sWave[kPlanQ][4];
-    const int t = threadIdx.x;
-    unsigned v[kPlanQ] = {0, 0, 0, 0, 0, 0};
+    if (tile >= n) return;
 #pragma unroll
-    for (int i = 0; i < kPlanPer; i++) {
-        const int tile = plan_tile(blockIdx.x, i, t);
-        const TilePlan w = tile_plan(tile < n ? cnt[tile] : 0u, tile < n, sh);
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) v[k] += w.q[k];
-    }
-    unsigned total[kPlanQ];
-    scan256x6(v, sWave, total);
-    if (t < kPlanQ) blockSums[blockIdx.x * kPlanQ + t] = total[t];
-}
-
-// The plan's totals: list entries, items, partial blocks, multi-part and
-// empty tiles; the overflow flags; the item streams' heads reset.
-__device__ __forceinline__ void plan_totals(const unsigned* carry, unsigned cap, const RasterQueue& q,
-                                            DeviceCounters* ctr) {
-    ctr->binTotal = carry[0];
-    const bool binFits = carry[0] <= cap;
-    if (!binFits) atomicOr(&ctr->status, kStatusBinOverflow);
-    const bool fits = carry[1] + carry[2] <= q.itemCap && carry[3] <= q.partialCap;
-    if (!fits) atomicOr(&ctr->status, kStatusRasterOverflow);
-    const bool go = binFits && fits;
-    ctr->numItems = go ? carry[1] + carry[2] : 0u;
-    ctr->numLongItems = carry[1];
-    ctr->numPartials = carry[3];
-    ctr->numMulti = go ? carry[4] : 0u;
-    ctr->numEmpty = go ? carry[5] : 0u;
-    for (int k = 0; k < kItemStreams; k++) ctr->itemHeads[k][0] = 0u;
-}
-
-// One 1024-thread workgroup: exclusive offsets of the block sums (in place)
-// and the totals.  On a bin or work-list overflow nothing is rasterised; the
-// host grows the buffers and draws again.
-__global__ void __launch_bounds__(1024) k_plan_scan(unsigned* __restrict__ blockSums, int nblk, unsigned cap,
-                                                    RasterQueue q, DeviceCounters* ctr) {
-    __shared__ unsigned sWave[kPlanQ][16];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    unsigned carry[kPlanQ] = {0, 0, 0, 0, 0, 0};
-    for (int base = 0; base < nblk; base += 1024) {
-        // the six quantities of block b scanned together: two barriers per 1024 blocks
-        const int b = base + t;
-        unsigned v[kPlanQ], x[kPlanQ];
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) {
-            v[k] = b < nblk ? blockSums[b * kPlanQ + k] : 0u;
-            x[k] = v[k];
+    for (int k = 0; k < kPlanQ; k++) v[k] += sBase[k];
+    const unsigned part = 1u << q.partShift;
+    const unsigned st = v[kTotEntries], p = w.q[kTotLong] + w.q[kTotShort];
+    start[tile] = st;
+    cursor[tile] = st + c.x;  // the entries with ranks come first
+    for (unsigned k = 0; k < p; k++) {
+        const uint4 item = make_uint4((unsigned)tile, st + k * part, min(part, total - k * part),
+                                      p > 1u ? v[kTotPartials] + k : 0xFFFFFFFFu);
+        if (k < w.q[kTotLong]) {
+            if (v[kTotLong] + k < q.itemCap) q.items[v[kTotLong] + k] = item;
+        } else if (v[kTotShort] < q.itemCap) {
+            q.items[q.itemCap - 1u - v[kTotShort]] = item;
         }
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) x[k] = dev::wave_incl_scan(x[k]);
-        __syncthreads();  // sWave is free
-        if (lane == 63)
-#pragma unroll
-            for (int k = 0; k < kPlanQ; k++) sWave[k][w] = x[k];
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) {
-            unsigned pre = 0, tot = 0;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                pre += i < w ? sWave[k][i] : 0u;
-                tot += sWave[k][i];
+    }
+    if (p > 1u) q.multiList[v[kTotMulti]] = (unsigned)tile;
+    if (p == 0u) q.multiList[(unsigned)n - 1u - v[kTotEmpty]] = (unsigned)tile;
+    q.tilePartial[tile] = p > 1u ? (int)v[kTotPartials] : -1;
+}
+
+// One geometry wave's entries as a scatter wave holds them.
+struct Region {
+    bool any;                  // uniform: there is one
+    unsigned r;                // geometry wave over all views
+    bool single, few, multi;   // the lane's kind of entry
+    uint2 e;
+    uint4 f;
+};
+
+template <class F>
+__device__ __forceinline__ Region next_region(const WaveInfo& W, unsigned long long& pend, F&& bcast, unsigned r0,
+                                              int lane, const BinBufs& B) {
+    Region R{pend != 0ull, 0u, false, false, false, make_uint2(0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
+    if (!R.any) return R;
+    const int l = __ffsll(pend) - 1;
+    pend &= pend - 1ull;
+    R.r = r0 + (unsigned)l;
+    R.single = (bcast(W.single, l) >> lane) & 1ull;
+    R.few = (bcast(W.few, l) >> lane) & 1ull;
+    R.multi = (bcast(W.multi, l) >> lane) & 1ull;
+    if (R.single || R.few || R.multi) R.e = B.entry[(size_t)R.r * 64 + lane];
+    if (R.few) R.f = B.entry1[(size_t)R.r * 64 + lane];
+    return R;
+}
+
+// Writes the tile lists.  A wave takes the 64 triangles of one geometry wave at
+// a time (one lane each), `regions` geometry waves after another: one where
+// that leaves enough waves to fill the chip, more in batches of many views,
+// where most geometry waves lie outside the view and are skipped by their
+// WaveInfo.
+__global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs recs, BinBufs B, RasterQueue q,
+                                                 StatPartials st, DeviceCounters* ctr) {
+    __shared__ unsigned sMade[4];
+    const int lane = dev::lane_id();
+    const unsigned gw = blockIdx.x * 4u + (threadIdx.x >> 6), G = gridDim.x * 4u;
+    const unsigned R = (unsigned)V.count * V.waves, C = (unsigned)P.regions;
+    unsigned made = 0;
+    for (unsigned r0 = gw * C; r0 < R; r0 += G * C) {
+        WaveInfo W{0ull, 0ull, 0ull, 0ull, 0u, 0u};
+        if ((unsigned)lane < C && r0 + (unsigned)lane < R) W = B.waves[r0 + (unsigned)lane];
+        made += W.made;
+        unsigned long long pend = __ballot((W.single | W.few | W.multi) != 0ull);
+        auto bcast = [](unsigned long long x, int l) {
+            return ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
+                   (unsigned)__builtin_amdgcn_readlane((int)x, l);
+        };
+        // the entries of the next geometry wave are read while the current one's are written
+        Region N = next_region(W, pend, bcast, r0, lane, B);
+        while (N.any) {
+            const Region A = N;
+            N = next_region(W, pend, bcast, r0, lane, B);
+            const unsigned v = A.r / V.waves;
+            const uint2 e = A.e;
+            const uint4 f = A.f;
+            const unsigned slot = v * V.slotsPerView + (A.r - v * V.waves) * 64u + (unsigned)lane;
+            if (A.single) {
+                const unsigned at = B.start[e.x & 0x7fffffffu] + e.y;
+                if (at < P.binCap) B.list[at] = slot | (e.x & 0x80000000u);
             }
-            if (b < nblk) blockSums[b * kPlanQ + k] = carry[k] + pre + x[k] - v[k];
-            carry[k] += tot;
-        }
-    }
-    if (t == 0) plan_totals(carry, cap, q, ctr);
-}
-
-// Writes the tiles' list starts and work items.  SCAN: blockOffs holds the
-// blocks' own sums (at most 256 blocks), which every block scans itself, and
-// block 0 also stores the totals, in place of k_plan_scan; otherwise
-// blockOffs holds the blocks' offsets from k_plan_scan.
-template <bool SCAN>
-__global__ void __launch_bounds__(256) k_plan_write(const unsigned* __restrict__ cnt, unsigned* __restrict__ start,
-                                                    int n, int sh, const unsigned* __restrict__ blockOffs, int nblk,
-                                                    unsigned cap, RasterQueue q, DeviceCounters* ctr) {
-    __shared__ unsigned sWave[kPlanQ][4];
-    __shared__ unsigned sOff[kPlanQ];
-    const int t = threadIdx.x;
-    if constexpr (SCAN) {
-        unsigned b[kPlanQ], tot[kPlanQ];
+            if (__ballot(A.few) != 0ull) {
+                const int tilesX = V.desc[v].tilesX;
+                const int cols = (int)(f.w & 3u) + 1;
+                const unsigned rank[4] = {e.y, f.x, f.y, f.z};
+                unsigned st[4];
 #pragma unroll
-        for (int k = 0; k < kPlanQ; k++) b[k] = t < nblk ? blockOffs[t * kPlanQ + k] : 0u;
-        scan256x6(b, sWave, tot);
-        if (t == (int)blockIdx.x)
+                for (int k = 0; k < 4; k++) {  // the list starts in one round trip
+                    st[k] = 0u;
+                    if ((f.w >> (8 + 2 * k)) & 3u)
+                        st[k] = B.start[e.x + (unsigned)(dev::few_row(k, cols) * tilesX + dev::few_col(k, cols))];
+                }
 #pragma unroll
-            for (int k = 0; k < kPlanQ; k++) sOff[k] = b[k];
-        if (blockIdx.x == 0 && t == 0) plan_totals(tot, cap, q, ctr);
-        __syncthreads();
-    }
-    unsigned c[kPlanPer];
-    unsigned v[kPlanQ] = {0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < kPlanPer; i++) {
-        const int tile = plan_tile(blockIdx.x, i, t);
-        c[i] = tile < n ? cnt[tile] : 0u;
-        const TilePlan w = tile_plan(c[i], tile < n, sh);
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) v[k] += w.q[k];
-    }
-    scan256x6(v, sWave, nullptr);
-#pragma unroll
-    for (int k = 0; k < kPlanQ; k++) v[k] += SCAN ? sOff[k] : blockOffs[blockIdx.x * kPlanQ + k];
-    const unsigned part = 1u << sh;
-    for (int i = 0; i < kPlanPer; i++) {
-        const int tile = plan_tile(blockIdx.x, i, t);
-        if (tile >= n) break;
-        const TilePlan w = tile_plan(c[i], true, sh);
-        const unsigned st = v[0], p = w.q[1] + w.q[2];
-        start[tile] = st;
-        for (unsigned k = 0; k < p; k++) {
-            const unsigned first = st + k * part;
-            const uint4 item = make_uint4((unsigned)tile, first, min(part, c[i] - k * part),
-                                          p > 1u ? v[3] + k : 0xFFFFFFFFu);
-            if (k < w.q[1]) {
-                if (v[1] + k < q.itemCap) q.items[v[1] + k] = item;
-            } else if (v[2] < q.itemCap) {
-                q.items[q.itemCap - 1u - v[2]] = item;
+                for (int k = 0; k < 4; k++) {
+                    const unsigned c = (f.w >> (8 + 2 * k)) & 3u, at = st[k] + rank[k];
+                    if (c && at < P.binCap) B.list[at] = slot | (c == 2u ? 0x80000000u : 0u);
+                }
+            }
+            if (__ballot(A.multi) != 0ull) {
+                const ViewDesc& D = V.desc[v];
+                Edges E = {};
+                if (A.multi) E = load_edges(recs, slot);
+                const int4 b = A.multi ? dev::unpack_box(e) : make_int4(1, 0, 0, 0);
+                dev::bin_lanes<true>(E, b, D.tileBase, D.tilesX, slot, B, P.binCap);
             }
         }
-        if (p > 1u) q.multiList[v[4]] = (unsigned)tile;
-        if (p == 0u) q.multiList[n + v[5]] = (unsigned)tile;
-        q.tilePartial[tile] = p > 1u ? (int)v[3] : -1;
-#pragma unroll
-        for (int k = 0; k < kPlanQ; k++) v[k] += w.q[k];
+    }
+    // clip fans, one lane each: wave k takes view k / per, as few fans per wave as that many
+    // waves allow (a large fan takes the whole wave)
+    const unsigned per = max(1u, G / (unsigned)V.count);
+    for (unsigned k = gw; k < per * (unsigned)V.count; k += G) {
+        const unsigned v = k / per;
+        const unsigned n = min(V.ctr[v].fans, P.clipCap), each = min(64u, (n + per - 1u) / per);
+        for (unsigned i0 = (k % per) * each; i0 < n; i0 += per * each) {
+            const ViewDesc& D = V.desc[v];
+            const unsigned i = i0 + (unsigned)lane, slot = D.slotBase + (unsigned)P.ntri + i;
+            int4 b = make_int4(1, 0, 0, 0);
+            Edges E = {};
+            if ((unsigned)lane < each && i < n) b = dev::unpack_box(B.fanBox[(size_t)v * P.clipCap + i]);
+            if (b.x <= b.z) E = load_edges(recs, slot);
+            dev::bin_lanes<true>(E, b, D.tileBase, D.tilesX, slot, B, P.binCap);
+        }
+    }
+    dev::bin_big<true>(min(ctr->bigCount, P.bigCap), V, recs, B, P.binCap);
+    // the workgroup's assembled triangles, for the statistics
+    made = dev::wave_incl_scan(made);
+    if (lane == 63) sMade[threadIdx.x >> 6] = made;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        st.setupAssembled[blockIdx.x] = sMade[0] + sMade[1] + sMade[2] + sMade[3];
+        if (blockIdx.x == 0) {
+            // on a bin or work-list overflow nothing is rasterised (plan_fits); the host grows the
+            // buffers and draws again
+            if (ctr->tot[kTotEntries] > q.binCap) atomicOr(&ctr->status, kStatusBinOverflow);
+            if (!dev::plan_items_fit(ctr, q)) atomicOr(&ctr->status, kStatusRasterOverflow);
+        }
     }
 }
 
 }  // namespace
 
-void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const uint4* binQueue, unsigned* binCount,
-                unsigned* binStart, unsigned* binCursor, unsigned* binList, unsigned* bigList, const RasterQueue& q,
-                DeviceCounters* ctr, hipStream_t s) {
-    const dim3 g(p.grid);
-    hipLaunchKernelGGL(k_bin_small<false>, g, dim3(256), 0, s, p, views, recs, binQueue, binCount, binStart, binCursor,
-                       binList, bigList, ctr);
-    hipLaunchKernelGGL(k_bin_big_count, dim3(256), dim3(256), 0, s, p, views, recs, binQueue, binCount, bigList,
-                       ctr);
-    const int nblk = (p.tiles + kPlanBlock - 1) / kPlanBlock;
-    hipLaunchKernelGGL(k_plan_sums, dim3(nblk), dim3(256), 0, s, binCount, p.tiles, q.partShift, q.planSums);
-    if (nblk <= 256) {
-        // few blocks: each block scans the block sums itself (no third launch)
-        hipLaunchKernelGGL(k_plan_write<true>, dim3(nblk), dim3(256), 0, s, binCount, binStart, p.tiles,
-                           q.partShift, q.planSums, nblk, p.binCap, q, ctr);
-    } else {
-        hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, s, q.planSums, nblk, p.binCap, q, ctr);
-        hipLaunchKernelGGL(k_plan_write<false>, dim3(nblk), dim3(256), 0, s, binCount, binStart, p.tiles,
-                           q.partShift, q.planSums, nblk, p.binCap, q, ctr);
-    }
-    hipLaunchKernelGGL(k_bin_small<true>, g, dim3(256), 0, s, p, views, recs, binQueue, binCount, binStart, binCursor,
-                       binList, bigList, ctr);
+void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
+                StatPartials st, DeviceCounters* ctr, hipStream_t s) {
+    hipLaunchKernelGGL(k_plan, dim3((p.tiles + kPlanTiles - 1) / kPlanTiles), dim3(kPlanTiles), 0, s,
+                       reinterpret_cast<uint2*>(bins.cnt), bins.start, bins.cursor, p.tiles, views, q, ctr);
+    hipLaunchKernelGGL(k_scatter, dim3(p.grid), dim3(256), 0, s, p, views, recs, bins, q, st, ctr);
 }
 
 }  // namespace ifrit_hip

@@ -24,22 +24,6 @@ __device__ __forceinline__ TriRec load_rec(const TriRecs& R, unsigned slot) {
     return r;
 }
 
-// Pixel box of a record: x0, y0, x1, y1 and the big flag.
-struct PixBox {
-    int x0, y0, x1, y1;
-    bool big;
-};
-__device__ __forceinline__ PixBox pix_box(const TriRec& r) {
-    const unsigned lo = __float_as_uint(r.q2.z), hi = __float_as_uint(r.q2.w);
-    PixBox b;
-    b.x0 = (int)(lo & 0xffffu);
-    b.y0 = (int)(lo >> 16);
-    b.x1 = (int)(hi & 0xffffu);
-    b.y1 = (int)((hi >> 16) & 0x7fffu);
-    b.big = (hi >> 31) != 0;
-    return b;
-}
-
 // Edge coefficients of a TriRec: inside when fma(ey, y, ex * x) < -ez.
 struct Edges {
     float x[3], y[3], z[3];
@@ -60,6 +44,17 @@ __device__ __forceinline__ Edges load_edges(const TriRecs& R, unsigned slot) {
     E.x[0] = a.x; E.y[0] = a.y; E.z[0] = a.z;
     E.x[1] = a.w; E.y[1] = b.x; E.z[1] = b.y;
     E.x[2] = b.z; E.y[2] = b.w; E.z[2] = c;
+    return E;
+}
+
+__device__ __forceinline__ Edges edges_of(const float e[3][3]) {
+    Edges E;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        E.x[k] = e[k][0];
+        E.y[k] = e[k][1];
+        E.z[k] = e[k][2];
+    }
     return E;
 }
 
@@ -172,16 +167,21 @@ __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
 // Wave-aggregated counter increment: every active lane adds one to
 // ctr[key] and receives a unique position; lanes sharing a key share one
 // atomic.  The lanes are grouped by key with ballots first, so all groups'
-// atomics go out as one instruction and the wave waits for memory once.
-// Must be called by the whole (converged) wave.
-__device__ __forceinline__ unsigned wave_inc(unsigned* ctr, int key, bool active) {
+// atomics go out as one instruction and the wave waits for memory once, or,
+// with several increments issued before the first value is taken, once for
+// all of them.  Must be called by the whole (converged) wave.
+struct WaveInc {
+    unsigned base, rank;
+    int leader;
+};
+__device__ __forceinline__ WaveInc wave_inc_issue(unsigned* ctr, int key, bool active) {
     const int lane = lane_id();
     unsigned long long pending = __ballot(active);
     int leader = lane;
     unsigned rank = 0, size = 0;
     while (pending) {
         const int l = __ffsll((unsigned long long)pending) - 1;
-        const int lk = __shfl(key, l, 64);
+        const int lk = __builtin_amdgcn_readlane(key, l);  // l is uniform
         const unsigned long long grp = __ballot(active && key == lk) & pending;
         if ((grp >> lane) & 1ull) {
             leader = l;
@@ -190,10 +190,93 @@ __device__ __forceinline__ unsigned wave_inc(unsigned* ctr, int key, bool active
         if (lane == l) size = (unsigned)__popcll(grp);
         pending &= ~grp;
     }
-    unsigned base = 0;
-    if (active && leader == lane) base = atomicAdd(&ctr[key], size);
-    base = __shfl(base, leader, 64);
-    return base + rank;
+    WaveInc r{0u, rank, leader};
+    if (active && leader == lane) r.base = atomicAdd(&ctr[key], size);
+    return r;
+}
+__device__ __forceinline__ unsigned wave_inc_value(const WaveInc& r) { return __shfl(r.base, r.leader, 64) + r.rank; }
+__device__ __forceinline__ unsigned wave_inc(unsigned* ctr, int key, bool active) {
+    return wave_inc_value(wave_inc_issue(ctr, key, active));
+}
+
+// A tile rectangle from its packed form (x0 | y0 << 16, x1 | y1 << 16).
+__device__ __forceinline__ int4 unpack_box(const uint2& e) {
+    return make_int4((int)(e.x & 0xFFFFu), (int)(e.x >> 16), (int)(e.y & 0xFFFFu), (int)(e.y >> 16));
+}
+
+// Tile k of a rectangle of `cols` columns whose tiles number at most four.
+__device__ __forceinline__ int few_col(int k, int cols) { return cols == 1 ? 0 : (cols == 2 ? k & 1 : k); }
+__device__ __forceinline__ int few_row(int k, int cols) { return cols == 1 ? k : (cols == 2 ? k >> 1 : 0); }
+
+// Where a triangle goes in the tiles: SCATTER = false counts it, true writes it
+// through the tile's cursor.
+template <bool SCATTER>
+__device__ __forceinline__ void bin_tile(const Edges& E, int tx, int ty, unsigned tileBase, int tilesX, unsigned slot,
+                                         const BinBufs& B, unsigned binCap) {
+    const int c = tile_class(E, tx, ty);
+    if (!c) return;
+    const unsigned t = tileBase + (unsigned)(ty * tilesX + tx);
+    if constexpr (!SCATTER) {
+        atomicAdd(&B.cnt[2 * t + 1], 1u);
+    } else {
+        const unsigned at = atomicAdd(&B.cursor[t], 1u);
+        if (at < binCap) B.list[at] = slot | (c == 2 ? 0x80000000u : 0u);
+    }
+}
+
+// Bins one triangle per lane (b.x > b.z: none): a lane walks a rectangle of up
+// to eight tiles by itself, the wave shares larger ones, one round trip for 64
+// tiles (a clip fan next to the eye often spans the whole frame).  The whole
+// wave must call it.
+template <bool SCATTER>
+__device__ __forceinline__ void bin_lanes(const Edges& E, int4 b, unsigned tileBase, int tilesX, unsigned slot,
+                                         const BinBufs& B, unsigned binCap) {
+    const int w = b.z - b.x + 1, area = b.x <= b.z ? w * (b.w - b.y + 1) : 0;
+    if (area <= 8) {
+        for (int q = 0; q < area; q++) bin_tile<SCATTER>(E, b.x + q % w, b.y + q / w, tileBase, tilesX, slot, B, binCap);
+    }
+    for (unsigned long long m = __ballot(area > 8); m; m &= m - 1ull) {
+        const int l = __ffsll(m) - 1;
+        auto rl = [l](int x) { return __builtin_amdgcn_readlane(x, l); };
+        Edges F;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            F.x[k] = __int_as_float(rl(__float_as_int(E.x[k])));
+            F.y[k] = __int_as_float(rl(__float_as_int(E.y[k])));
+            F.z[k] = __int_as_float(rl(__float_as_int(E.z[k])));
+        }
+        const int x0 = rl(b.x), y0 = rl(b.y), fw = rl(w), fa = rl(area);
+        const unsigned fs = (unsigned)rl((int)slot);
+        for (int q = lane_id(); q < fa; q += 64)
+            bin_tile<SCATTER>(F, x0 + q % fw, y0 + q / fw, tileBase, tilesX, fs, B, binCap);
+    }
+}
+
+// Deferred triangles: units of up to 256 tiles, kBigParts units per triangle in
+// turn, so that a screen-sized one spreads over as many workgroups.
+constexpr unsigned kBigParts = 32;
+template <bool SCATTER>
+__device__ __forceinline__ void bin_big(unsigned nbig, const Views& V, const TriRecs& recs, const BinBufs& B,
+                                        unsigned binCap) {
+    for (unsigned u = blockIdx.x; u < nbig * kBigParts; u += gridDim.x) {
+        const uint4 g = B.big[u / kBigParts];
+        const int4 b = unpack_box(make_uint2(g.y, g.z));
+        const int w = b.z - b.x + 1, area = w * (b.w - b.y + 1);
+        const int first = (int)(u % kBigParts) * 256;
+        if (first >= area) continue;
+        const ViewDesc& D = V.desc[g.w];
+        const Edges E = load_edges(recs, g.x);
+        for (int q = first + (int)threadIdx.x; q < area; q += (int)kBigParts * 256)
+            bin_tile<SCATTER>(E, b.x + q % w, b.y + q / w, D.tileBase, D.tilesX, g.x, B, binCap);
+    }
+}
+
+// Whether the tile plan's raster work fits its buffers, and its lists too.
+__device__ __forceinline__ bool plan_items_fit(const DeviceCounters* ctr, const RasterQueue& q) {
+    return ctr->tot[kTotLong] + ctr->tot[kTotShort] <= q.itemCap && ctr->tot[kTotPartials] <= q.partialCap;
+}
+__device__ __forceinline__ bool plan_fits(const DeviceCounters* ctr, const RasterQueue& q) {
+    return ctr->tot[kTotEntries] <= q.binCap && plan_items_fit(ctr, q);
 }
 
 // Sum over a 256-thread workgroup (all threads must call it).
@@ -205,11 +288,6 @@ __device__ __forceinline__ unsigned long long block_sum256(unsigned long long v)
     const unsigned long long r = part[0] + part[1] + part[2] + part[3];
     __syncthreads();
     return r;
-}
-
-__device__ __forceinline__ int wave_max(int v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return v;
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave with DPP moves: row

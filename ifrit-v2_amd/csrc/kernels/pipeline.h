@@ -7,14 +7,18 @@
 //   views       ViewDesc[N]               per-view camera, size and bases
 //   tileView    ushort[tiles]             view of each 16x16 tile (tiles of all views)
 //   shadeView   ushort[shadeTiles]        view of each shading tile
-//   clip        float4[N][V]              vertex stage output
+//   clip        float4[N][V]              vertex stage output (point and line modes; triangle draws
+//                                         transform in the geometry kernel)
 //   recs        TriRecs, N * SV slots     assembled triangles; in view v, slot v*SV + prim
 //                                         for unclipped triangles, v*SV + T + k for clip fans
-//   bary        float4[2 * N * SV]        vertex-weight bases bx, by of clip fans (shading only)
-//   binQueue    uint4[N * SV]             per view, the assembled triangles to bin: (slot,
-//                                         x0 | y0 << 16, x1 | y1 << 16, 0), view-local tiles
-//   slotOf      uint[N][T]                first slot of each primitive (its fans follow)
-//   binCount/binStart/binCursor  uint[tiles]
+//   bary        float4[2 * N * clipCap]   vertex-weight bases bx, by of clip fans (shading only), or of
+//                                         every slot in the point and line modes
+//   waves       WaveInfo[N][waves]        per 64 triangles, what the geometry kernel made of them
+//   entry       uint2, uint4[N][64 waves] per triangle, its bin entries or tile rectangle (WaveInfo)
+//   fanBox      uint2[N][clipCap]         tile rectangle of each clip fan
+//   slotOf      uint[N][T]                first fan slot of each clipped primitive (its fans follow)
+//   binCnt      uint2[tiles]              entries counted: triangles of up to four tiles, others
+//   binStart/binCursor  uint[tiles]       a tile's list; after binning the cursor is its end
 //   binList     uint[binCap]              slot | 0x80000000 when the tile is fully covered
 //   visId/visDepth/visSlot  [pixels * S]  per-sample winner; views one after another, pixels
 //                                         row-major within a view, samples innermost
@@ -29,12 +33,10 @@ namespace ifrit_hip {
 
 // One assembled triangle for coverage and depth (6 x 16 bytes):
 //   q0 = e1.xyz, e2.x   q1 = e2.yz, e3.xy
-//   q2 = e3.z, key, pixel box (x0 | y0 << 16), (x1 | y1 << 16 | big << 31)
+//   q2 = e3.z, key, 0, 0
 //   f1, f2, f3 = interpolation bases (x, y, z) and vz = (z/w) * w.
 // key = prim * 4 + fan orders fragments the way the reference's per-tile
-// sort by originalPrimitive does (TileRasterWorker.cpp:1244-1258).  The
-// pixel box is the padded screen extent, a hint that selects the fine-raster
-// path (triangles flagged big are rasterised one pixel per lane).
+// sort by originalPrimitive does (TileRasterWorker.cpp:1244-1258).
 struct __align__(16) TriRec {
     float4 q0, q1, q2;
     float4 f1, f2, f3;
@@ -48,7 +50,7 @@ struct TriRecs {
 
 // One view of a draw.  View v owns tiles [tileBase, tileBase + tilesX *
 // tilesY), record slots [slotBase, slotBase + SV), slotOf entries
-// [primBase, primBase + T) and pixels [pixBase, pixBase + width * height).
+// [primBase, primBase + T), the geometry waves [v * waves, (v + 1) * waves) and pixels [pixBase, pixBase + width * height).
 struct ViewDesc {
     float mvp[16];
     float camera[3];
@@ -62,14 +64,42 @@ struct ViewDesc {
     unsigned long long pixBase;  // first pixel of the view's outputs
 };
 
-// Per-view counters (zeroed each draw), one 128-byte line each so
-// that the views' atomics do not share a line.
+// Per-view counters, one 128-byte line each so that the views' atomics do not
+// share a line.  The first two are counted by the geometry and clip kernels;
+// the tile plan moves them to the last two, which later kernels read, and
+// leaves zeros for the next draw.
 struct ViewCounters {
-    unsigned clipCount;    // clip fan slots taken
-    unsigned clipInCount;  // triangles crossing w = 0
-    unsigned queued;       // assembled triangles queued for binning
-    unsigned pad[29];
+    unsigned fanLive;   // clip fan slots taken so far
+    unsigned clipLive;  // triangles found to cross w = 0 so far
+    unsigned fans;      // clip fan slots of the draw
+    unsigned clipIn;    // triangles of the draw crossing w = 0
+    unsigned pad[28];
 };
+
+// What the geometry kernel made of the 64 triangles of one wave (triangles
+// 64 w .. 64 w + 63 of a view).  A triangle in `single` lies in one tile: its
+// entry is (tile | full << 31, rank in the tile's list); one in `few` spans two
+// to four, (first tile, rank there) and in entry1 the ranks in the others and
+// its FewTiles; one in `multi` spans more: (x0 | y0 << 16, x1 | y1 << 16),
+// view-local tiles.  `clipped` triangles crossed w = 0 (slotOf names their
+// first fan).
+struct __align__(8) WaveInfo {
+    unsigned long long single, few, multi, clipped;
+    unsigned made;  // triangles assembled (clip fans not counted)
+    unsigned pad;
+};
+
+// A rectangle of up to four tiles in entry1.w: columns - 1 in bits 0-1, tiles
+// in bits 2-4, and from bit 8 on two bits per tile, row by row: its
+// classification (dev::tile_class).
+__host__ __device__ inline unsigned few_tiles(int cols, int area) { return (unsigned)(cols - 1) | ((unsigned)area << 2); }
+
+// Waves of the geometry kernel per view: whole workgroups of four.
+constexpr int kGeomBlock = 256;
+__host__ __device__ inline unsigned geom_waves(int ntri) {
+    const unsigned b = (unsigned)((ntri + kGeomBlock - 1) / kGeomBlock);
+    return (b ? b : 1u) * (kGeomBlock / 64);
+}
 
 struct Views {
     const ViewDesc* desc;
@@ -78,6 +108,7 @@ struct Views {
     ViewCounters* ctr;
     int count;
     unsigned slotsPerView;            // SV = T + clipCap
+    unsigned waves;                   // geometry waves per view
 };
 
 // Scissor rectangles (SetScissors / setScissorTestEnable of the CUDA renderer,
@@ -110,23 +141,43 @@ struct SetupParams {
     float invW, invH;   // 1 / width, 1 / height (TileRasterRenderer.cpp:59-60)
     float invTileWidth; // ApproxReciprocal(16.0f) (TileRasterWorker.cpp:499)
     int rcpModel;       // ifx::RcpModel: whose RCPPS the reciprocals of w and of the area reproduce
-    // per view, per group of kGroupTris triangles: 1 when the group's bounds lie
-    // outside a frustum plane with a margin (null: no group culling)
-    const unsigned char* groupOut;
+    // object-space bounds of each group of kGroupTris triangles (null: no group culling)
+    const float4* groupBounds;
     int groups;
+    unsigned bigCap;
+    int bigThreshold;   // triangles spanning more tiles are binned by whole workgroups
 };
 
-// Triangles per culling group (a multiple of the 64-lane wave).
-constexpr int kGroupTris = 256;
+// Vertex input of the geometry kernel: clipAt < 0 transforms a record's first
+// three floats by each view's matrix, otherwise the record holds the clip
+// position at float clipAt.
+struct VertexInput {
+    const float* vtx;
+    int stride, clipAt;
+};
+
+// Binning buffers (see the layout above).
+struct BinBufs {
+    uint2* entry;
+    uint4* entry1;
+    WaveInfo* waves;
+    uint2* fanBox;
+    uint4* big;  // deferred triangles: slot, tile rectangle (as in entry), view
+    unsigned* cnt;
+    unsigned *start, *cursor, *list;
+};
+
+// Triangles per culling group (one workgroup of the geometry kernel).
+constexpr int kGroupTris = kGeomBlock;
 
 struct BinParams {
     int tiles;          // tiles of all views
-    int grid;           // workgroups of the binning launches
+    int grid;           // workgroups of the scatter launch
+    int regions;        // geometry waves a scatter wave takes at a time (1 .. 64)
     int ntri;
     unsigned clipCap;
     unsigned binCap;
     unsigned bigCap;
-    int bigThreshold;   // triangles spanning more tiles go to the per-workgroup binner
 };
 
 struct RasterParams {
@@ -205,33 +256,38 @@ enum StatusBits : unsigned {
 // Per-workgroup statistics (no same-address atomics in the hot kernels);
 // k_finalize reduces them into DeviceCounters.
 struct StatPartials {
-    unsigned long long* setupAssembled;  // one per setup workgroup
+    unsigned long long* setupAssembled;  // one per scatter workgroup
     unsigned long long* rasterFrags;     // one per raster workgroup
     unsigned long long* rasterCovs;      // one per raster workgroup
     int setupBlocks, rasterBlocks;
 };
 
-// Counters written by the kernels (device memory, zeroed each draw by the vertex or reset kernel).
 // Raster work items are drained through this many counters, one per XCD:
 // stream k holds items k, k + kItemStreams, ... and is taken by the
 // workgroups with blockIdx.x % kItemStreams == k (one XCD's), so the claims
 // of the persistent raster spread over separate lines instead of one.
 constexpr int kItemStreams = 8;
 
+// Totals of the tile plan (DeviceCounters::tot).
+enum PlanTotal { kTotEntries = 0, kTotLong, kTotShort, kTotPartials, kTotMulti, kTotEmpty, kTotCount = 6 };
+
+// Counters written by the kernels (device memory).  `live` is counted by the
+// geometry and clip kernels; the tile plan moves it to the fields above and
+// leaves zeros for the next draw, so that a draw needs no clearing launch.
+// The totals and item heads are cleared by the geometry kernel.
 struct DeviceCounters {
     unsigned status;
     unsigned clipCount;  // clip fan slots of all views (reduced with the statistics)
     unsigned bigCount;
-    unsigned binTotal;
+    unsigned clipMax;    // largest per-view fan or clip count (sizes clipCap on overflow)
     unsigned long long fragments;
     unsigned long long coveredSamples;
     unsigned long long assembled;
-    unsigned clipMax;    // largest per-view clipCount or clipInCount (sizes clipCap on overflow)
-    unsigned numItems;
-    unsigned numMulti;     // tiles cut into several parts
-    unsigned numPartials;  // partial blocks those need
-    unsigned numEmpty;     // tiles with an empty list
-    unsigned numLongItems; // items of more than kRasterPass entries (front of the item array)
+    unsigned tot[8];     // PlanTotal: list entries, items of more than kRasterPass entries (front of the
+                         // item array), other items, partial blocks, tiles cut into parts, empty tiles
+    struct alignas(128) Live {
+        unsigned status, bigCount, clipMax, fans;  // fans: fan triangles assembled
+    } live;
     alignas(128) unsigned itemHeads[kItemStreams][32];  // next item of each stream, one 128-byte line each
 };
 
@@ -239,57 +295,54 @@ struct DeviceCounters {
 // one tile (256 to 1024), taken in passes of kRasterPass entries (the LDS
 // capacity).
 constexpr int kRasterPass = 128;
-// Tiles per workgroup of the tile-plan kernels (one per thread): their block
-// sums take (tiles + kPlanTiles - 1) / kPlanTiles + 1 groups of six words.
+// Tiles per workgroup of the tile-plan kernel (one per thread).
 constexpr int kPlanTiles = 256;
 constexpr int kRasterPartShift = 9;
 
 // Raster work: items {tile, first list entry, entries, partial block or
 // ~0u} drained through DeviceCounters::itemHeads; per tile the first partial
 // block of a tile cut into several items (-1 otherwise); the list of such
-// tiles followed, from index `tiles`, by the empty tiles; partial key blocks
-// of 256 * samples keys each; planning scratch (6 words per 2048 tiles).
+// tiles from the front and of the empty tiles from the back (index `tiles` - 1
+// down); partial key blocks of 256 * samples keys each.
 struct RasterQueue {
     uint4* items;
     int* tilePartial;
     unsigned* multiList;
     unsigned long long* partials;
-    unsigned* planSums;
-    unsigned itemCap, partialCap;
+    unsigned itemCap, partialCap, binCap;
     int grid;         // raster workgroups
     int mergeGrid;    // half the merge workgroups
     int partShift;
     int tileThreads;  // threads per tile at 1 sample per pixel: 64 or 256
 };
 
-// Launch wrappers.  clipAt: -1 transforms attribute 0 (xyz) by each view's
-// matrix; otherwise the record holds the clip position at float clipAt.
-void launch_vertex(const float* vtx, int stride, int nverts, const Views& views, int clipAt, float4* clip,
-                   unsigned* binCount, unsigned* binCursor, int tiles, DeviceCounters* ctr,
-                   const float4* groupBounds, int groups, unsigned char* groupOut, hipStream_t s);
+// Launch wrappers.  launch_vertex (point and line modes) writes every view's
+// clip positions and clears the counters; launch_reset only clears them.
+void launch_vertex(const VertexInput& in, int nverts, const Views& views, float4* clip, DeviceCounters* ctr,
+                   hipStream_t s);
 void launch_group_bounds(const float* vtx, int stride, int nverts, const int* idx, int ntri, float4* bounds,
                          hipStream_t s);
-void launch_reset(unsigned* binCount, unsigned* binCursor, int tiles, const Views& views, DeviceCounters* ctr,
-                  hipStream_t s);
-void launch_setup(const SetupParams& p, const Views& views, const float4* clip, const int* idx, TriRecs recs, float4* bary, uint4* binQueue,
-                  unsigned* slotOf, unsigned* clipList, StatPartials st, DeviceCounters* ctr, hipStream_t s);
+void launch_reset(const Views& views, DeviceCounters* ctr, hipStream_t s);
+// Vertex transform, triangle setup and the bin counts, then the triangles that
+// cross w = 0 and those deferred by the bin count.
+void launch_geometry(const SetupParams& p, const Views& views, const VertexInput& in, const int* idx, TriRecs recs,
+                     float4* bary, const BinBufs& bins, unsigned* slotOf, unsigned* clipList, DeviceCounters* ctr,
+                     hipStream_t s);
 void launch_finalize(StatPartials st, const Views& views, DeviceCounters* ctr, hipStream_t s);
-void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const uint4* binQueue, unsigned* binCount, unsigned* binStart,
-                unsigned* binCursor, unsigned* binList, unsigned* bigList, const RasterQueue& q, DeviceCounters* ctr,
-                hipStream_t s);
+// The tile plan and the scatter into the tile lists.
+void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
+                StatPartials st, DeviceCounters* ctr, hipStream_t s);
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
-                   const unsigned* binStart, const unsigned* binCount, const unsigned* binList, const RasterQueue& q,
-                   int tiles, float* visDepth, uint32_t* visSlot, uint8_t* visClass, StatPartials st,
-                   DeviceCounters* ctr, hipStream_t s);
+                   const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
+                   uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s);
 void launch_raster_merge(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
-                         const unsigned* binStart, const unsigned* binCount, const RasterQueue& q, float* visDepth,
-                         uint32_t* visSlot, uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s);
+                         const BinBufs& bins, const RasterQueue& q, float* visDepth, uint32_t* visSlot,
+                         uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s);
 // Depth functions other than LESS: each tile's list in primitive order, folded
 // per pixel (replaces launch_raster and launch_raster_merge).
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
-                           const unsigned* binStart, const unsigned* binCount, const unsigned* binList, int tiles,
-                           int grid, float* visDepth, uint32_t* visSlot, uint8_t* visClass, StatPartials st,
-                           hipStream_t s);
+                           const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
+                           uint8_t* visClass, StatPartials st, hipStream_t s);
 // IDs from record slots: the primitive key >> 2, or for point and line records (polygon) the key's
 // triangle * 3 + its point or edge.
 void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32_t* visId, hipStream_t s,
@@ -303,10 +356,9 @@ void launch_shade(const ShadeParams& p, const Views& views, int shadeTiles, TriR
 // merge and shade launches).
 void launch_blend_ordered(const ShadeParams& p, const BlendCoefs& b, int depthFunc, int clear, unsigned binCap,
                           const Views& views, TriRecs recs, const float4* bary, const float* vtx, const int* idx,
-                          const TexDesc* tex, const uint8_t* texPool, const unsigned* binStart,
-                          const unsigned* binCount, const unsigned* binList, int tiles, int grid, float* visDepth,
-                          uint32_t* visSlot, uint8_t* visClass, uchar4* rgba8, float4* rgba32f, StatPartials st,
-                          hipStream_t s);
+                          const TexDesc* tex, const uint8_t* texPool, const BinBufs& bins, int tiles, int grid,
+                          float* visDepth, uint32_t* visSlot, uint8_t* visClass, uchar4* rgba8, float4* rgba32f,
+                          StatPartials st, hipStream_t s);
 
 // Point (mode 2) and line (mode 1) polygon modes, one sample per pixel (polygon.hip):
 // candidates per pixel meet in keys (order_key(depth) << 32 | primitive id),

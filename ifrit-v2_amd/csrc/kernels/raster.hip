@@ -218,31 +218,35 @@ __device__ __forceinline__ unsigned key_tie(unsigned long long k) {
     return S == 1 ? (unsigned)k >> 2 : (unsigned)k;
 }
 
-// The record slot of a key's triangle: ptr[prim] + fan from the slot map, or,
-// in a view where no triangle crossed w = 0 (direct != all ones), direct +
-// prim: the setup kernel puts triangle p in slot slotBase + p, and only the
-// clip kernel moves a triangle's slots.
+// The record slot of a key's triangle: the geometry kernel puts triangle p in
+// slot base + p, and only the triangles that crossed w = 0 (a bit per triangle
+// in the geometry waves' WaveInfo) have their fans from slot ptr[p] on.
 struct SlotMap {
     const unsigned* ptr;
-    unsigned direct;
+    const WaveInfo* waves;
+    unsigned base;
+    bool clips;  // the view has such triangles
 };
 
-// Record slots of a pixel's S final keys (slotOf[prim] + fan), all S lookups
-// issued before the first is used; a key that holds no fragment looks up
-// primitive 0 and its slot is not used.
+// Record slots of a pixel's S final keys, all S lookups issued before the first
+// is used; a key that holds no fragment looks up primitive 0 and its slot is
+// not used.
 template <int S>
 __device__ __forceinline__ void key_slots(const SlotMap& slotOf, const unsigned long long* keys,
                                           unsigned long long none, unsigned* slots) {
-    if (slotOf.direct != 0xffffffffu) {
-        // no triangle of the view was clipped: triangle p sits in slot slotBase + p
 #pragma unroll
-        for (int s = 0; s < S; s++) slots[s] = slotOf.direct + (key_tie<S>(keys[s]) >> 2);
-        return;
+    for (int s = 0; s < S; s++) slots[s] = slotOf.base + (key_tie<S>(keys[s]) >> 2);
+    if (!slotOf.clips) return;
+    unsigned long long m[S];
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        const unsigned prim = keys[s] != none ? key_tie<S>(keys[s]) >> 2 : 0u;
+        m[s] = slotOf.waves[prim >> 6].clipped >> (prim & 63u);
     }
 #pragma unroll
     for (int s = 0; s < S; s++) {
         const unsigned tie = key_tie<S>(keys[s]);
-        slots[s] = slotOf.ptr[keys[s] != none ? tie >> 2 : 0u] + (tie & 3u);
+        if (keys[s] != none && (m[s] & 1ull)) slots[s] = slotOf.ptr[tie >> 2] + (tie & 3u);
     }
 }
 
@@ -473,9 +477,8 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 template <int S, int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slotOfAll,
-         const unsigned* __restrict__ binList, const uint4* __restrict__ items, unsigned itemCap,
-         const unsigned* __restrict__ emptyList,
-         unsigned long long* __restrict__ partials, float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
+         const WaveInfo* __restrict__ waves, const unsigned* __restrict__ binList, RasterQueue q,
+         const unsigned* __restrict__ emptyEnd, float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
          uint8_t* __restrict__ visClassAll, StatPartials st, DeviceCounters* ctr) {
     constexpr int PASS = NT / 2;            // list entries per pass through LDS
     constexpr int UNITS = S == 1 ? NT * 16 : NT * 8;  // units expanded into LDS per round
@@ -493,11 +496,12 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
     __shared__ unsigned sItem;
 
     const int t = threadIdx.x;
-    const unsigned numItems = ctr->numItems, numLong = ctr->numLongItems;
+    const bool fits = plan_fits(ctr, q);
+    const unsigned numLong = ctr->tot[kTotLong], numItems = fits ? numLong + ctr->tot[kTotShort] : 0u;
     // tiles with an empty list follow the items: their clear values, KE tiles
     // per claim at 1 sample per pixel (a small write each)
     constexpr unsigned KE = S == 1 ? 8u : 1u;
-    const unsigned numEmpty = P.clear ? ctr->numEmpty : 0u;
+    const unsigned numEmpty = P.clear && fits ? ctr->tot[kTotEmpty] : 0u;
     const unsigned numEmptyItems = (numEmpty + KE - 1u) / KE;
     unsigned long long frags = 0, covs = 0;
 
@@ -521,13 +525,13 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             if (e >= numEmptyItems) break;
             if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             for (unsigned k = e * KE; k < min(e * KE + KE, numEmpty); k++)
-                clear_tile<S, NT>(view_of_tile(V, (int)emptyList[k]), P.clearDepth, P.scissor, visDepthAll,
+                clear_tile<S, NT>(view_of_tile(V, (int)*(emptyEnd - k)), P.clearDepth, P.scissor, visDepthAll,
                                   visSlotAll, visClassAll);
             __syncthreads();  // every lane has read sItem
             continue;
         }
         // long items from the front of the array, then short ones from its back
-        const uint4 it = items[item < numLong ? item : itemCap - 1u - (item - numLong)];
+        const uint4 it = q.items[item < numLong ? item : q.itemCap - 1u - (item - numLong)];
         const int tile = __builtin_amdgcn_readfirstlane((int)it.x);
         const unsigned first = __builtin_amdgcn_readfirstlane(it.y);
         const int cnt = __builtin_amdgcn_readfirstlane((int)it.z);
@@ -536,7 +540,8 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         float* const visDepth = visDepthAll + G.pixBase * S;
         uint32_t* const visSlot = visSlotAll + G.pixBase * S;
         uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
-        const SlotMap slotOf{slotOfAll + G.primBase, V.ctr[G.view].clipInCount == 0u ? G.slotBase : 0xffffffffu};
+        const SlotMap slotOf{slotOfAll + G.primBase, waves + (size_t)G.view * V.waves, G.slotBase,
+                             V.ctr[G.view].clipIn != 0u};
         const int ttx = G.tile % G.tilesX, tty = G.tile / G.tilesX;
         const int tx0 = ttx * 16, ty0 = tty * 16;
 
@@ -745,7 +750,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (pslot != 0xFFFFFFFFu) {
             // one item of a longer list: its keys, sample-major like sVis
-            unsigned long long* g = partials + (size_t)pslot * 256 * S;
+            unsigned long long* g = q.partials + (size_t)pslot * 256 * S;
 #pragma unroll
             for (int k = 0; k < PPT; k++)
 #pragma unroll
@@ -801,29 +806,26 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
 template <int S>
 __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, TriRecs recs,
                                                       const unsigned* __restrict__ slotOfAll,
+                                                      const WaveInfo* __restrict__ waves,
                                                       const unsigned* __restrict__ binStart,
-                                                      const unsigned* __restrict__ binCount,
-                                                      const unsigned* __restrict__ multiList,
-                                                      const int* __restrict__ tilePartial,
-                                                      const unsigned long long* __restrict__ partials,
+                                                      const unsigned* __restrict__ binEnd, RasterQueue q,
                                                       float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
-                                                      uint8_t* __restrict__ visClassAll, int tiles, int partShift,
-                                                      const DeviceCounters* ctr) {
-    const unsigned numMulti = ctr->numMulti;
+                                                      uint8_t* __restrict__ visClassAll, const DeviceCounters* ctr) {
+    const unsigned numMulti = plan_fits(ctr, q) ? ctr->tot[kTotMulti] : 0u;
     const int t = threadIdx.x;
     // tiles whose list was cut into several items: the minimum over their partial blocks
     for (unsigned m = blockIdx.x; m < numMulti; m += gridDim.x) {
-        const int tile = (int)multiList[m];
+        const int tile = (int)q.multiList[m];
         const ViewGeom G = view_of_tile(V, tile);
         float* const visDepth = visDepthAll + G.pixBase * S;
         uint32_t* const visSlot = visSlotAll + G.pixBase * S;
         uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
-        const SlotMap slotOf{slotOfAll + G.primBase, V.ctr[G.view].clipInCount == 0u ? G.slotBase : 0xffffffffu};
+        const SlotMap slotOf{slotOfAll + G.primBase, waves + (size_t)G.view * V.waves, G.slotBase,
+                             V.ctr[G.view].clipIn != 0u};
         const PixelCtx C = pixel_ctx(G, t & 15, t >> 4);
-        const unsigned start = binStart[tile];
-        const unsigned total = start >= P.binCap ? 0u : min(binCount[tile], P.binCap - start);
-        const unsigned nparts = (total + (1u << partShift) - 1u) >> partShift;
-        const unsigned long long* g = partials + (size_t)tilePartial[tile] * 256 * S + t;
+        const unsigned total = binEnd[tile] - binStart[tile];
+        const unsigned nparts = (total + (1u << q.partShift) - 1u) >> q.partShift;
+        const unsigned long long* g = q.partials + (size_t)q.tilePartial[tile] * 256 * S + t;
         unsigned long long keys[S];
 #pragma unroll
         for (int s = 0; s < S; s++) keys[s] = g[s * 256];
@@ -862,7 +864,7 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
 template <int S>
 __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V, TriRecs recs,
                                                         const unsigned* __restrict__ binStart,
-                                                        const unsigned* __restrict__ binCount,
+                                                        const unsigned* __restrict__ binEnd,
                                                         const unsigned* __restrict__ binList, int tiles,
                                                         float* __restrict__ visDepthAll,
                                                         uint32_t* __restrict__ visSlotAll,
@@ -886,7 +888,7 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
         }
         if (!P.clear && S == 1 && visClass && C.inFb) cls = visClass[C.pix];
         const unsigned start = binStart[tile];
-        const unsigned cnt = start >= P.binCap ? 0u : min(binCount[tile], P.binCap - start);
+        const unsigned cnt = start >= P.binCap ? 0u : min(binEnd[tile] - start, P.binCap - start);
         for_each_ordered(recs, binList, start, cnt, sA, sB, [&](unsigned ent) {
             const unsigned sl = ent & 0x7fffffffu;
             const bool full = (ent >> 31) != 0;
@@ -983,14 +985,11 @@ void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32
 
 // The raster and merge launches are separate so that the host can time them.
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
-                   const unsigned* binStart, const unsigned* binCount, const unsigned* binList, const RasterQueue& q,
-                   int tiles, float* visDepth, uint32_t* visSlot, uint8_t* visClass, StatPartials st,
-                   DeviceCounters* ctr, hipStream_t s) {
-    (void)binStart;
-    (void)binCount;
-#define IFRIT_RASTER_LAUNCH(SN, NT)                                                                                 \
-    hipLaunchKernelGGL((k_raster<SN, NT>), dim3(q.grid), dim3(NT), 0, s, p, views, recs, slotOf, binList, q.items, \
-                       q.itemCap, q.multiList + tiles, q.partials, visDepth, visSlot, visClass, st, ctr)
+                   const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
+                   uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s) {
+#define IFRIT_RASTER_LAUNCH(SN, NT)                                                                                \
+    hipLaunchKernelGGL((k_raster<SN, NT>), dim3(q.grid), dim3(NT), 0, s, p, views, recs, slotOf, bins.waves,      \
+                       bins.list, q, q.multiList + tiles - 1, visDepth, visSlot, visClass, st, ctr)
     switch (samples) {
         case 1:
             if (q.tileThreads == 64)
@@ -1005,12 +1004,11 @@ void launch_raster(const RasterParams& p, const Views& views, int samples, TriRe
 }
 
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
-                           const unsigned* binStart, const unsigned* binCount, const unsigned* binList, int tiles,
-                           int grid, float* visDepth, uint32_t* visSlot, uint8_t* visClass, StatPartials st,
-                           hipStream_t s) {
+                           const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
+                           uint8_t* visClass, StatPartials st, hipStream_t s) {
 #define IFRIT_ORDERED_LAUNCH(SN)                                                                                  \
-    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, binStart, binCount,     \
-                       binList, tiles, visDepth, visSlot, visClass, st)
+    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, bins.start, bins.cursor, \
+                       bins.list, tiles, visDepth, visSlot, visClass, st)
     switch (samples) {
         case 1: IFRIT_ORDERED_LAUNCH(1); break;
         case 4: IFRIT_ORDERED_LAUNCH(4); break;
@@ -1020,12 +1018,13 @@ void launch_raster_ordered(const RasterParams& p, const Views& views, int sample
 }
 
 void launch_raster_merge(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
-                         const unsigned* binStart, const unsigned* binCount, const RasterQueue& q, float* visDepth,
-                         uint32_t* visSlot, uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s) {
+                         const BinBufs& bins, const RasterQueue& q, float* visDepth, uint32_t* visSlot,
+                         uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s) {
+    // a workgroup per tile at most
+    const int grid = std::max(1, std::min(2 * q.mergeGrid, tiles));
 #define IFRIT_MERGE_LAUNCH(SN)                                                                                     \
-    hipLaunchKernelGGL(k_raster_merge<SN>, dim3(2 * q.mergeGrid), dim3(256), 0, s, p, views, recs, slotOf, binStart, \
-                       binCount, q.multiList, q.tilePartial, q.partials, visDepth, visSlot, visClass, tiles,       \
-                       q.partShift, ctr)
+    hipLaunchKernelGGL(k_raster_merge<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, slotOf, bins.waves,       \
+                       bins.start, bins.cursor, q, visDepth, visSlot, visClass, ctr)
     switch (samples) {
         case 1: IFRIT_MERGE_LAUNCH(1); break;
         case 4: IFRIT_MERGE_LAUNCH(4); break;

@@ -38,7 +38,8 @@ struct ShadeTri {
 // The ntri slots below fanStart (the view's first clip fan slot) are the
 // unclipped triangles, triangle p in slot fanStart - ntri + p: their
 // primitive comes from the slot itself, so the vertex indices can be read in
-// the same round trip as the record (a fan slot reads its key first).  The
+// the same round trip as the record (a fan slot reads its key first, and its
+// vertex weights from the view's `bary`).  The
 // record's planes are read last: a load still in flight when the two kinds
 // of slot rejoin would otherwise be waited for there.
 __device__ __forceinline__ void load_shade_tri(const TriRecs& recs, const float4* bary, unsigned fanStart,
@@ -51,7 +52,7 @@ __device__ __forceinline__ void load_shade_tri(const TriRecs& recs, const float4
         T.by[0] = 1.0f; T.by[1] = 0.0f; T.by[2] = 0.0f;
     } else {
         T.prim = (int)(__float_as_uint(recs.q2[slot].y) >> 2);
-        const float4 a = bary[2 * slot], b = bary[2 * slot + 1];
+        const float4 a = bary[2 * (slot - fanStart)], b = bary[2 * (slot - fanStart) + 1];
         T.bx[0] = a.x; T.bx[1] = a.y; T.bx[2] = a.z;
         T.by[0] = a.w; T.by[1] = b.x; T.by[2] = b.y;
     }
@@ -59,6 +60,12 @@ __device__ __forceinline__ void load_shade_tri(const TriRecs& recs, const float4
     T.f1 = recs.f1[slot];
     T.f2 = recs.f2[slot];
     T.f3 = recs.f3[slot];
+}
+
+// Where a view's fan weights start: its clip capacity of fans follows the
+// previous view's (the point and line modes, one view, have ntri = 0).
+__device__ __forceinline__ size_t view_bary(const Views& V, unsigned view, int ntri) {
+    return 2 * (size_t)view * (V.slotsPerView - (unsigned)ntri);
 }
 
 // Perspective-correct weights of the three original vertices at (x, y).
@@ -901,15 +908,18 @@ constexpr int kShadeRun = 64;
 
 template <int S, bool NEURAL, bool FP8, int N, bool LAYERED, bool GENERIC = false>
 __device__ __forceinline__ void shade_tiles(const ShadeParams& P, const Views& V, const TriRecs& recs,
-                                            const float4* __restrict__ bary, const uint32_t* __restrict__ visSlot,
-                                            const float* __restrict__ vtx, const int* __restrict__ idx,
-                                            const TexDesc* __restrict__ tex, const uint8_t* __restrict__ pool,
-                                            uchar4* __restrict__ rgba8, float4* __restrict__ rgba32f, int tiles) {
+                                            const float4* __restrict__ baryAll,
+                                            const uint32_t* __restrict__ visSlot, const float* __restrict__ vtx,
+                                            const int* __restrict__ idx, const TexDesc* __restrict__ tex,
+                                            const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8,
+                                            float4* __restrict__ rgba32f, int tiles) {
     constexpr int T = 8 * N;
     const int g = (int)(blockIdx.x >> 3);
     const int tile = (g / kShadeRun) * (8 * kShadeRun) + (int)(blockIdx.x & 7u) * kShadeRun + g % kShadeRun;
     if (tile >= tiles) return;
-    const ViewDesc& D = V.desc[V.shadeView[tile]];
+    const unsigned view = V.shadeView[tile];
+    const ViewDesc& D = V.desc[view];
+    const float4* const bary = baryAll + view_bary(V, view, P.ntri);
     const int width = D.width, height = D.height;
     const int local = tile - (int)D.shadeBase, perRow = (width + T - 1) / T;
     const int ox0 = (local % perRow) * T, oy0 = (local / perRow) * T;
@@ -1003,11 +1013,12 @@ using dev::load_rec;
 // visibility (last writer), the FP32 colour and its RGBA8 rounding.
 __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs B, int depthFunc, int clear,
                                                        unsigned binCap, Views V, TriRecs recs,
-                                                       const float4* __restrict__ bary, const float* __restrict__ vtx,
-                                                       const int* __restrict__ idx, const TexDesc* __restrict__ tex,
+                                                       const float4* __restrict__ baryAll,
+                                                       const float* __restrict__ vtx, const int* __restrict__ idx,
+                                                       const TexDesc* __restrict__ tex,
                                                        const uint8_t* __restrict__ pool,
                                                        const unsigned* __restrict__ binStart,
-                                                       const unsigned* __restrict__ binCount,
+                                                       const unsigned* __restrict__ binEnd,
                                                        const unsigned* __restrict__ binList, int tiles,
                                                        float* __restrict__ visDepthAll,
                                                        uint32_t* __restrict__ visSlotAll,
@@ -1019,6 +1030,7 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const ViewDesc& D = V.desc[V.tileView[tile]];
         const rc::ViewGeom G = rc::view_of_tile(V, tile);
+        const float4* const bary = baryAll + view_bary(V, (unsigned)G.view, P.ntri);
         const rc::PixelCtx C = rc::pixel_ctx(G, t & 15, t >> 4);
         const size_t pix = G.pixBase + C.pix;
         const float3 cam = make_float3(D.camera[0], D.camera[1], D.camera[2]);
@@ -1035,7 +1047,7 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
             col = rgba32fAll[pix];
         }
         const unsigned start = binStart[tile];
-        const unsigned cnt = start >= binCap ? 0u : min(binCount[tile], binCap - start);
+        const unsigned cnt = start >= binCap ? 0u : min(binEnd[tile] - start, binCap - start);
         rc::for_each_ordered(recs, binList, start, cnt, sA, sB, [&](unsigned ent) {
             const unsigned sl = ent & 0x7fffffffu;
             const bool full = (ent >> 31) != 0;
@@ -1123,12 +1135,11 @@ k_shade_neural(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ 
 
 void launch_blend_ordered(const ShadeParams& p, const BlendCoefs& b, int depthFunc, int clear, unsigned binCap,
                           const Views& views, TriRecs recs, const float4* bary, const float* vtx, const int* idx,
-                          const TexDesc* tex, const uint8_t* texPool, const unsigned* binStart,
-                          const unsigned* binCount, const unsigned* binList, int tiles, int grid, float* visDepth,
-                          uint32_t* visSlot, uint8_t* visClass, uchar4* rgba8, float4* rgba32f, StatPartials st,
-                          hipStream_t s) {
+                          const TexDesc* tex, const uint8_t* texPool, const BinBufs& bins, int tiles, int grid,
+                          float* visDepth, uint32_t* visSlot, uint8_t* visClass, uchar4* rgba8, float4* rgba32f,
+                          StatPartials st, hipStream_t s) {
     hipLaunchKernelGGL(k_blend_ordered, dim3(grid), dim3(256), 0, s, p, b, depthFunc, clear, binCap, views, recs, bary,
-                       vtx, idx, tex, texPool, binStart, binCount, binList, tiles, visDepth, visSlot, visClass, rgba8,
+                       vtx, idx, tex, texPool, bins.start, bins.cursor, bins.list, tiles, visDepth, visSlot, visClass, rgba8,
                        rgba32f, st);
 }
 
