@@ -1019,10 +1019,13 @@ StatPartials TileRasterRenderer::statPtrs() const {
     return st;
 }
 
-// Raster workgroups: rasterGroupsPerCU_ per compute unit, four times as many
-// when a 1-sample tile takes one wave.
+// Raster workgroups: five for every four of rasterGroupsPerCU_ per compute unit
+// (five fit at 1 and 4 samples; at 8, where four do, the fifth starts as one
+// ends, which evens out the tail), four times rasterGroupsPerCU_ when a 1-sample
+// tile takes one wave.
 int TileRasterRenderer::rasterGrid() const {
-    return numCUs_ * rasterGroupsPerCU_ * (samples_ == 1 && tileThreads_ == 64 ? 4 : 1);
+    const int groups = numCUs_ * rasterGroupsPerCU_;
+    return samples_ == 1 && tileThreads_ == 64 ? groups * 4 : (groups * 5 + 3) / 4;
 }
 
 // Uniform block of the bound fragment program for the shading kernels.

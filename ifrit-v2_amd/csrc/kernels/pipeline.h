@@ -33,7 +33,7 @@ namespace ifrit_hip {
 
 // One assembled triangle for coverage and depth (6 x 16 bytes):
 //   q0 = e1.xyz, e2.x   q1 = e2.yz, e3.xy
-//   q2 = e3.z, key, 0, 0
+//   q2 = e3.z, key, pixel box lo, hi (common/pixel_box.h: no sample outside it is covered)
 //   f1, f2, f3 = interpolation bases (x, y, z) and vz = (z/w) * w.
 // key = prim * 4 + fan orders fragments the way the reference's per-tile
 // sort by originalPrimitive does (TileRasterWorker.cpp:1244-1258).

@@ -13,14 +13,22 @@
 // (depth, prim * 4 + fan), which is order-independent: visibility is held as
 // 64-bit keys (ordered depth << 32 | prim * 4 + fan) merged with atomic min.
 //
-// Work expansion.  Two lanes per list entry (one per half tile) run the block
-// tests and build the entry's candidate mask: pixels (MSAA) or 4x2 groups (1
-// sample) of the blocks that pass trivial reject, pruned by a monotone corner
-// bound of the pixel test, which is exact.  A workgroup scan turns the masks into a flat
-// list of (entry, pixel or group) units in LDS, and every lane then takes
-// one unit: its sample tests, depths and LDS atomic-min merges.  Lanes stay
-// busy whatever the mix of triangle sizes, which one-triangle-per-lane loops
-// do not achieve.
+// Work expansion.  One lane per list entry lists the entry's 4x4 windows: those
+// that its pixel box (the record's proven bound) covers where they are at most
+// four, wherever they start, else the tile's blocks that pass trivial reject.
+// One lane per (entry, window) then finds the window's pixels: at 1 sample the
+// covered ones, each with its coverage class, with MSAA those whose unit square
+// the triangle may cover (a monotone corner bound of the sample test, exact).
+// Workgroup scans turn both into flat lists in LDS, and every lane takes one
+// (entry, pixel) unit: its sample tests, depths and LDS atomic-min merges.
+// Lanes stay busy whatever the mix of triangle sizes, which one-triangle-per-
+// lane loops do not achieve, and a triangle of a few pixels costs one window.
+//
+// Block reject and, with MSAA, block accept decide nothing that the sample test
+// does not: a block's corner minimises (maximises) every edge over it and
+// rounding is monotone, so a rejected block has no covered sample and an
+// accepted one no other.  Only the binner's whole-tile accept (another
+// expression) and, at 1 sample, the class of an accepted block do.
 //
 // Scheduling.  A tile's list is cut into parts of at most 1 << partShift entries and
 // all parts form one work queue that a persistent grid drains, so a few
@@ -35,6 +43,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "raster_common.h"
 
@@ -60,21 +69,7 @@ __device__ __forceinline__ void merge(unsigned long long* cell, float d, unsigne
     if (d == d) atomicMin(cell, frag_key(d, tie));
 }
 
-// Rejects every integer point of [x, x + w] x [y, y + h] when an edge
-// excludes the corner that minimises it; rounding is monotone, so no such
-// point can pass inside() when this returns false.
-__device__ __forceinline__ bool rect_may_cover(const Edges& E, float x, float y, float w, float h) {
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const float cx = E.x[k] < 0.0f ? x + w : x;
-        const float cy = E.y[k] < 0.0f ? y + h : y;
-        ok &= fmaf(E.y[k], cy, E.x[k] * cx) < ifx::neg(E.z[k]);
-    }
-    return ok;
-}
-
-// rect_may_cover of the 16 unit squares of the 4x4 block at (x0, y0), bit
+// square_may_cover of the 16 unit squares of the 4x4 window at (x0, y0), bit
 // 4 * row + column: the same products and fused sums per square (corners
 // are small integers, so x0 + column + 1 is exact either way), with each
 // edge's column products and row corners shared and no branches.
@@ -92,20 +87,20 @@ __device__ __forceinline__ unsigned block_square_mask(const Edges& E, float x0, 
     }
     unsigned m = 0;
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
+    for (int q = 15; q >= 0; q--) {  // bits shifted in from the last: no constant per bit
         const int i = q & 3, j = q >> 2;
         const unsigned c = (unsigned)(fmaf(E.y[0], cy[0][j], ax[0][i]) < nz[0]) &
                            (unsigned)(fmaf(E.y[1], cy[1][j], ax[1][i]) < nz[1]) &
                            (unsigned)(fmaf(E.y[2], cy[2][j], ax[2][i]) < nz[2]);
-        m |= c << q;
+        m = m + m + c;
     }
     return m;
 }
 
 // Exclusive scan over an NT-thread workgroup (64 or 256); every thread must call it.
 template <int NT>
-__device__ __forceinline__ unsigned scan_nt(unsigned v, unsigned* sWave, unsigned& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__device__ __forceinline__ unsigned scan_nt(int t, unsigned v, unsigned* sWave, unsigned& total) {
+    const int lane = t & 63, w = t >> 6;
     const unsigned x = wave_incl_scan(v);
     if constexpr (NT == 64) {
         total = __shfl(x, 63, 64);
@@ -134,27 +129,72 @@ __device__ __forceinline__ unsigned long long sum_nt(unsigned long long v) {
     }
 }
 
-// block_test of the eight 4x4 blocks of tile half h (blocks 8h .. 8h + 7,
-// block rows 2h and 2h + 1): bit j of tr when block 8h + j is not rejected,
-// of ta when it is trivially accepted; a tile-accepted entry (full) takes
-// every block.
-__device__ __forceinline__ void half_blocks(const Edges& E, bool full, int tx, int ty, int h, unsigned& tr,
-                                            unsigned& ta) {
-    if (full) {
-        tr = ta = 0xFFu;
-        return;
-    }
-    const float tileMinX = (float)(tx * 16) * 1.0f, tileMinY = (float)(ty * 16) * 1.0f;
-    tr = 0;
-    ta = 0;
+// The tile's 4x4 blocks (bit 4 * row + column) that pass trivial reject: the
+// corner that minimises an edge is inside it, for all three edges.
+__device__ __forceinline__ unsigned blocks_not_rejected(const Edges& E, int tx0, int ty0) {
+    float ax[3][4], cy[3][4], nz[3];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int bi = 8 * h + j;
-        int trn, tan;
-        block_test(E, fmaf((float)(bi & 3), 4.0f, tileMinX), fmaf((float)(bi >> 2), 4.0f, tileMinY), trn, tan);
-        tr |= (unsigned)(trn == 3) << j;
-        ta |= (unsigned)(tan == 3) << j;
+    for (int k = 0; k < 3; k++) {
+        const float ox = E.x[k] < 0.0f ? 4.0f : 0.0f, oy = E.y[k] < 0.0f ? 4.0f : 0.0f;
+        nz[k] = ifx::neg(E.z[k]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            ax[k][i] = E.x[k] * ((float)(tx0 + 4 * i) + ox);
+            cy[k][i] = (float)(ty0 + 4 * i) + oy;
+        }
     }
+    unsigned m = 0;
+#pragma unroll
+    for (int q = 15; q >= 0; q--) {  // bits shifted in from the last: no constant per bit
+        const int i = q & 3, j = q >> 2;
+        const unsigned c = (unsigned)(fmaf(E.y[0], cy[0][j], ax[0][i]) < nz[0]) &
+                           (unsigned)(fmaf(E.y[1], cy[1][j], ax[1][i]) < nz[1]) &
+                           (unsigned)(fmaf(E.y[2], cy[2][j], ax[2][i]) < nz[2]);
+        m = m + m + c;
+    }
+    return m;
+}
+
+// The pixels of the 4x4 window at (x0, y0) that pass the pixel test at their
+// corner (1 sample per pixel), bit 4 * row + column.
+__device__ __forceinline__ unsigned window_inside(const Edges& E, float x0, float y0) {
+    float ax[3][4], nz[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        nz[k] = ifx::neg(E.z[k]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) ax[k][i] = E.x[k] * (x0 + (float)i);
+    }
+    unsigned m = 0;
+#pragma unroll
+    for (int q = 15; q >= 0; q--) {  // as in blocks_not_rejected
+        const float y = y0 + (float)(q >> 2);
+        const unsigned c = (unsigned)(fmaf(E.y[0], y, ax[0][q & 3]) < nz[0]) &
+                           (unsigned)(fmaf(E.y[1], y, ax[1][q & 3]) < nz[1]) &
+                           (unsigned)(fmaf(E.y[2], y, ax[2][q & 3]) < nz[2]);
+        m = m + m + c;
+    }
+    return m;
+}
+
+// 4x4 block trivial accept (block_test): the corner that maximises each edge is inside it.
+__device__ __forceinline__ bool block_accepted(const Edges& E, float bMinX, float bMinY) {
+    int trn, tan;
+    block_test(E, bMinX, bMinY, trn, tan);
+    return tan == 3;
+}
+
+// Of the covered pixels m of the 4x4 window at tile column ox and row oy, those
+// whose 4x2 group (groups) and whose 2x2 quad (quads) is all covered.  A group or
+// quad that reaches out of the window is not: a window off the blocks' grid
+// holds every pixel its triangle can cover.
+__device__ __forceinline__ void window_classes(unsigned m, int ox, int oy, unsigned& groups, unsigned& quads) {
+    const unsigned rows = oy & 1 ? 0x00F0u : 0x0F0Fu;  // rows where a quad starts
+    const unsigned h = m & (m >> 1);
+    const unsigned q = h & (h >> 4) & rows & (ox & 1 ? 0x2222u : 0x5555u);
+    quads = q | (q << 1) | (q << 4) | (q << 5);
+    const unsigned r = (ox & 3) == 0 ? h & (h >> 2) & 0x1111u : 0u;  // full rows
+    groups = (r & (r >> 4) & rows) * 0xFFu;
 }
 
 // Pixels of a 4x4 block inside the frame (bit 4 * row + column), given the
@@ -163,33 +203,6 @@ __device__ __forceinline__ unsigned block_fb_mask(int ncols, int nrows) {
     const unsigned c = ncols >= 4 ? 0xFu : (ncols <= 0 ? 0u : (1u << ncols) - 1u);
     const unsigned r = nrows >= 4 ? 0xFFFFu : (nrows <= 0 ? 0u : (1u << (4 * nrows)) - 1u);
     return (c * 0x1111u) & r;
-}
-
-// Candidate 4x2 groups of one half of a tile at 1 sample per pixel for one
-// list entry (two lanes share an entry): 16 bits (block - 8h) * 2 + row
-// pair, masked by fbMask.  Also returns the trivially accepted blocks of the
-// half (bit block - 8h).
-__device__ __forceinline__ void group_mask_half(const Edges& E, bool full, int tx, int ty, int h, unsigned fbMask,
-                                                unsigned& m, unsigned& ta) {
-    unsigned tr;
-    half_blocks(E, full, tx, ty, h, tr, ta);
-    if (full) {
-        m = fbMask;
-        return;
-    }
-    m = 0;
-    while (tr) {
-        const int j = __ffs(tr) - 1;
-        tr &= tr - 1u;
-        const int bi = 8 * h + j;
-        const float x0 = (float)(tx * 16 + (bi & 3) * 4), y0 = (float)(ty * 16 + (bi >> 2) * 4);
-        unsigned g = 3u;
-        if (!((ta >> j) & 1u))
-            g = (unsigned)rect_may_cover(E, x0, y0, 3.0f, 1.0f) |
-                ((unsigned)rect_may_cover(E, x0, y0 + 2.0f, 3.0f, 1.0f) << 1);
-        m |= g << (j * 2);
-    }
-    m &= fbMask;
 }
 
 // Coverage class and depth of the winning triangle at a 1-sample pixel,
@@ -203,7 +216,7 @@ __device__ __forceinline__ unsigned winner_class(const TriRec& R, int tx, int ty
         block_test(E, bMinX, bMinY, trn, tan);
         accepted = tan == 3;
     }
-    const unsigned c = pixel_class(E, accepted, fpx, fpy, bMinX, tagging);
+    const unsigned c = pixel_class<1>(E, accepted, fpx, fpy, bMinX, tagging);  // rare: few registers, not speed
     d = class_depth(c, R.f1, R.f2, R.f3, fpx, fpy, tagging);
     return c;
 }
@@ -391,12 +404,12 @@ __device__ __forceinline__ void emit_pixel(const RasterParams& P, const TriRecs&
 // view's outputs; a view's first pixel starts a 16-byte line when S > 1 or its
 // pixel base is a multiple of 4.
 template <int S, int NT = 256>
-__device__ __forceinline__ void store_tile(const ViewGeom& G, int tx, int ty, const TileOut<S>* O,
+__device__ __forceinline__ void store_tile(int t, const ViewGeom& G, int tx, int ty, const TileOut<S>* O,
                                            float* visDepth, uint32_t* visSlot) {
     constexpr int perRow = 16 * S / 4;  // float4 per tile row
     const int cols = min(16, G.width - tx * 16), rows = min(16, G.height - ty * 16);
     const bool vec = cols == 16 && (S > 1 || ((G.width & 3) == 0 && (G.pixBase & 3) == 0));
-    for (int i = threadIdx.x; i < 64 * S; i += NT) {
+    for (int i = t; i < 64 * S; i += NT) {
         const int row = i / perRow, q = i - row * perRow;
         if (row >= rows) continue;
         const size_t g = ((size_t)(ty * 16 + row) * G.width + tx * 16) * S + q * 4;
@@ -423,7 +436,7 @@ __device__ __forceinline__ void store_tile(const ViewGeom& G, int tx, int ty, co
 // 0xffffffff and, at 1 sample per pixel, class 0) by NT threads, with 16-byte
 // stores where the tile's rows are whole.
 template <int S, int NT>
-__device__ __forceinline__ void clear_tile(const ViewGeom& G, float clearDepth, const Scissor& sc,
+__device__ __forceinline__ void clear_tile(int t, const ViewGeom& G, float clearDepth, const Scissor& sc,
                                            float* visDepthAll, uint32_t* visSlotAll, uint8_t* visClassAll) {
     const int tx = G.tile % G.tilesX, ty = G.tile / G.tilesX;
     const int cols = min(16, G.width - tx * 16), rows = min(16, G.height - ty * 16);
@@ -432,7 +445,7 @@ __device__ __forceinline__ void clear_tile(const ViewGeom& G, float clearDepth, 
     float* const visDepth = visDepthAll + G.pixBase * S;
     uint32_t* const visSlot = visSlotAll + G.pixBase * S;
     constexpr int perRow = 16 * S / 4;  // 16-byte words per tile row
-    for (int i = threadIdx.x; i < 64 * S; i += NT) {
+    for (int i = t; i < 64 * S; i += NT) {
         const int row = i / perRow, q = i - row * perRow;
         if (row >= rows) continue;
         const size_t g = ((size_t)(ty * 16 + row) * G.width + tx * 16) * S + q * 4;
@@ -452,7 +465,7 @@ __device__ __forceinline__ void clear_tile(const ViewGeom& G, float clearDepth, 
     }
     if (S == 1 && visClassAll) {
         uint8_t* const visClass = visClassAll + G.pixBase;
-        for (int i = threadIdx.x; i < 256; i += NT) {
+        for (int i = t; i < 256; i += NT) {
             const int row = i >> 4, col = i & 15;
             if (row < rows && col < cols &&
                 (whole || scissor_pass(sc, (float)(tx * 16 + col), (float)(ty * 16 + row))))
@@ -472,30 +485,36 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 
 // NT threads per tile: 256 (one pixel per thread) or, at 1 sample per pixel,
 // 64 (one wave per tile, four pixels per lane: more tiles in flight per
-// compute unit, for many small tiles).  Passes hold NT / 2 entries.  Held to
-// 128 VGPRs so that four workgroups of 256 share a compute unit.
+// compute unit, for many small tiles).  Passes hold NT / 2 entries.
+//
+// Bound by the latency of an item's chain (claim, item, view, list entries,
+// records, then the window and unit rounds) and by VALU issue: 63 % of its
+// cycles at 1920x1080, 8 samples, 1.3M triangles, 41 % at 1 sample.  Held to the
+// registers of five workgroups per compute unit at 1 and 4 samples (at 8 the
+// keys' LDS allows four).  Windows from pixel boxes, one lane per entry, instead of block
+// tests of every entry by two: 105 -> 84 us there, and 78 us with fewer registers; 4.2M
+// half-pixel triangles at 4 samples 327 -> 213 us, 34 views at 1 sample 525 -> 355 us.
 template <int S, int NT>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S == 8 ? 4 : 5, 8)))
 k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slotOfAll,
          const WaveInfo* __restrict__ waves, const unsigned* __restrict__ binList, RasterQueue q,
          const unsigned* __restrict__ emptyEnd, float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
          uint8_t* __restrict__ visClassAll, StatPartials st, DeviceCounters* ctr) {
     constexpr int PASS = NT / 2;            // list entries per pass through LDS
-    constexpr int UNITS = S == 1 ? NT * 16 : NT * 8;  // units expanded into LDS per round
-    constexpr int PAIRS = S == 1 ? 1 : 16 * PASS;     // (entry, block) pairs of a pass (S > 1)
+    constexpr int UNITS = NT * 8;           // units expanded into LDS per round
+    constexpr int PAIRS = 16 * PASS;        // (entry, window) pairs of a pass
+    using Unit = typename std::conditional<S == 1, unsigned, unsigned short>::type;
     constexpr int PPT = 256 / NT;           // tile pixels per thread
-    static_assert(PASS <= kPass, "units encode the entry in 7 bits");
+    static_assert(PASS <= kPass, "pairs and units encode the entry in 7 bits");
     // key of sample s of tile pixel p at vis_at(s, p)
     __shared__ unsigned long long sVis[S * kVisStride];
     static_assert(sizeof(TileOut<S>) <= sizeof(sVis), "output staging reuses sVis");
-    __shared__ TriRec sRec[PASS];
-    __shared__ unsigned char sTa[2 * PASS];  // accepted blocks of each half
-    __shared__ unsigned short sUnit[UNITS];
-    __shared__ unsigned short sPair[PAIRS];
+    __shared__ TriRec sRec[PASS];            // q2.z: bit 31 when the tile is accepted, else the pixel box
+    __shared__ Unit sUnit[UNITS];            // entry << 8 | tile pixel, and << 2 | class at 1 sample
+    __shared__ unsigned short sPair[PAIRS];  // entry << 9 | window row << 5 | column << 1 | a tile's block
     __shared__ unsigned sWave[4];
     __shared__ unsigned sItem;
 
-    const int t = threadIdx.x;
     const bool fits = plan_fits(ctr, q);
     const unsigned numLong = ctr->tot[kTotLong], numItems = fits ? numLong + ctr->tot[kTotShort] : 0u;
     // tiles with an empty list follow the items: their clear values, KE tiles
@@ -515,8 +534,12 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         (__attribute__((address_space(1))) unsigned*)&ctr->itemHeads[stream][0];
     asm volatile("" : "+v"(head));
     unsigned claimed = 0;
-    if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
+        // opaque to the compiler, which would otherwise keep every thread's share of the
+        // output and clear stages' index arithmetic in registers across the whole loop
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
         if (t == 0) sItem = claimed;
         __syncthreads();
         const unsigned item = sItem * kItemStreams + stream;
@@ -525,7 +548,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             if (e >= numEmptyItems) break;
             if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             for (unsigned k = e * KE; k < min(e * KE + KE, numEmpty); k++)
-                clear_tile<S, NT>(view_of_tile(V, (int)*(emptyEnd - k)), P.clearDepth, P.scissor, visDepthAll,
+                clear_tile<S, NT>(t, view_of_tile(V, (int)*(emptyEnd - k)), P.clearDepth, P.scissor, visDepthAll,
                                   visSlotAll, visClassAll);
             __syncthreads();  // every lane has read sItem
             continue;
@@ -554,67 +577,32 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                 sVis[vis_at(s, p)] = frag_key(P.clear || !C.inFb ? P.clearDepth : visDepth[C.pix * S + s], 0u);
         }
 
-        // two lanes per list entry: lane h = t & 1 takes block rows 2h, 2h + 1
-        const int e0 = t >> 1, h = t & 1;
-        // frame mask of this half tile: 4x2 groups with a pixel inside (S == 1;
-        // pixels are checked again per unit), blocks with a pixel inside (S > 1)
         const int cols = min(16, G.width - tx0), rows = min(16, G.height - ty0);
-        unsigned fbMask = 0, blkFb = 0;
-        if constexpr (S == 1) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const int g = 16 * h + j;
-                fbMask |= (unsigned)(((g >> 1) & 3) * 4 < cols && ((g >> 3) * 4 + (g & 1) * 2) < rows) << j;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; j++) blkFb |= (unsigned)((j & 3) * 4 < cols && (2 * h + (j >> 2)) * 4 < rows) << j;
-        }
+        // blocks with a pixel inside the frame
+        const unsigned blkFb = ((1u << ((cols + 3) >> 2)) - 1u) * 0x1111u & ((1u << (4 * ((rows + 3) >> 2))) - 1u);
 
-        // merges units sUnit[0, nu) (entry << 8 | tile pixel or group) into sVis
+        // merges units sUnit[0, nu) into sVis
         auto merge_units = [&](int nu) {
             for (int i = t; i < nu; i += NT) {
-                const unsigned u = sUnit[i];
-                const int e = (int)(u >> 8), c = (int)(u & 255u);
-                const TriRec R = sRec[e];
-                const Edges E = load_edges(R);
-                const unsigned tie = __float_as_uint(R.q2.y);
+                unsigned u = sUnit[i];
                 if constexpr (S == 1) {
-                    const int bi = c >> 1;
-                    const unsigned ta = sTa[2 * e + (bi >> 3)];
-                    const int px0 = tx0 + (bi & 3) * 4, gy = ty0 + (bi >> 2) * 4 + (c & 1) * 2;
-                    // pixels of the 4x2 group: (0,0) (1,0) (0,1) (1,1) (2,0) (3,0) (2,1) (3,1)
-                    const bool accepted = (ta >> (bi & 7)) & 1u;
-                    unsigned acc = 0xFFu;
-                    if (!accepted) {
-                        acc = 0;
-#pragma unroll
-                        for (int l = 0; l < 8; l++) {
-                            const int ox = (l & 1) + ((l >> 2) << 1), oy = (l >> 1) & 1;
-                            acc |= (unsigned)inside(E, (float)(px0 + ox), (float)(gy + oy)) << l;
-                        }
-                    }
-                    // as with MSAA: every pixel's class depth is computed, only the merge is
-                    // conditional
-                    unsigned non = 0;
-#pragma unroll
-                    for (int l = 0; l < 8; l++) {
-                        const int px = px0 + (l & 1) + ((l >> 2) << 1), py = gy + ((l >> 1) & 1);
-                        const bool on = ((acc >> l) & 1u) & (px < G.width) & (py < G.height);
-                        const unsigned quad = (acc >> (l & 4)) & 0xFu;
-                        const unsigned cls = expr_code(accepted, acc == 0xFFu, quad == 0xFu, P.tagging);
-                        const float d = class_depth_all(cls, R.f1, R.f2, R.f3, (float)px, (float)py, P.tagging);
-                        non += on;
-                        if (on & (d == d))
-                            atomicMin(&sVis[vis_at(0, (py - ty0) * 16 + (px - tx0))], frag_key(d, (tie << 2) | cls));
-                    }
-                    frags += non;
-                    covs += non;
+                    const unsigned cls = u & 3u;
+                    u >>= 2;
+                    const int e = (int)(u >> 8), c = (int)(u & 255u);
+                    const float4 F1 = sRec[e].f1, F2 = sRec[e].f2, F3 = sRec[e].f3;
+                    const unsigned tie = __float_as_uint(sRec[e].q2.y);
+                    // every class's depth is computed and one selected: a wave's lanes hold all of them
+                    const float d = class_depth_all(cls, F1, F2, F3, (float)(tx0 + (c & 15)), (float)(ty0 + (c >> 4)),
+                                                    P.tagging);
+                    if (d == d) atomicMin(&sVis[vis_at(0, c)], frag_key(d, (tie << 2) | cls));
+                    frags++;
                 } else {
-                    const int lx = c & 15, ly = c >> 4;
-                    const int bi = (ly >> 2) * 4 + (lx >> 2);
-                    const bool accept = (sTa[2 * e + (bi >> 3)] >> (bi & 7)) & 1u;
-                    const float fx = (float)(tx0 + lx), fy = (float)(ty0 + ly);
+                    const int e = (int)(u >> 8), c = (int)(u & 255u);
+                    const TriRec R = sRec[e];
+                    const Edges E = load_edges(R);
+                    const unsigned tie = __float_as_uint(R.q2.y);
+                    const bool accept = (__float_as_uint(R.q2.z) >> 31) != 0u;
+                    const float fx = (float)(tx0 + (c & 15)), fy = (float)(ty0 + (c >> 4));
                     // every sample's coverage and depth are computed (the lanes of a
                     // wave cover different pixels, so branches would run both ways);
                     // only the merge is conditional
@@ -636,38 +624,112 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         // passes of PASS entries through LDS, all merging into sVis
         for (int pb = 0; pb < cnt; pb += PASS) {
             const int pc = min(PASS, cnt - pb);
-            if constexpr (S == 1) {
-                unsigned m = 0;
-                if (e0 < pc) {
-                    const unsigned ent = binList[first + pb + e0];
-                    const TriRec R = load_rec(recs, ent & 0x7fffffffu);
-                    if (h == 0) sRec[e0] = R;
-                    unsigned ta;
-                    group_mask_half(load_edges(R), (ent >> 31) != 0, ttx, tty, h, fbMask, m, ta);
-                    sTa[t] = (unsigned char)ta;
+            // one lane per entry: its windows
+            unsigned n = 0, blocks = 0;
+            int bx0 = 0, by0 = 0, wcols = 0;
+            if (t < pc) {
+                const unsigned ent = binList[first + pb + t];
+                const TriRec R = load_rec(recs, ent & 0x7fffffffu);
+                sRec[t] = R;
+                const Edges E = load_edges(R);
+                const bool full = (ent >> 31) != 0u;
+                const unsigned lo = __float_as_uint(R.q2.z), hi = __float_as_uint(R.q2.w);
+                // the pixel box within the tile
+                const int x0 = max((int)(lo & 0xFFFFu) - tx0, 0), y0 = max((int)(lo >> 16) - ty0, 0);
+                const int x1 = min((int)(hi & 0xFFFFu) - tx0, 15), y1 = min((int)(hi >> 16) - ty0, 15);
+                if (full) {
+                    blocks = blkFb;
+                    n = (unsigned)__popc(blocks);
+                } else if (x0 <= x1 && y0 <= y1) {
+                    // at 1 sample a window off the blocks' grid must hold the whole box (window_classes)
+                    constexpr int kFew = S == 1 ? 4 : 8;
+                    if (x1 - x0 < kFew && y1 - y0 < kFew) {
+                        wcols = (x1 - x0 + 4) >> 2;
+                        n = (unsigned)(wcols * ((y1 - y0 + 4) >> 2));
+                        bx0 = x0;
+                        by0 = y0;
+                    } else {
+                        blocks = blocks_not_rejected(E, tx0, ty0) & blkFb;
+                        n = (unsigned)__popc(blocks);
+                    }
                 }
-                const unsigned n = (unsigned)__popc(m);
+                // the box within the tile, for the window lanes; an accepted tile has none
+                sRec[t].q2.z = __uint_as_float(full ? 0x80000000u
+                                                    : (unsigned)(x0 | (y0 << 4) | (max(x1, 0) << 8) | (max(y1, 0) << 12)));
+            }
+            unsigned TP;
+            int pp = (int)scan_nt<NT>(t, n, sWave, TP);
+            if (blocks) {
+                while (blocks) {
+                    const int q = __ffs(blocks) - 1;
+                    blocks &= blocks - 1u;
+                    sPair[pp++] = (unsigned short)((t << 9) | ((q >> 2) << 7) | ((q & 3) << 3) | 1);
+                }
+            } else {
+                for (int k = 0; k < (int)n; k++) {
+                    const int wx = bx0 + 4 * few_col(k, wcols), wy = by0 + 4 * few_row(k, wcols);
+                    sPair[pp++] = (unsigned short)((t << 9) | (wy << 5) | (wx << 1));
+                }
+            }
+            __syncthreads();
+            for (unsigned p0 = 0; p0 < TP; p0 += NT) {
+                // one lane per window: its pixels
+                unsigned pm = 0, groups = 0, quads = 0;
+                int pe = 0, wx = 0, wy = 0;
+                bool acc = false;
+                if (p0 + t < TP) {
+                    const unsigned pr = sPair[p0 + t];
+                    pe = (int)(pr >> 9);
+                    wx = (int)((pr >> 1) & 15u);
+                    wy = (int)((pr >> 5) & 15u);
+                    const unsigned bits = __float_as_uint(sRec[pe].q2.z);
+                    acc = (bits >> 31) != 0u;  // the tile, or below the block, is accepted
+                    // up to the frame's and the box's last column and row
+                    const int lx = acc ? cols : min(cols, (int)((bits >> 8) & 15u) + 1);
+                    const int ly = acc ? rows : min(rows, (int)((bits >> 12) & 15u) + 1);
+                    pm = block_fb_mask(lx - wx, ly - wy);
+                    if (!acc) {
+                        const Edges E = load_edges(sRec[pe]);
+                        const float fx = (float)(tx0 + wx), fy = (float)(ty0 + wy);
+                        if constexpr (S == 1) {
+                            if (pr & 1u) acc = block_accepted(E, fx, fy);
+                            const unsigned in = window_inside(E, fx, fy);
+                            window_classes(in, wx, wy, groups, quads);
+                            pm &= in;
+                        } else {
+                            pm &= block_square_mask(E, fx, fy);
+                        }
+                    }
+                }
+                const int np = __popc(pm);
                 unsigned T;
-                const unsigned off = scan_nt<NT>(n, sWave, T);
-
+                const unsigned off = scan_nt<NT>(t, (unsigned)np, sWave, T);
                 for (unsigned w0 = 0; w0 < T; w0 += UNITS) {
-                    // write this lane's units that fall in [w0, w0 + UNITS): entry << 8 | group
+                    // write this lane's units that fall in [w0, w0 + UNITS): window pixel b is tile
+                    // pixel (wy + (b >> 2)) * 16 + wx + (b & 3)
                     int pos = (int)off - (int)w0;
-                    if (n && pos < UNITS && pos + (int)n > 0) {
-                        unsigned bits = m;
-                        const int cb = (e0 << 8) | (16 * h);
-                        if (pos >= 0 && pos + (int)n <= UNITS) {
+                    if (np && pos < UNITS && pos + np > 0) {
+                        const int cb = (pe << 8) | (wy * 16 + wx);
+                        auto unit = [&](int b) {
+                            const unsigned u = (unsigned)(cb + ((b >> 2) << 4) + (b & 3));
+                            if constexpr (S == 1)
+                                return (Unit)((u << 2) | expr_code(acc, (groups >> b) & 1u, (quads >> b) & 1u, P.tagging));
+                            else
+                                return (Unit)u;
+                        };
+                        unsigned bits = pm;
+                        if (pos >= 0 && pos + np <= UNITS) {
                             // the lane's units all fall in this window
                             while (bits) {
                                 const int b = __ffs(bits) - 1;
                                 bits &= bits - 1u;
-                                sUnit[pos++] = (unsigned short)(cb + b);
+                                sUnit[pos++] = unit(b);
                             }
                         } else {
                             while (bits) {
                                 const int b = __ffs(bits) - 1;
                                 bits &= bits - 1u;
-                                if (pos >= 0 && pos < UNITS) sUnit[pos] = (unsigned short)(cb + b);
+                                if (pos >= 0 && pos < UNITS) sUnit[pos] = unit(b);
                                 pos++;
                             }
                         }
@@ -676,75 +738,9 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                     merge_units((int)min((unsigned)UNITS, T - w0));
                     __syncthreads();
                 }
-            } else {
-                // entry lanes find the blocks their half may cover; every
-                // (entry, block) pair then takes one lane for its pixel mask
-                unsigned tr = 0;
-                if (e0 < pc) {
-                    const unsigned ent = binList[first + pb + e0];
-                    const TriRec R = load_rec(recs, ent & 0x7fffffffu);
-                    if (h == 0) sRec[e0] = R;
-                    unsigned ta;
-                    half_blocks(load_edges(R), (ent >> 31) != 0, ttx, tty, h, tr, ta);
-                    tr &= blkFb;
-                    sTa[t] = (unsigned char)ta;
-                }
-                unsigned TP;
-                int pp = (int)scan_nt<NT>((unsigned)__popc(tr), sWave, TP);
-                while (tr) {
-                    const int j = __ffs(tr) - 1;
-                    tr &= tr - 1u;
-                    sPair[pp++] = (unsigned short)((e0 << 4) | (8 * h + j));
-                }
-                __syncthreads();
-                for (unsigned p0 = 0; p0 < TP; p0 += NT) {
-                    unsigned pm = 0;
-                    int pe = 0, bi = 0;
-                    if (p0 + t < TP) {
-                        const unsigned pr = sPair[p0 + t];
-                        pe = (int)(pr >> 4);
-                        bi = (int)(pr & 15u);
-                        pm = block_fb_mask(cols - (bi & 3) * 4, rows - (bi >> 2) * 4);
-                        if (!((sTa[2 * pe + (bi >> 3)] >> (bi & 7)) & 1u)) {
-                            const Edges E = load_edges(sRec[pe]);
-                            pm &= block_square_mask(E, (float)(tx0 + (bi & 3) * 4), (float)(ty0 + (bi >> 2) * 4));
-                        }
-                    }
-                    const int n = __popc(pm);
-                    unsigned T;
-                    const unsigned off = scan_nt<NT>((unsigned)n, sWave, T);
-                    for (unsigned w0 = 0; w0 < T; w0 += UNITS) {
-                        // write this lane's units that fall in [w0, w0 + UNITS): tile pixel
-                        // (4 (bi >> 2) + (b >> 2)) * 16 + 4 (bi & 3) + (b & 3) of block bit b
-                        int pos = (int)off - (int)w0;
-                        if (n && pos < UNITS && pos + n > 0) {
-                            unsigned bits = pm;
-                            const int cb = (pe << 8) | ((bi >> 2) * 64 + (bi & 3) * 4);
-                            if (pos >= 0 && pos + n <= UNITS) {
-                                // the lane's units all fall in this window
-                                while (bits) {
-                                    const int b = __ffs(bits) - 1;
-                                    bits &= bits - 1u;
-                                    sUnit[pos++] = (unsigned short)(cb + ((b >> 2) << 4) + (b & 3));
-                                }
-                            } else {
-                                while (bits) {
-                                    const int b = __ffs(bits) - 1;
-                                    bits &= bits - 1u;
-                                    if (pos >= 0 && pos < UNITS)
-                                        sUnit[pos] = (unsigned short)(cb + ((b >> 2) << 4) + (b & 3));
-                                    pos++;
-                                }
-                            }
-                        }
-                        __syncthreads();
-                        merge_units((int)min((unsigned)UNITS, T - w0));
-                        __syncthreads();
-                    }
-                    if (T == 0) __syncthreads();  // sWave is read by the next round's scan
-                }
+                if (T == 0) __syncthreads();  // sWave is read by the next round's scan
             }
-            __syncthreads();  // sRec, sTa and sWave are reused by the next pass
+            __syncthreads();  // sRec and sWave are reused by the next pass
         }
 
         if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -780,7 +776,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                                        visDepth, visSlot);
                     }
                     __syncthreads();
-                    store_tile<S, NT>(G, ttx, tty, O, visDepth, visSlot);
+                    store_tile<S, NT>(t, G, ttx, tty, O, visDepth, visSlot);
                 }
             } else {
 #pragma unroll
@@ -794,8 +790,8 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         __syncthreads();  // every lane has read sItem and the LDS of this item
     }
     const unsigned long long tf = sum_nt<NT>(frags);
-    const unsigned long long tc = sum_nt<NT>(covs);
-    if (t == 0) {
+    const unsigned long long tc = S == 1 ? tf : sum_nt<NT>(covs);  // at 1 sample a fragment is a covered sample
+    if (threadIdx.x == 0) {
         st.rasterFrags[blockIdx.x] = tf;
         st.rasterCovs[blockIdx.x] = tc;
     }
@@ -842,7 +838,7 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
                 __syncthreads();          // the previous tile's staging has been stored
                 stage_pixel<S>(P, recs, slotOf, C, t, keys, O, visClass, visDepth, visSlot);
                 __syncthreads();
-                store_tile<S>(G, C.tx, C.ty, &O, visDepth, visSlot);
+                store_tile<S>(t, G, C.tx, C.ty, &O, visDepth, visSlot);
             }
         } else {
             write_pixel<S>(P, recs, slotOf, C, keys, visDepth, visSlot, visClass);

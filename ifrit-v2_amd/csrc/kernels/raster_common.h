@@ -149,17 +149,18 @@ __device__ __forceinline__ bool covers(const Edges& E, bool full, int tan, int t
 
 // Expression code of a covered 1-sample pixel (class_depth): accepted, its
 // 4x2 group all inside, its 2x2 quad all inside, or a single pixel.
+template <int UNROLL = 8>
 __device__ __forceinline__ unsigned pixel_class(const Edges& E, bool accepted, float fpx, float fpy, float bMinX,
                                                 bool tagging) {
     if (accepted) return expr_code(true, false, false, tagging);
     const float gy = floorf(fpy * 0.5f) * 2.0f;
     bool g = true;
-#pragma unroll
+#pragma unroll UNROLL
     for (int l = 0; l < 8; l++) g = g && inside(E, bMinX + (float)(l & 3), gy + (float)(l >> 2));
     if (g) return 1u;
     const float qx = floorf(fpx * 0.5f) * 2.0f;
     bool q = true;
-#pragma unroll
+#pragma unroll UNROLL
     for (int l = 0; l < 4; l++) q = q && inside(E, qx + (float)(l & 1), gy + (float)(l >> 1));
     return expr_code(false, false, q, tagging);
 }
