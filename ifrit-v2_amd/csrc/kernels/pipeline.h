@@ -17,7 +17,8 @@
 //   entry       uint2, uint4[N][64 waves] per triangle, its bin entries or tile rectangle (WaveInfo)
 //   fanBox      uint2[N][clipCap]         tile rectangle of each clip fan
 //   slotOf      uint[N][T]                first fan slot of each clipped primitive (its fans follow)
-//   binCnt      uint2[tiles]              entries counted: triangles of up to four tiles, others
+//   binCnt      uint2[tiles]              entries counted: triangles of up to four tiles, others (zero
+//                                         after the plan, then marks of tiles with NaN depths)
 //   binStart/binCursor  uint[tiles]       a tile's list; after binning the cursor is its end
 //   binList     uint[binCap]              slot | 0x80000000 when the tile is fully covered
 //   visId/visDepth/visSlot  [pixels * S]  per-sample winner; views one after another, pixels
@@ -189,6 +190,10 @@ struct RasterParams {
     float depthScale, depthBias;
     Scissor scissor;
     unsigned binCap;
+    // cleared draws with a depth function other than LESS that is a minimum of keys (raster.hip
+    // general_key)
+    int general, last;
+    unsigned keyXor, keyMask;
     float sx[8], sy[8];  // sample offsets from the pixel corner
 };
 
@@ -338,11 +343,12 @@ void launch_raster(const RasterParams& p, const Views& views, int samples, TriRe
 void launch_raster_merge(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                          const BinBufs& bins, const RasterQueue& q, float* visDepth, uint32_t* visSlot,
                          uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s);
-// Depth functions other than LESS: each tile's list in primitive order, folded
-// per pixel (replaces launch_raster and launch_raster_merge).
+// Depth functions that are no minimum: each tile's list in primitive order, folded
+// per pixel (replaces launch_raster and launch_raster_merge); with nanTilesOnly the tiles in which
+// they met a NaN depth (after launch_raster_merge of a general draw).
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
                            const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
-                           uint8_t* visClass, StatPartials st, hipStream_t s);
+                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, hipStream_t s);
 // IDs from record slots: the primitive key >> 2, or for point and line records (polygon) the key's
 // triangle * 3 + its point or edge.
 void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32_t* visId, hipStream_t s,

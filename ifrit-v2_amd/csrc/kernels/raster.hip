@@ -65,10 +65,6 @@ __device__ __forceinline__ bool inside_and(const Edges& E, float x, float y) {
     return a & b & c;
 }
 
-__device__ __forceinline__ void merge(unsigned long long* cell, float d, unsigned tie) {
-    if (d == d) atomicMin(cell, frag_key(d, tie));
-}
-
 // square_may_cover of the 16 unit squares of the 4x4 window at (x0, y0), bit
 // 4 * row + column: the same products and fused sums per square (corners
 // are small integers, so x0 + column + 1 is exact either way), with each
@@ -231,6 +227,31 @@ __device__ __forceinline__ unsigned key_tie(unsigned long long k) {
     return S == 1 ? (unsigned)k >> 2 : (unsigned)k;
 }
 
+// Keys of the other depth functions whose result is a minimum too, whatever the
+// order of the fragments (cleared draws): LESS_OR_EQUAL keeps the nearest and
+// among equal depths the last fragment, GREATER and GREATER_OR_EQUAL the
+// farthest, first or last, ALWAYS the last.  The depth's order is inverted by
+// keyXor and ignored by keyMask 0; `last` inverts the low word's, whose value is
+// then at least 1 (S == 1: the class bits; else the primitive key + 1), so that
+// no fragment meets the clear value's low word.
+template <int S>
+__device__ __forceinline__ unsigned long long general_key(const RasterParams& P, float d, unsigned tie) {
+    const unsigned hi = (order_key(d) ^ P.keyXor) & P.keyMask;
+    const unsigned lo = P.last ? ~(tie + (S > 1 ? 1u : 0u)) : tie;
+    return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long general_clear_key(const RasterParams& P) {
+    return ((unsigned long long)((order_key(P.clearDepth) ^ P.keyXor) & P.keyMask) << 32) | (P.last ? ~0u : 0u);
+}
+// A LESS key of the same fragment, for the output stage; ALWAYS keys, which hold no
+// depth, take the depth of +-0, whose value the output stage reads from the record.
+template <int S>
+__device__ __forceinline__ unsigned long long less_key(const RasterParams& P, unsigned long long k) {
+    const unsigned hi = P.keyMask ? (unsigned)(k >> 32) ^ P.keyXor : 0x80000000u;
+    const unsigned lo = P.last ? ~(unsigned)k - (S > 1 ? 1u : 0u) : (unsigned)k;
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 // The record slot of a key's triangle: the geometry kernel puts triangle p in
 // slot base + p, and only the triangles that crossed w = 0 (a bit per triangle
 // in the geometry waves' WaveInfo) have their fans from slot ptr[p] on.
@@ -242,53 +263,45 @@ struct SlotMap {
 };
 
 // Record slots of a pixel's S final keys, all S lookups issued before the first
-// is used; a key that holds no fragment looks up primitive 0 and its slot is
-// not used.
+// is used; a key that holds no fragment (its bit of `won` is 0) looks up
+// primitive 0 and its slot is not used.
 template <int S>
 __device__ __forceinline__ void key_slots(const SlotMap& slotOf, const unsigned long long* keys,
-                                          unsigned long long none, unsigned* slots) {
+                                          unsigned won, unsigned* slots) {
 #pragma unroll
     for (int s = 0; s < S; s++) slots[s] = slotOf.base + (key_tie<S>(keys[s]) >> 2);
     if (!slotOf.clips) return;
     unsigned long long m[S];
 #pragma unroll
     for (int s = 0; s < S; s++) {
-        const unsigned prim = keys[s] != none ? key_tie<S>(keys[s]) >> 2 : 0u;
+        const unsigned prim = (won >> s) & 1u ? key_tie<S>(keys[s]) >> 2 : 0u;
         m[s] = slotOf.waves[prim >> 6].clipped >> (prim & 63u);
     }
 #pragma unroll
     for (int s = 0; s < S; s++) {
         const unsigned tie = key_tie<S>(keys[s]);
-        if (keys[s] != none && (m[s] & 1ull)) slots[s] = slotOf.ptr[tie >> 2] + (tie & 3u);
+        if (((won >> s) & 1u) && (m[s] & 1ull)) slots[s] = slotOf.ptr[tie >> 2] + (tie & 3u);
     }
 }
 
-// Writes the outputs of one pixel from its S final keys: depth and record
-// slot per sample (the primitive ID is the slot's key >> 2, expanded only on
-// readback).
+// Writes the outputs of one pixel of a draw without clear from its S final keys:
+// depth and record slot per sample where a fragment won (the primitive ID is the
+// slot's key >> 2, expanded only on readback).
 template <int S>
 __device__ __forceinline__ void write_pixel(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
                                             const PixelCtx& C, const unsigned long long* keys, float* visDepth,
                                             uint32_t* visSlot, uint8_t* visClass) {
     if (!C.inFb || !scissor_pass(P.scissor, C.fpx, C.fpy)) return;
-    unsigned long long prev[S];
+    unsigned won = 0;
 #pragma unroll
-    for (int s = 0; s < S; s++) prev[s] = frag_key(P.clear ? P.clearDepth : visDepth[C.pix * S + s], 0u);
+    for (int s = 0; s < S; s++) won |= (unsigned)(keys[s] != frag_key(visDepth[C.pix * S + s], 0u)) << s;
     unsigned slots[S];
-    key_slots<S>(slotOf, keys, P.clear ? frag_key(P.clearDepth, 0u) : ~0ull, slots);
+    key_slots<S>(slotOf, keys, won, slots);
     unsigned cls = 0;
-    bool won = false;
 #pragma unroll
     for (int s = 0; s < S; s++) {
         const unsigned long long k = keys[s];
-        if (k == prev[s]) {
-            if (P.clear) {
-                visDepth[C.pix * S + s] = P.clearDepth;
-                visSlot[C.pix * S + s] = 0xffffffffu;
-            }
-            continue;
-        }
-        won = true;
+        if (!((won >> s) & 1u)) continue;
         const unsigned slot = slots[s];
         float d = order_key_inv((unsigned)(k >> 32));
         if (S == 1 && (unsigned)(k >> 32) == 0x80000000u) {
@@ -303,7 +316,7 @@ __device__ __forceinline__ void write_pixel(const RasterParams& P, const TriRecs
         visDepth[C.pix * S + s] = d;
         visSlot[C.pix * S + s] = slot;
     }
-    if (S == 1 && visClass && (won || P.clear)) visClass[C.pix] = class_out(cls, P.tagging);
+    if (S == 1 && visClass && won) visClass[C.pix] = class_out(cls, P.tagging);
 }
 
 // One tile's outputs staged in LDS in global order (pixel-major, sample-
@@ -316,23 +329,36 @@ struct TileOut {
     unsigned slot[256 * S];
 };
 
+// The S final keys of a cleared draw's pixel in the form the output stage takes
+// (LESS keys), and which of them hold a fragment.
+template <int S, bool G>
+__device__ __forceinline__ unsigned final_keys(const RasterParams& P, unsigned long long* keys) {
+    unsigned won = 0;
+    const unsigned long long none = G ? general_clear_key(P) : frag_key(P.clearDepth, 0u);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        won |= (unsigned)(keys[s] != none) << s;
+        if constexpr (G) keys[s] = less_key<S>(P, keys[s]);
+    }
+    return won;
+}
+
 // Outputs of one pixel of a cleared draw from its S final keys: depth and
 // record slot per sample (the clear values where no fragment won) and, at 1
 // sample per pixel, the coverage class.
 template <int S>
 __device__ __forceinline__ unsigned pixel_outputs(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
-                                                  const PixelCtx& C, const unsigned long long* keys, float* d,
-                                                  unsigned* slot) {
+                                                  const PixelCtx& C, const unsigned long long* keys, unsigned won,
+                                                  float* d, unsigned* slot) {
     unsigned cls = 0;
-    const unsigned long long clearKey = frag_key(P.clearDepth, 0u);
     unsigned slots[S];
-    key_slots<S>(slotOf, keys, clearKey, slots);
+    key_slots<S>(slotOf, keys, won, slots);
 #pragma unroll
     for (int s = 0; s < S; s++) {
         const unsigned long long k = keys[s];
         d[s] = P.clearDepth;
         slot[s] = 0xffffffffu;
-        if (k != clearKey) {
+        if ((won >> s) & 1u) {
             slot[s] = slots[s];
             d[s] = order_key_inv((unsigned)(k >> 32));
             if (S == 1 && (unsigned)(k >> 32) == 0x80000000u) {
@@ -355,8 +381,9 @@ __device__ __forceinline__ unsigned pixel_outputs(const RasterParams& P, const T
 // class byte goes straight out.
 template <int S>
 __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
-                                            const PixelCtx& C, int t, const unsigned long long* keys, TileOut<S>& O,
-                                            uint8_t* visClass, const float* visDepth, const uint32_t* visSlot) {
+                                            const PixelCtx& C, int t, const unsigned long long* keys, unsigned won,
+                                            TileOut<S>& O, uint8_t* visClass, const float* visDepth,
+                                            const uint32_t* visSlot) {
     if (!C.inFb) return;
     if (!scissor_pass(P.scissor, C.fpx, C.fpy)) {
         // outside the scissor: the tile's line stores write the pixel's current contents back
@@ -369,7 +396,7 @@ __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs
     }
     float d[S];
     unsigned slot[S];
-    const unsigned cls = pixel_outputs<S>(P, recs, slotOf, C, keys, d, slot);
+    const unsigned cls = pixel_outputs<S>(P, recs, slotOf, C, keys, won, d, slot);
 #pragma unroll
     for (int s = 0; s < S; s++) {
         O.d[t * S + s] = d[s];
@@ -383,13 +410,13 @@ __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs
 // a row of pixels whole lines).
 template <int S>
 __device__ __forceinline__ void emit_pixel(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
-                                           const PixelCtx& C, const unsigned long long* keys, float* visDepth,
+                                           const PixelCtx& C, const unsigned long long* keys, unsigned won, float* visDepth,
                                            uint32_t* visSlot) {
     static_assert(S % 4 == 0, "whole 16-byte words per pixel");
     if (!C.inFb || !scissor_pass(P.scissor, C.fpx, C.fpy)) return;
     float d[S];
     unsigned slot[S];
-    pixel_outputs<S>(P, recs, slotOf, C, keys, d, slot);
+    pixel_outputs<S>(P, recs, slotOf, C, keys, won, d, slot);
     float4* const dd = reinterpret_cast<float4*>(visDepth + C.pix * S);
     uint4* const ds = reinterpret_cast<uint4*>(visSlot + C.pix * S);
 #pragma unroll
@@ -485,7 +512,10 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 
 // NT threads per tile: 256 (one pixel per thread) or, at 1 sample per pixel,
 // 64 (one wave per tile, four pixels per lane: more tiles in flight per
-// compute unit, for many small tiles).  Passes hold NT / 2 entries.
+// compute unit, for many small tiles).  Passes hold NT / 2 entries.  G: the
+// general keys of a cleared draw with another depth function than LESS, which
+// also marks the tiles that met a NaN depth (nanTile): in those the function's
+// result depends on the order after all.
 //
 // Bound by the latency of an item's chain (claim, item, view, list entries,
 // records, then the window and unit rounds) and by VALU issue: 63 % of its
@@ -494,12 +524,12 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 // keys' LDS allows four).  Windows from pixel boxes, one lane per entry, instead of block
 // tests of every entry by two: 105 -> 84 us there, and 78 us with fewer registers; 4.2M
 // half-pixel triangles at 4 samples 327 -> 213 us, 34 views at 1 sample 525 -> 355 us.
-template <int S, int NT>
+template <int S, int NT, bool G = false>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S == 8 ? 4 : 5, 8)))
 k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slotOfAll,
          const WaveInfo* __restrict__ waves, const unsigned* __restrict__ binList, RasterQueue q,
          const unsigned* __restrict__ emptyEnd, float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
-         uint8_t* __restrict__ visClassAll, StatPartials st, DeviceCounters* ctr) {
+         uint8_t* __restrict__ visClassAll, StatPartials st, DeviceCounters* ctr, unsigned* __restrict__ nanTile) {
     constexpr int PASS = NT / 2;            // list entries per pass through LDS
     constexpr int UNITS = NT * 8;           // units expanded into LDS per round
     constexpr int PAIRS = 16 * PASS;        // (entry, window) pairs of a pass
@@ -559,27 +589,38 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         const unsigned first = __builtin_amdgcn_readfirstlane(it.y);
         const int cnt = __builtin_amdgcn_readfirstlane((int)it.z);
         const unsigned pslot = __builtin_amdgcn_readfirstlane(it.w);
-        const ViewGeom G = view_of_tile(V, tile);
-        float* const visDepth = visDepthAll + G.pixBase * S;
-        uint32_t* const visSlot = visSlotAll + G.pixBase * S;
-        uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
-        const SlotMap slotOf{slotOfAll + G.primBase, waves + (size_t)G.view * V.waves, G.slotBase,
-                             V.ctr[G.view].clipIn != 0u};
-        const int ttx = G.tile % G.tilesX, tty = G.tile / G.tilesX;
+        const ViewGeom G_ = view_of_tile(V, tile);
+        float* const visDepth = visDepthAll + G_.pixBase * S;
+        uint32_t* const visSlot = visSlotAll + G_.pixBase * S;
+        uint8_t* const visClass = visClassAll ? visClassAll + G_.pixBase : nullptr;
+        const SlotMap slotOf{slotOfAll + G_.primBase, waves + (size_t)G_.view * V.waves, G_.slotBase,
+                             V.ctr[G_.view].clipIn != 0u};
+        const int ttx = G_.tile % G_.tilesX, tty = G_.tile / G_.tilesX;
         const int tx0 = ttx * 16, ty0 = tty * 16;
 
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
             const int p = t + k * NT;
-            const PixelCtx C = pixel_ctx(G, p & 15, p >> 4);
+            const PixelCtx C = pixel_ctx(G_, p & 15, p >> 4);
 #pragma unroll
             for (int s = 0; s < S; s++)
-                sVis[vis_at(s, p)] = frag_key(P.clear || !C.inFb ? P.clearDepth : visDepth[C.pix * S + s], 0u);
+                sVis[vis_at(s, p)] =
+                    G ? general_clear_key(P)
+                      : frag_key(P.clear || !C.inFb ? P.clearDepth : visDepth[C.pix * S + s], 0u);
         }
 
-        const int cols = min(16, G.width - tx0), rows = min(16, G.height - ty0);
+        const int cols = min(16, G_.width - tx0), rows = min(16, G_.height - ty0);
         // blocks with a pixel inside the frame
         const unsigned blkFb = ((1u << ((cols + 3) >> 2)) - 1u) * 0x1111u & ((1u << (4 * ((rows + 3) >> 2))) - 1u);
+
+        auto merge = [&](unsigned long long* cell, bool on, float d, unsigned tie) {
+            if constexpr (G) {
+                if (on & ((d == d) | (P.keyMask == 0u))) atomicMin(cell, general_key<S>(P, d, tie));
+                if (on & (d != d) & (P.keyMask != 0u)) nanTile[2 * tile] = 1u;
+            } else {
+                if (on & (d == d)) atomicMin(cell, frag_key(d, tie));
+            }
+        };
 
         // merges units sUnit[0, nu) into sVis
         auto merge_units = [&](int nu) {
@@ -594,7 +635,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                     // every class's depth is computed and one selected: a wave's lanes hold all of them
                     const float d = class_depth_all(cls, F1, F2, F3, (float)(tx0 + (c & 15)), (float)(ty0 + (c >> 4)),
                                                     P.tagging);
-                    if (d == d) atomicMin(&sVis[vis_at(0, c)], frag_key(d, (tie << 2) | cls));
+                    merge(&sVis[vis_at(0, c)], true, d, (tie << 2) | cls);
                     frags++;
                 } else {
                     const int e = (int)(u >> 8), c = (int)(u & 255u);
@@ -613,7 +654,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                         const bool cov = accept | inside_and(E, sx, sy);
                         const float d = depth256(R.f1, R.f2, R.f3, sx, sy);
                         ncov += cov;
-                        if (cov & (d == d)) atomicMin(&sVis[vis_at(s, c)], frag_key(d, tie));
+                        merge(&sVis[vis_at(s, c)], cov, d, tie);
                     }
                     covs += ncov;
                     frags += ncov != 0u;
@@ -757,13 +798,14 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             for (int k = 0; k < PPT; k++)
 #pragma unroll
                 for (int s = 0; s < S; s++) keys[k][s] = sVis[vis_at(s, t + k * NT)];
-            if (P.clear) {
+            if (G || P.clear) {
                 if constexpr (S > 1) {
                     // a pixel's samples are whole 16-byte words: straight out
 #pragma unroll
                     for (int k = 0; k < PPT; k++) {
                         const int p = t + k * NT;
-                        emit_pixel<S>(P, recs, slotOf, pixel_ctx(G, p & 15, p >> 4), keys[k], visDepth, visSlot);
+                        const unsigned won = final_keys<S, G>(P, keys[k]);
+                        emit_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], won, visDepth, visSlot);
                     }
                 } else {
                     // every key is in registers: stage the outputs over sVis
@@ -772,17 +814,18 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
 #pragma unroll
                     for (int k = 0; k < PPT; k++) {
                         const int p = t + k * NT;
-                        stage_pixel<S>(P, recs, slotOf, pixel_ctx(G, p & 15, p >> 4), p, keys[k], *O, visClass,
+                        const unsigned won = final_keys<S, G>(P, keys[k]);
+                        stage_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), p, keys[k], won, *O, visClass,
                                        visDepth, visSlot);
                     }
                     __syncthreads();
-                    store_tile<S, NT>(t, G, ttx, tty, O, visDepth, visSlot);
+                    store_tile<S, NT>(t, G_, ttx, tty, O, visDepth, visSlot);
                 }
             } else {
 #pragma unroll
                 for (int k = 0; k < PPT; k++) {
                     const int p = t + k * NT;
-                    write_pixel<S>(P, recs, slotOf, pixel_ctx(G, p & 15, p >> 4), keys[k], visDepth, visSlot,
+                    write_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], visDepth, visSlot,
                                    visClass);
                 }
             }
@@ -831,12 +874,13 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
             for (int s = 0; s < S; s++) keys[s] = min(keys[s], g[s * 256]);
         }
         if (P.clear) {
+            const unsigned won = P.general ? final_keys<S, true>(P, keys) : final_keys<S, false>(P, keys);
             if constexpr (S > 1) {
-                emit_pixel<S>(P, recs, slotOf, C, keys, visDepth, visSlot);
+                emit_pixel<S>(P, recs, slotOf, C, keys, won, visDepth, visSlot);
             } else {
                 __shared__ TileOut<S> O;  // output staging at 1 sample per pixel
                 __syncthreads();          // the previous tile's staging has been stored
-                stage_pixel<S>(P, recs, slotOf, C, t, keys, O, visClass, visDepth, visSlot);
+                stage_pixel<S>(P, recs, slotOf, C, t, keys, won, O, visClass, visDepth, visSlot);
                 __syncthreads();
                 store_tile<S>(t, G, C.tx, C.ty, &O, visDepth, visSlot);
             }
@@ -847,16 +891,19 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
 }
 
 // ---------------------------------------------------------------------------
-// Ordered raster: depth functions other than LESS (and the depth test off,
-// which is ALWAYS).  Their result depends on the order of the fragments, so
-// each tile's list is taken in the order of the reference's per-tile sort
+// Ordered raster: what the keys cannot express -- EQUAL, NOT_EQUAL and NEVER,
+// GREATER at one sample (its scalar path), every function but LESS without
+// clear, depth-writing programs, and tiles with NaN depths.  The result
+// depends on the order of the fragments, so each tile's list is taken in the order of the reference's per-tile sort
 // (TileRasterWorker.cpp:1225-1259) and every thread folds the fragments of
 // its own pixel in that order (TileRasterWorker.cpp:2272-2311 and the SIMD
 // forms); the scalar path's GREATER tests nothing
 // (TileRasterWorker.cpp:2278-2280).
 // ---------------------------------------------------------------------------
 // One workgroup per tile (persistent over the tiles of all views), one
-// thread per pixel holding its S samples' depth and winning slot.
+// thread per pixel holding its S samples' depth and winning slot.  With nanTile
+// only the tiles it marks are drawn, over the key raster's result, and their
+// marks cleared.
 template <int S>
 __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V, TriRecs recs,
                                                         const unsigned* __restrict__ binStart,
@@ -864,11 +911,13 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
                                                         const unsigned* __restrict__ binList, int tiles,
                                                         float* __restrict__ visDepthAll,
                                                         uint32_t* __restrict__ visSlotAll,
-                                                        uint8_t* __restrict__ visClassAll, StatPartials st) {
+                                                        uint8_t* __restrict__ visClassAll, StatPartials st,
+                                                        unsigned* __restrict__ nanTile) {
     __shared__ unsigned long long sA[kOrderCap], sB[kOrderCap];
     const int t = threadIdx.x;
     unsigned long long frags = 0, covs = 0;
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        if (nanTile && nanTile[2 * tile] == 0u) continue;
         const ViewGeom G = view_of_tile(V, tile);
         const PixelCtx C = pixel_ctx(G, t & 15, t >> 4);
         float* const visDepth = visDepthAll + G.pixBase * S;
@@ -928,7 +977,12 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
             }
             if (S == 1 && visClass) visClass[C.pix] = (uint8_t)cls;
         }
+        if (nanTile) {
+            __syncthreads();  // every thread has read the mark
+            if (t == 0) nanTile[2 * tile] = 0u;
+        }
     }
+    if (nanTile) return;  // the key raster has counted
     const unsigned long long tf = block_sum256(frags);
     const unsigned long long tc = block_sum256(covs);
     if (t == 0) {
@@ -983,9 +1037,23 @@ void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                    const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
                    uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s) {
-#define IFRIT_RASTER_LAUNCH(SN, NT)                                                                                \
-    hipLaunchKernelGGL((k_raster<SN, NT>), dim3(q.grid), dim3(NT), 0, s, p, views, recs, slotOf, bins.waves,      \
-                       bins.list, q, q.multiList + tiles - 1, visDepth, visSlot, visClass, st, ctr)
+#define IFRIT_RASTER_LAUNCH(...)                                                                                   \
+    hipLaunchKernelGGL((k_raster<__VA_ARGS__>), dim3(q.grid), dim3(q.tileThreads), 0, s, p, views, recs, slotOf,  \
+                       bins.waves, bins.list, q, q.multiList + tiles - 1, visDepth, visSlot, visClass, st, ctr,   \
+                       bins.cnt)
+    if (p.general) {
+        switch (samples) {
+            case 1:
+                if (q.tileThreads == 64)
+                    IFRIT_RASTER_LAUNCH(1, 64, true);
+                else
+                    IFRIT_RASTER_LAUNCH(1, 256, true);
+                break;
+            case 4: IFRIT_RASTER_LAUNCH(4, 256, true); break;
+            default: IFRIT_RASTER_LAUNCH(8, 256, true); break;
+        }
+        return;
+    }
     switch (samples) {
         case 1:
             if (q.tileThreads == 64)
@@ -1001,10 +1069,10 @@ void launch_raster(const RasterParams& p, const Views& views, int samples, TriRe
 
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
                            const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
-                           uint8_t* visClass, StatPartials st, hipStream_t s) {
+                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, hipStream_t s) {
 #define IFRIT_ORDERED_LAUNCH(SN)                                                                                  \
     hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, bins.start, bins.cursor, \
-                       bins.list, tiles, visDepth, visSlot, visClass, st)
+                       bins.list, tiles, visDepth, visSlot, visClass, st, nanTilesOnly ? bins.cnt : nullptr)
     switch (samples) {
         case 1: IFRIT_ORDERED_LAUNCH(1); break;
         case 4: IFRIT_ORDERED_LAUNCH(4); break;
