@@ -1139,6 +1139,7 @@ void TileRasterRenderer::enqueue(bool clear) {
     rp.depthBias = fs_.desc.depthBias;
     rp.scissor = activeScissor();
     rp.binCap = binCap_;
+    rp.ntri = (unsigned)curTris_;
     // depth functions that are a minimum of keys on cleared draws; GREATER at one sample is not, as
     // its scalar path tests nothing outside the tagging mode (TRW:2278-2280)
     // (at 720p with 4 samples and 82k triangles the keys and their pass over NaN tiles take 36 us, the
@@ -1159,10 +1160,10 @@ void TileRasterRenderer::enqueue(bool clear) {
     uint8_t* cls = batch_.empty() ? visClass_.as<uint8_t>() : nullptr;
     if (blend_.blendEnable) {
         // blending: fragments shaded and blended in primitive order (the shade stage is part of it)
-        launch_blend_ordered(shadeParams(true), blendCoefs_, depthFunc_, clear ? 1 : 0, binCap_, V, recPtrs(),
+        launch_blend_ordered(shadeParams(true), blendCoefs_, depthFunc_, clear ? 1 : 0, V, recPtrs(),
                              bary_.as<float4>(), vtx_.as<float>(), idx_.as<int>(), texDesc_.as<TexDesc>(), texPool_,
-                             bins, tiles, rasterGrid(), visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, rgba8_.as<uchar4>(),
-                             rgba32f_.as<float4>(), statPtrs(), s);
+                             bins, q, tiles, visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, rgba8_.as<uchar4>(),
+                             rgba32f_.as<float4>(), statPtrs(), ctr_.as<DeviceCounters>(), s);
         mark(4);
     } else if ((depthFunc_ == IF_COMPARE_OP_LESS || rp.general) && !rp.depthWrite) {
         // order-independent: the lexicographic minimum of (depth, primitive), or of the general keys
@@ -1172,12 +1173,12 @@ void TileRasterRenderer::enqueue(bool clear) {
         launch_raster_merge(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), bins, q, visDepth_.as<float>(),
                             visSlot_.as<uint32_t>(), cls, tiles, ctr_.as<DeviceCounters>(), s);
         if (rp.general)
-            launch_raster_ordered(rp, V, samples_, recPtrs(), bins, tiles, rasterGrid(), visDepth_.as<float>(),
-                                  visSlot_.as<uint32_t>(), cls, statPtrs(), true, s);
+            launch_raster_ordered(rp, V, samples_, recPtrs(), bins, q, tiles, visDepth_.as<float>(),
+                                  visSlot_.as<uint32_t>(), cls, statPtrs(), true, ctr_.as<DeviceCounters>(), s);
     } else {
         // what is no minimum folds each pixel's fragments in primitive order
-        launch_raster_ordered(rp, V, samples_, recPtrs(), bins, tiles, rasterGrid(), visDepth_.as<float>(),
-                              visSlot_.as<uint32_t>(), cls, statPtrs(), false, s);
+        launch_raster_ordered(rp, V, samples_, recPtrs(), bins, q, tiles, visDepth_.as<float>(),
+                              visSlot_.as<uint32_t>(), cls, statPtrs(), false, ctr_.as<DeviceCounters>(), s);
         mark(4);
     }
     mark(5);

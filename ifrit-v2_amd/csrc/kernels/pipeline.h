@@ -189,7 +189,7 @@ struct RasterParams {
     int depthWrite;      // the fragment program stores depth * depthScale + depthBias after the test
     float depthScale, depthBias;
     Scissor scissor;
-    unsigned binCap;
+    unsigned binCap, ntri;
     // cleared draws with a depth function other than LESS that is a minimum of keys (raster.hip
     // general_key)
     int general, last;
@@ -347,8 +347,9 @@ void launch_raster_merge(const RasterParams& p, const Views& views, int samples,
 // per pixel (replaces launch_raster and launch_raster_merge); with nanTilesOnly the tiles in which
 // they met a NaN depth (after launch_raster_merge of a general draw).
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
-                           const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
-                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, hipStream_t s);
+                           const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
+                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, DeviceCounters* ctr,
+                           hipStream_t s);
 // IDs from record slots: the primitive key >> 2, or for point and line records (polygon) the key's
 // triangle * 3 + its point or edge.
 void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32_t* visId, hipStream_t s,
@@ -360,11 +361,11 @@ void launch_shade(const ShadeParams& p, const Views& views, int shadeTiles, TriR
 // Blending, 1 sample per pixel: the ordered traversal with the depth test, each
 // passing fragment shaded and blended in primitive order (replaces the raster,
 // merge and shade launches).
-void launch_blend_ordered(const ShadeParams& p, const BlendCoefs& b, int depthFunc, int clear, unsigned binCap,
+void launch_blend_ordered(const ShadeParams& p, const BlendCoefs& b, int depthFunc, int clear,
                           const Views& views, TriRecs recs, const float4* bary, const float* vtx, const int* idx,
-                          const TexDesc* tex, const uint8_t* texPool, const BinBufs& bins, int tiles, int grid,
-                          float* visDepth, uint32_t* visSlot, uint8_t* visClass, uchar4* rgba8, float4* rgba32f,
-                          StatPartials st, hipStream_t s);
+                          const TexDesc* tex, const uint8_t* texPool, const BinBufs& bins,
+                          const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot, uint8_t* visClass,
+                          uchar4* rgba8, float4* rgba32f, StatPartials st, DeviceCounters* ctr, hipStream_t s);
 
 // Point (mode 2) and line (mode 1) polygon modes, one sample per pixel (polygon.hip):
 // candidates per pixel meet in keys (order_key(depth) << 32 | primitive id),

@@ -65,34 +65,6 @@ __device__ __forceinline__ bool inside_and(const Edges& E, float x, float y) {
     return a & b & c;
 }
 
-// square_may_cover of the 16 unit squares of the 4x4 window at (x0, y0), bit
-// 4 * row + column: the same products and fused sums per square (corners
-// are small integers, so x0 + column + 1 is exact either way), with each
-// edge's column products and row corners shared and no branches.
-__device__ __forceinline__ unsigned block_square_mask(const Edges& E, float x0, float y0) {
-    float ax[3][4], cy[3][4], nz[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const float ox = E.x[k] < 0.0f ? 1.0f : 0.0f, oy = E.y[k] < 0.0f ? 1.0f : 0.0f;
-        nz[k] = ifx::neg(E.z[k]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            ax[k][i] = E.x[k] * ((x0 + (float)i) + ox);
-            cy[k][i] = (y0 + (float)i) + oy;
-        }
-    }
-    unsigned m = 0;
-#pragma unroll
-    for (int q = 15; q >= 0; q--) {  // bits shifted in from the last: no constant per bit
-        const int i = q & 3, j = q >> 2;
-        const unsigned c = (unsigned)(fmaf(E.y[0], cy[0][j], ax[0][i]) < nz[0]) &
-                           (unsigned)(fmaf(E.y[1], cy[1][j], ax[1][i]) < nz[1]) &
-                           (unsigned)(fmaf(E.y[2], cy[2][j], ax[2][i]) < nz[2]);
-        m = m + m + c;
-    }
-    return m;
-}
-
 // Exclusive scan over an NT-thread workgroup (64 or 256); every thread must call it.
 template <int NT>
 __device__ __forceinline__ unsigned scan_nt(int t, unsigned v, unsigned* sWave, unsigned& total) {
@@ -149,56 +121,6 @@ __device__ __forceinline__ unsigned blocks_not_rejected(const Edges& E, int tx0,
         m = m + m + c;
     }
     return m;
-}
-
-// The pixels of the 4x4 window at (x0, y0) that pass the pixel test at their
-// corner (1 sample per pixel), bit 4 * row + column.
-__device__ __forceinline__ unsigned window_inside(const Edges& E, float x0, float y0) {
-    float ax[3][4], nz[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        nz[k] = ifx::neg(E.z[k]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) ax[k][i] = E.x[k] * (x0 + (float)i);
-    }
-    unsigned m = 0;
-#pragma unroll
-    for (int q = 15; q >= 0; q--) {  // as in blocks_not_rejected
-        const float y = y0 + (float)(q >> 2);
-        const unsigned c = (unsigned)(fmaf(E.y[0], y, ax[0][q & 3]) < nz[0]) &
-                           (unsigned)(fmaf(E.y[1], y, ax[1][q & 3]) < nz[1]) &
-                           (unsigned)(fmaf(E.y[2], y, ax[2][q & 3]) < nz[2]);
-        m = m + m + c;
-    }
-    return m;
-}
-
-// 4x4 block trivial accept (block_test): the corner that maximises each edge is inside it.
-__device__ __forceinline__ bool block_accepted(const Edges& E, float bMinX, float bMinY) {
-    int trn, tan;
-    block_test(E, bMinX, bMinY, trn, tan);
-    return tan == 3;
-}
-
-// Of the covered pixels m of the 4x4 window at tile column ox and row oy, those
-// whose 4x2 group (groups) and whose 2x2 quad (quads) is all covered.  A group or
-// quad that reaches out of the window is not: a window off the blocks' grid
-// holds every pixel its triangle can cover.
-__device__ __forceinline__ void window_classes(unsigned m, int ox, int oy, unsigned& groups, unsigned& quads) {
-    const unsigned rows = oy & 1 ? 0x00F0u : 0x0F0Fu;  // rows where a quad starts
-    const unsigned h = m & (m >> 1);
-    const unsigned q = h & (h >> 4) & rows & (ox & 1 ? 0x2222u : 0x5555u);
-    quads = q | (q << 1) | (q << 4) | (q << 5);
-    const unsigned r = (ox & 3) == 0 ? h & (h >> 2) & 0x1111u : 0u;  // full rows
-    groups = (r & (r >> 4) & rows) * 0xFFu;
-}
-
-// Pixels of a 4x4 block inside the frame (bit 4 * row + column), given the
-// frame's columns and rows left from the block's corner.
-__device__ __forceinline__ unsigned block_fb_mask(int ncols, int nrows) {
-    const unsigned c = ncols >= 4 ? 0xFu : (ncols <= 0 ? 0u : (1u << ncols) - 1u);
-    const unsigned r = nrows >= 4 ? 0xFFFFu : (nrows <= 0 ? 0u : (1u << (4 * nrows)) - 1u);
-    return (c * 0x1111u) & r;
 }
 
 // Coverage class and depth of the winning triangle at a 1-sample pixel,
@@ -900,26 +822,37 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
 // forms); the scalar path's GREATER tests nothing
 // (TileRasterWorker.cpp:2278-2280).
 // ---------------------------------------------------------------------------
-// One workgroup per tile (persistent over the tiles of all views), one
-// thread per pixel holding its S samples' depth and winning slot.  With nanTile
+// One workgroup per tile (persistent over the tiles of all views, in the order
+// of OrderedTiles), one thread per pixel holding its S samples' depth and winning
+// slot; bound as k_blend_ordered is.  With nanTile
 // only the tiles it marks are drawn, over the key raster's result, and their
 // marks cleared.
 template <int S>
 __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V, TriRecs recs,
-                                                        const unsigned* __restrict__ binStart,
-                                                        const unsigned* __restrict__ binEnd,
-                                                        const unsigned* __restrict__ binList, int tiles,
+                                                        BinBufs B, RasterQueue q, int tiles, unsigned ntri,
                                                         float* __restrict__ visDepthAll,
                                                         uint32_t* __restrict__ visSlotAll,
                                                         uint8_t* __restrict__ visClassAll, StatPartials st,
-                                                        unsigned* __restrict__ nanTile) {
-    __shared__ unsigned long long sA[kOrderCap], sB[kOrderCap];
+                                                        unsigned* __restrict__ nanTile, DeviceCounters* ctr) {
+    __shared__ OrderLds L;
+    __shared__ unsigned sItem;
     const int t = threadIdx.x;
     unsigned long long frags = 0, covs = 0;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        if (nanTile && nanTile[2 * tile] == 0u) continue;
+    OrderedTiles T(q, ctr, nanTile == nullptr);
+    int tile = (int)blockIdx.x - (int)gridDim.x;
+    for (;;) {
+        unsigned start, cnt;
+        if (nanTile) {
+            tile += gridDim.x;
+            if (tile >= tiles) break;
+            if (nanTile[2 * tile] == 0u) continue;
+            start = B.start[tile];
+            cnt = start >= P.binCap ? 0u : min(B.cursor[tile] - start, P.binCap - start);
+        } else if (!T.next(q, B, tiles, &sItem, tile, start, cnt)) {
+            break;
+        }
         const ViewGeom G = view_of_tile(V, tile);
-        const PixelCtx C = pixel_ctx(G, t & 15, t >> 4);
+        const PixelCtx C = pixel_ctx(G, quarter_x(t), quarter_y(t));
         float* const visDepth = visDepthAll + G.pixBase * S;
         uint32_t* const visSlot = visSlotAll + G.pixBase * S;
         uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
@@ -932,43 +865,36 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
             slot[s] = P.clear || !C.inFb ? 0xffffffffu : visSlot[C.pix * S + s];
         }
         if (!P.clear && S == 1 && visClass && C.inFb) cls = visClass[C.pix];
-        const unsigned start = binStart[tile];
-        const unsigned cnt = start >= P.binCap ? 0u : min(binEnd[tile] - start, P.binCap - start);
-        for_each_ordered(recs, binList, start, cnt, sA, sB, [&](unsigned ent) {
-            const unsigned sl = ent & 0x7fffffffu;
-            const bool full = (ent >> 31) != 0;
-            if (!C.inFb) return;
-            const TriRec R = load_rec(recs, sl);
-            const Edges E = load_edges(R);
-            int trn, tan;
-            block_test(E, C.bMinX, C.bMinY, trn, tan);
-            if constexpr (S == 1) {
-                if (!covers(E, full, tan, trn, C.fpx, C.fpy)) return;
-                const unsigned c = pixel_class(E, full || tan == 3, C.fpx, C.fpy, C.bMinX, P.tagging);
-                const float d = class_depth(c, R.f1, R.f2, R.f3, C.fpx, C.fpy, P.tagging);
-                frags++;
-                covs++;
-                // the scalar path's GREATER quirk belongs to the deterministic mode's single pixels
-                if (!depth_pass(P.depthFunc, d, dep[0], c == 3u && !P.tagging)) return;
-                dep[0] = P.depthWrite ? d * P.depthScale + P.depthBias : d;
-                slot[0] = sl;
-                cls = class_out(c, P.tagging);
-            } else {
-                bool any = false;
-#pragma unroll
-                for (int s = 0; s < S; s++) {
-                    const float sx = C.fpx + P.sx[s], sy = C.fpy + P.sy[s];
-                    if (!covers(E, full, tan, trn, sx, sy)) continue;
-                    any = true;
+        for_each_ordered<S>(
+            recs, B.list, start, cnt, G.slotBase, ntri, C, P.tagging, L,
+            [&](const TriRec& R, unsigned sl, unsigned c) {
+                if (!C.inFb) return;
+                if constexpr (S == 1) {
+                    const float d = class_depth(c, R.f1, R.f2, R.f3, C.fpx, C.fpy, P.tagging);
+                    frags++;
                     covs++;
-                    const float d = depth256(R.f1, R.f2, R.f3, sx, sy);
-                    if (!depth_pass(P.depthFunc, d, dep[s], false)) continue;
-                    dep[s] = P.depthWrite ? d * P.depthScale + P.depthBias : d;
-                    slot[s] = sl;
+                    // the scalar path's GREATER quirk belongs to the deterministic mode's single pixels
+                    if (!depth_pass(P.depthFunc, d, dep[0], c == 3u && !P.tagging)) return;
+                    dep[0] = P.depthWrite ? d * P.depthScale + P.depthBias : d;
+                    slot[0] = sl;
+                    cls = class_out(c, P.tagging);
+                } else {
+                    const Edges E = load_edges(R);
+                    bool any = false;
+#pragma unroll
+                    for (int s = 0; s < S; s++) {
+                        const float sx = C.fpx + P.sx[s], sy = C.fpy + P.sy[s];
+                        if (!(c == 3u || inside(E, sx, sy))) continue;
+                        any = true;
+                        covs++;
+                        const float d = depth256(R.f1, R.f2, R.f3, sx, sy);
+                        if (!depth_pass(P.depthFunc, d, dep[s], false)) continue;
+                        dep[s] = P.depthWrite ? d * P.depthScale + P.depthBias : d;
+                        slot[s] = sl;
+                    }
+                    frags += any;
                 }
-                frags += any;
-            }
-        });
+            });
         if (C.inFb && scissor_pass(P.scissor, C.fpx, C.fpy)) {
 #pragma unroll
             for (int s = 0; s < S; s++) {
@@ -1068,11 +994,12 @@ void launch_raster(const RasterParams& p, const Views& views, int samples, TriRe
 }
 
 void launch_raster_ordered(const RasterParams& p, const Views& views, int samples, TriRecs recs,
-                           const BinBufs& bins, int tiles, int grid, float* visDepth, uint32_t* visSlot,
-                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, hipStream_t s) {
+                           const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
+                           uint8_t* visClass, StatPartials st, bool nanTilesOnly, DeviceCounters* ctr,
+                           hipStream_t s) {
 #define IFRIT_ORDERED_LAUNCH(SN)                                                                                  \
-    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, bins.start, bins.cursor, \
-                       bins.list, tiles, visDepth, visSlot, visClass, st, nanTilesOnly ? bins.cnt : nullptr)
+    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(q.grid), dim3(256), 0, s, p, views, recs, bins, q, tiles, p.ntri,  \
+                       visDepth, visSlot, visClass, st, nanTilesOnly ? bins.cnt : nullptr, ctr)
     switch (samples) {
         case 1: IFRIT_ORDERED_LAUNCH(1); break;
         case 4: IFRIT_ORDERED_LAUNCH(4); break;
