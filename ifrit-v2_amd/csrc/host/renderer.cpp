@@ -76,6 +76,7 @@ TileRasterRenderer::~TileRasterRenderer() {
     for (auto& e : ev_)
         if (e) (void)hipEventDestroy(e);
     if (stream_) (void)hipStreamDestroy(stream_);
+    if (hostCtr_) (void)hipHostFree(hostCtr_);
 }
 
 void TileRasterRenderer::setError(const std::string& e) {
@@ -107,6 +108,9 @@ void TileRasterRenderer::Init() {
     for (auto& e : ev_)
         if (!ok(hipEventCreate(&e), "hipEventCreate")) return;
     if (!ensureZeroed(ctr_, sizeof(DeviceCounters))) setError("hipMalloc counters");
+    if (!ok(hipHostMalloc(reinterpret_cast<void**>(&hostCtr_), sizeof(HostCounters), hipHostMallocDefault),
+            "hipHostMalloc counters"))
+        return;
     std::string err;
     if (!noalloc_register_device(&err)) setError(err);
     int dev = 0, cus = 0;
@@ -1304,10 +1308,9 @@ bool TileRasterRenderer::finish(bool clear, int indexCount) {
     (void)clear;
     (void)indexCount;
     // frame statistics are reduced from the per-workgroup partials only when read
-    launch_finalize(statPtrs(), deviceViews(), ctr_.as<DeviceCounters>(), stream_);
+    launch_finalize(statPtrs(), deviceViews(), ctr_.as<DeviceCounters>(), hostCtr_, stream_);
     if (!ok(hipStreamSynchronize(stream_), "frame")) return false;
-    DeviceCounters c{};
-    if (!ok(hipMemcpy(&c, ctr_.ptr, sizeof(c), hipMemcpyDeviceToHost), "counters")) return false;
+    const HostCounters c = *hostCtr_;
     stats_.inputTriangles = (int64_t)curTris_ * (int64_t)viewDesc_.size();
     stats_.assembledTriangles = (int64_t)c.assembled;
     stats_.clippedTriangles = (int64_t)c.clipCount;

@@ -262,6 +262,7 @@ private:
     std::vector<int> viewLayout_;           // (width, height, shade) per view + shading tile
     unsigned totalTiles_ = 0, shadeTiles_ = 0;
     size_t totalPixels_ = 0;
+    HostCounters* hostCtr_ = nullptr;  // pinned: the last finished draw's counters
     DevBuf viewDev_, tileView_, shadeView_, viewCtr_, digest_;
 
     // launch parameters (IfritTuning) and graph replay

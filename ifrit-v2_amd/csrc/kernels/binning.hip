@@ -102,7 +102,6 @@ __global__ void __launch_bounds__(kPlanTiles) k_plan(uint2* __restrict__ cnt, un
             ctr->bigCount = ctr->live.bigCount;
             ctr->clipMax = ctr->live.clipMax;
             ctr->assembled = ctr->live.fans;
-            ctr->clipCount = 0u;
             ctr->live.status = 0u;
             ctr->live.bigCount = 0u;
             ctr->live.clipMax = 0u;

@@ -282,11 +282,8 @@ enum PlanTotal { kTotEntries = 0, kTotLong, kTotShort, kTotPartials, kTotMulti, 
 // The totals and item heads are cleared by the geometry kernel.
 struct DeviceCounters {
     unsigned status;
-    unsigned clipCount;  // clip fan slots of all views (reduced with the statistics)
     unsigned bigCount;
-    unsigned clipMax;    // largest per-view fan or clip count (sizes clipCap on overflow)
-    unsigned long long fragments;
-    unsigned long long coveredSamples;
+    unsigned clipMax;    // largest per-view fan or clip count so far (sizes clipCap on overflow)
     unsigned long long assembled;
     unsigned tot[8];     // PlanTotal: list entries, items of more than kRasterPass entries (front of the
                          // item array), other items, partial blocks, tiles cut into parts, empty tiles
@@ -294,6 +291,14 @@ struct DeviceCounters {
         unsigned status, bigCount, clipMax, fans;  // fans: fan triangles assembled
     } live;
     alignas(128) unsigned itemHeads[kItemStreams][32];  // next item of each stream, one 128-byte line each
+};
+
+// A finished draw's counters as the host reads them (pinned memory written by
+// k_finalize: a copy of DeviceCounters after the stream's end cost a second round trip).
+struct HostCounters {
+    unsigned long long fragments, coveredSamples, assembled;
+    unsigned status, clipCount, bigCount, clipMax;
+    unsigned tot[8];  // PlanTotal
 };
 
 // Raster work: a work item covers at most 1 << partShift list entries of
@@ -333,7 +338,7 @@ void launch_reset(const Views& views, DeviceCounters* ctr, hipStream_t s);
 void launch_geometry(const SetupParams& p, const Views& views, const VertexInput& in, const int* idx, TriRecs recs,
                      float4* bary, const BinBufs& bins, unsigned* slotOf, unsigned* clipList, DeviceCounters* ctr,
                      hipStream_t s);
-void launch_finalize(StatPartials st, const Views& views, DeviceCounters* ctr, hipStream_t s);
+void launch_finalize(StatPartials st, const Views& views, DeviceCounters* ctr, HostCounters* out, hipStream_t s);
 // The tile plan and the scatter into the tile lists.
 void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
                 StatPartials st, DeviceCounters* ctr, hipStream_t s);
