@@ -183,6 +183,8 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
             r.fb_ = fb;
             r.floatOut_ = floatOut;
             r.texPool_ = pool;
+            r.ids_ = nullptr;
+            r.keepSlots_ = true;
         }
     } restore(*this, bufs);
 
@@ -191,7 +193,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     nverts_ = d.numVertices;
     stride_ = d.strideFloats;
     nidx_ = d.numIndices;
-    boundsTris_ = vs_.desc.kind == IFHIP_VS_TRANSFORM ? ntri : 0;
+    boundsTris_ = 0;  // bounding the groups anew (3 to 5 us) costs what testing their triangles does
     fb_ = nullptr;
     floatOut_ = false;
     clipCap_ = std::max(4096u, (unsigned)(ntri / 8));
@@ -219,7 +221,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
 
     // the scratch layout: every buffer of the draw except the caller's inputs and outputs
     const size_t slots = (size_t)ntri + clipCap_, tiles = totalTiles_, px = (size_t)width_ * height_;
-    const size_t groups = (size_t)(boundsTris_ + kGroupTris - 1) / kGroupTris;
+    const size_t groups = vs_.desc.kind == IFHIP_VS_TRANSFORM ? (size_t)(ntri + kGroupTris - 1) / kGroupTris : 0;
     Arena A{base, (size_t)IFHIP_NOALLOC_SCRATCH_BYTES};
     auto put = [&](DevBuf& b, size_t n) {
         b.ptr = A.take(n);
@@ -294,11 +296,10 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
         hipLaunchKernelGGL(k_tables, dim3((unsigned)std::max<size_t>(1, (words + 255) / 256)), dim3(256), 0, stream_, a,
                            viewDev_.as<ViewDesc>(), texDesc_.as<TexDesc>(), reinterpret_cast<uint4*>(base), words);
     }
-    if (boundsTris_ > 0)
-        launch_group_bounds(vtx_.as<float>(), stride_, nverts_, idx_.as<int>(), ntri, groupBounds_.as<float4>(), stream_);
+    ids_ = d.primIds;
+    keepSlots_ = false;
+    reducePending_ = !drawsKeys(true);
     enqueue(true);
-    if (d.primIds && px)
-        launch_slot_to_prim(visSlot_.as<uint32_t>(), recPtrs(), px * samples_, d.primIds, stream_);
     if (!ok(hipGetLastError(), "kernel launch")) return;
     if (!finish(true, d.numIndices))
         setError("iftrDrawNoAlloc: the frame overflowed its scratch buffers (clip, bin or raster queue); the "

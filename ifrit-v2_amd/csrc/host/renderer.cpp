@@ -111,6 +111,7 @@ void TileRasterRenderer::Init() {
     if (!ok(hipHostMalloc(reinterpret_cast<void**>(&hostCtr_), sizeof(HostCounters), hipHostMallocDefault),
             "hipHostMalloc counters"))
         return;
+    *hostCtr_ = HostCounters{};
     std::string err;
     if (!noalloc_register_device(&err)) setError(err);
     int dev = 0, cus = 0;
@@ -978,11 +979,9 @@ constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 size_t TileRasterRenderer::frontBytes() const {
     const size_t nv = std::max<size_t>(1, viewDesc_.size()), W = (size_t)geom_waves(curTris_) * nv;
-    int grid, regions;
-    scatterShape(&grid, &regions);
     return align256(W * 64 * sizeof(uint2)) + align256(W * 64 * sizeof(uint4)) + align256(W * sizeof(WaveInfo)) +
            align256((size_t)clipCap_ * nv * sizeof(uint2)) + align256((size_t)bigCap_ * sizeof(uint4)) +
-           align256((size_t)grid * 8);
+           (size_t)kMadeSums * kMadeStride * 8;
 }
 
 BinBufs TileRasterRenderer::binBufs() const {
@@ -998,6 +997,8 @@ BinBufs TileRasterRenderer::binBufs() const {
     b.fanBox = reinterpret_cast<uint2*>(p);
     p += align256((size_t)clipCap_ * nv * sizeof(uint2));
     b.big = reinterpret_cast<uint4*>(p);
+    p += align256((size_t)bigCap_ * sizeof(uint4));
+    b.made = reinterpret_cast<unsigned long long*>(p);
     b.cnt = binCount_.as<unsigned>();
     b.start = binStart_.as<unsigned>();
     b.cursor = binCursor_.as<unsigned>();
@@ -1012,12 +1013,9 @@ TriRecs TileRasterRenderer::recPtrs() const {
 
 StatPartials TileRasterRenderer::statPtrs() const {
     StatPartials st{};
-    int regions;
-    scatterShape(&st.setupBlocks, &regions);
     st.rasterBlocks = rasterGrid();
     unsigned long long* base = statPart_.as<unsigned long long>();
-    st.setupAssembled = reinterpret_cast<unsigned long long*>(
-        reinterpret_cast<uint8_t*>(binBufs().big) + align256((size_t)bigCap_ * sizeof(uint4)));
+    st.made = binBufs().made;
     st.rasterFrags = base;
     st.rasterCovs = base + st.rasterBlocks;
     return st;
@@ -1079,6 +1077,25 @@ ShadeParams TileRasterRenderer::shadeParams(bool writeFloat) const {
     sh.depthBias = d.depthBias;
     sh.scissor = activeScissor();
     return sh;
+}
+
+// Depth functions that are a minimum of keys on cleared draws; GREATER at one sample is not, as
+// its scalar path tests nothing outside the tagging mode (TRW:2278-2280).  At 720p with 4
+// samples and 82k triangles the keys and their pass over NaN tiles take 36 us; the fold in
+// primitive order, which stays for what depends on the order, took 519 one entry after the other.
+bool TileRasterRenderer::generalKeys(bool clear) const {
+    const int f = depthFunc_;
+    const bool tagging = !deterministic_ && samples_ == 1;
+    return clear && !(fsWritesDepth() && !tagging) &&
+           (f == IF_COMPARE_OP_LESS_OR_EQUAL || f == IF_COMPARE_OP_GREATER_OR_EQUAL || f == IF_COMPARE_OP_ALWAYS ||
+            (f == IF_COMPARE_OP_GREATER && (samples_ > 1 || tagging)));
+}
+
+// The key raster and its merge draw it: the merge's launch reduces the statistics too.
+bool TileRasterRenderer::drawsKeys(bool clear) const {
+    return polygonMode_ == 0 && !blend_.blendEnable &&
+           (generalKeys(clear) ||
+            (depthFunc_ == IF_COMPARE_OP_LESS && !(fsWritesDepth() && (deterministic_ || samples_ != 1))));
 }
 
 void TileRasterRenderer::enqueue(bool clear) {
@@ -1144,14 +1161,10 @@ void TileRasterRenderer::enqueue(bool clear) {
     rp.scissor = activeScissor();
     rp.binCap = binCap_;
     rp.ntri = (unsigned)curTris_;
-    // depth functions that are a minimum of keys on cleared draws; GREATER at one sample is not, as
-    // its scalar path tests nothing outside the tagging mode (TRW:2278-2280)
-    // (at 720p with 4 samples and 82k triangles the keys and their pass over NaN tiles take 36 us, the
-    // fold in primitive order 519; the fold stays for what depends on the order)
     const int f = depthFunc_;
-    rp.general = clear && !rp.depthWrite &&
-                 (f == IF_COMPARE_OP_LESS_OR_EQUAL || f == IF_COMPARE_OP_GREATER_OR_EQUAL ||
-                  f == IF_COMPARE_OP_ALWAYS || (f == IF_COMPARE_OP_GREATER && (samples_ > 1 || rp.tagging)));
+    rp.general = generalKeys(clear) ? 1 : 0;
+    rp.ids = ids_;
+    rp.idsWide = (reinterpret_cast<uintptr_t>(ids_) & 15u) == 0u ? 1 : 0;
     rp.last = f != IF_COMPARE_OP_LESS && f != IF_COMPARE_OP_GREATER ? 1 : 0;
     rp.keyXor = f == IF_COMPARE_OP_GREATER || f == IF_COMPARE_OP_GREATER_OR_EQUAL ? ~0u : 0u;
     rp.keyMask = f == IF_COMPARE_OP_ALWAYS ? 0u : ~0u;
@@ -1161,7 +1174,8 @@ void TileRasterRenderer::enqueue(bool clear) {
         rp.sy[i] = st[2 * i + 1];
     }
     // the 1-sample coverage class is a single-view diagnostic
-    uint8_t* cls = batch_.empty() ? visClass_.as<uint8_t>() : nullptr;
+    uint8_t* cls = batch_.empty() && keepSlots_ ? visClass_.as<uint8_t>() : nullptr;
+    uint32_t* const slots = keepSlots_ || shadeTiles_ > 0 ? visSlot_.as<uint32_t>() : nullptr;
     if (blend_.blendEnable) {
         // blending: fragments shaded and blended in primitive order (the shade stage is part of it)
         launch_blend_ordered(shadeParams(true), blendCoefs_, depthFunc_, clear ? 1 : 0, V, recPtrs(),
@@ -1169,20 +1183,20 @@ void TileRasterRenderer::enqueue(bool clear) {
                              bins, q, tiles, visDepth_.as<float>(), visSlot_.as<uint32_t>(), cls, rgba8_.as<uchar4>(),
                              rgba32f_.as<float4>(), statPtrs(), ctr_.as<DeviceCounters>(), s);
         mark(4);
-    } else if ((depthFunc_ == IF_COMPARE_OP_LESS || rp.general) && !rp.depthWrite) {
+    } else if (drawsKeys(clear)) {
         // order-independent: the lexicographic minimum of (depth, primitive), or of the general keys
         launch_raster(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), bins, q, tiles, visDepth_.as<float>(),
-                      visSlot_.as<uint32_t>(), cls, statPtrs(), ctr_.as<DeviceCounters>(), s);
+                      slots, cls, statPtrs(), ctr_.as<DeviceCounters>(), s);
         mark(4);
         launch_raster_merge(rp, V, samples_, recPtrs(), slotOf_.as<unsigned>(), bins, q, visDepth_.as<float>(),
-                            visSlot_.as<uint32_t>(), cls, tiles, ctr_.as<DeviceCounters>(), s);
+                            slots, cls, tiles, ctr_.as<DeviceCounters>(), statPtrs(), hostCtr_, s);
         if (rp.general)
             launch_raster_ordered(rp, V, samples_, recPtrs(), bins, q, tiles, visDepth_.as<float>(),
-                                  visSlot_.as<uint32_t>(), cls, statPtrs(), true, ctr_.as<DeviceCounters>(), s);
+                                  slots, cls, statPtrs(), true, ctr_.as<DeviceCounters>(), s);
     } else {
         // what is no minimum folds each pixel's fragments in primitive order
         launch_raster_ordered(rp, V, samples_, recPtrs(), bins, q, tiles, visDepth_.as<float>(),
-                              visSlot_.as<uint32_t>(), cls, statPtrs(), false, ctr_.as<DeviceCounters>(), s);
+                              slots, cls, statPtrs(), false, ctr_.as<DeviceCounters>(), s);
         mark(4);
     }
     mark(5);
@@ -1215,7 +1229,7 @@ void TileRasterRenderer::enqueuePolygons(bool clear, const Views& V) {
     pp.clearDepth = clearDepth_;
     pp.keys = polyKeys_.as<unsigned long long>();
     const StatPartials st = statPtrs();
-    const int grid = std::max(std::max(st.setupBlocks, st.rasterBlocks), 1);
+    const int grid = std::max(kMadeSums, st.rasterBlocks);
     mark(2);
     mark(3);
     launch_polygons(pp, clip_.as<float4>(), idx_.as<int>(), recPtrs(), bary_.as<float4>(), visDepth_.as<float>(),
@@ -1281,6 +1295,7 @@ void TileRasterRenderer::dropGraph() {
 // Issues one draw: directly, or as a replay of the captured graph of this
 // configuration (captured on first use).
 void TileRasterRenderer::submit(bool clear) {
+    reducePending_ = !drawsKeys(clear);
     if (!graphMode_) {
         enqueue(clear);
         return;
@@ -1307,8 +1322,10 @@ void TileRasterRenderer::submit(bool clear) {
 bool TileRasterRenderer::finish(bool clear, int indexCount) {
     (void)clear;
     (void)indexCount;
-    // frame statistics are reduced from the per-workgroup partials only when read
-    launch_finalize(statPtrs(), deviceViews(), ctr_.as<DeviceCounters>(), hostCtr_, stream_);
+    // frame statistics are reduced by the key raster's merge, else only when read
+    if (reducePending_)
+        launch_finalize(statPtrs(), deviceViews(), ctr_.as<DeviceCounters>(), hostCtr_, stream_);
+    reducePending_ = false;
     if (!ok(hipStreamSynchronize(stream_), "frame")) return false;
     const HostCounters c = *hostCtr_;
     stats_.inputTriangles = (int64_t)curTris_ * (int64_t)viewDesc_.size();

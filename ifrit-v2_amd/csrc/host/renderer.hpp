@@ -210,6 +210,8 @@ private:
     Views deviceViews() const;
     ShadeParams shadeParams(bool writeFloat) const;
     bool finish(bool clear, int indexCount);
+    bool generalKeys(bool clear) const;
+    bool drawsKeys(bool clear) const;
     void copyOutToHost();
     void runHostVertexShader();
 
@@ -263,6 +265,9 @@ private:
     unsigned totalTiles_ = 0, shadeTiles_ = 0;
     size_t totalPixels_ = 0;
     HostCounters* hostCtr_ = nullptr;  // pinned: the last finished draw's counters
+    bool reducePending_ = false;       // the last draw left its statistics to be reduced
+    uint32_t* ids_ = nullptr;          // where the current draw writes primitive IDs itself
+    bool keepSlots_ = true;            // whether the current draw's record slots and classes are read later
     DevBuf viewDev_, tileView_, shadeView_, viewCtr_, digest_;
 
     // launch parameters (IfritTuning) and graph replay

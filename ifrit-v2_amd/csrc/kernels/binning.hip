@@ -252,7 +252,8 @@ __global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs r
     if (lane == 63) sMade[threadIdx.x >> 6] = made;
     __syncthreads();
     if (threadIdx.x == 0) {
-        st.setupAssembled[blockIdx.x] = sMade[0] + sMade[1] + sMade[2] + sMade[3];
+        atomicAdd(&B.made[(blockIdx.x % kMadeSums) * kMadeStride],
+                  (unsigned long long)(sMade[0] + sMade[1] + sMade[2] + sMade[3]));
         if (blockIdx.x == 0) {
             // on a bin or work-list overflow nothing is rasterised (plan_fits); the host grows the
             // buffers and draws again

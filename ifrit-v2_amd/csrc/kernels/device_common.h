@@ -290,6 +290,65 @@ __device__ __forceinline__ unsigned long long block_sum256(unsigned long long v)
     return r;
 }
 
+// Reduces the per-workgroup statistics of one frame into the counters and writes them
+// to the host (pinned memory, visible once the stream is synchronized).  NT threads.
+// Latency only; a launch of its own took 5 us at the end of every draw, and 15 us with
+// 34 views whose counters one thread read in turn.
+template <int NT>
+__device__ __forceinline__ void finalize_block(const StatPartials& st, const Views& V, const DeviceCounters* ctr,
+                                               HostCounters* out) {
+    __shared__ unsigned long long red[NT / 64][4];
+    __shared__ unsigned most[NT / 64];
+    const int t = threadIdx.x;
+    if (t < 8) out->tot[t] = ctr->tot[t];
+    // what the tile plan (or the point and line kernels) left
+    unsigned long long asmb = t == 0 ? ctr->assembled : 0ull, frag = 0, cov = 0, clip = 0;
+    unsigned mx = t == 0 ? ctr->clipMax : 0u;
+    if (t == 0) {
+        out->status = ctr->status;
+        out->bigCount = ctr->bigCount;
+    }
+    for (int i = t; i < V.count; i += NT) {
+        const unsigned fans = V.ctr[i].fans;
+        clip += fans;
+        mx = max(mx, max(fans, V.ctr[i].clipIn));
+    }
+    if (t < kMadeSums) asmb += st.made[t * kMadeStride];
+    // independent loads: a thread's share is in flight together
+#pragma unroll 4
+    for (int i = t; i < st.rasterBlocks; i += NT) {
+        frag += st.rasterFrags[i];
+        cov += st.rasterCovs[i];
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        asmb += __shfl_down(asmb, off, 64);
+        frag += __shfl_down(frag, off, 64);
+        cov += __shfl_down(cov, off, 64);
+        clip += __shfl_down(clip, off, 64);
+        mx = max(mx, (unsigned)__shfl_down((int)mx, off, 64));
+    }
+    if ((t & 63) == 0) {
+        red[t >> 6][0] = asmb;
+        red[t >> 6][1] = frag;
+        red[t >> 6][2] = cov;
+        red[t >> 6][3] = clip;
+        most[t >> 6] = mx;
+    }
+    __syncthreads();
+    if (t < 4) {
+        unsigned long long r = 0;
+        for (int w = 0; w < NT / 64; w++) r += red[w][t];
+        if (t == 0) out->assembled = r;
+        if (t == 1) out->fragments = r;
+        if (t == 2) out->coveredSamples = r;
+        if (t == 3) out->clipCount = (unsigned)r;
+    } else if (t == 4) {
+        unsigned m = 0;
+        for (int w = 0; w < NT / 64; w++) m = max(m, most[w]);
+        out->clipMax = m;
+    }
+}
+
 // Inclusive prefix sum over the 64 lanes of a wave with DPP moves: row
 // shifts by 1, 2, 4 and 8 (a lane whose source lies outside its row of 16
 // adds 0), then the last lane of rows 0 and 2 added to rows 1 and 3

@@ -164,9 +164,12 @@ struct BinBufs {
     WaveInfo* waves;
     uint2* fanBox;
     uint4* big;  // deferred triangles: slot, tile rectangle (as in entry), view
+    unsigned long long* made;  // triangles assembled: kMadeSums sums of the scatter workgroups
     unsigned* cnt;
     unsigned *start, *cursor, *list;
 };
+// The scatter's workgroups add to as many sums as spread their atomics, a 128-byte line each.
+constexpr int kMadeSums = 64, kMadeStride = 16;
 
 // Triangles per culling group (one workgroup of the geometry kernel).
 constexpr int kGroupTris = kGeomBlock;
@@ -194,6 +197,10 @@ struct RasterParams {
     // general_key)
     int general, last;
     unsigned keyXor, keyMask;
+    // primitive ID per sample of a cleared draw, written with the depth (null: the caller expands slots
+    // itself); idsWide: the array starts on a 16-byte line
+    uint32_t* ids;
+    int idsWide;
     float sx[8], sy[8];  // sample offsets from the pixel corner
 };
 
@@ -261,10 +268,10 @@ enum StatusBits : unsigned {
 // Per-workgroup statistics (no same-address atomics in the hot kernels);
 // k_finalize reduces them into DeviceCounters.
 struct StatPartials {
-    unsigned long long* setupAssembled;  // one per scatter workgroup
+    unsigned long long* made;            // BinBufs::made
     unsigned long long* rasterFrags;     // one per raster workgroup
     unsigned long long* rasterCovs;      // one per raster workgroup
-    int setupBlocks, rasterBlocks;
+    int rasterBlocks;
 };
 
 // Raster work items are drained through this many counters, one per XCD:
@@ -294,7 +301,7 @@ struct DeviceCounters {
 };
 
 // A finished draw's counters as the host reads them (pinned memory written by
-// k_finalize: a copy of DeviceCounters after the stream's end cost a second round trip).
+// finalize_block: a copy of DeviceCounters after the stream's end cost a second round trip).
 struct HostCounters {
     unsigned long long fragments, coveredSamples, assembled;
     unsigned status, clipCount, bigCount, clipMax;
@@ -347,7 +354,8 @@ void launch_raster(const RasterParams& p, const Views& views, int samples, TriRe
                    uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s);
 void launch_raster_merge(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                          const BinBufs& bins, const RasterQueue& q, float* visDepth, uint32_t* visSlot,
-                         uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s);
+                         uint8_t* visClass, int tiles, DeviceCounters* ctr, StatPartials st, HostCounters* out,
+                         hipStream_t s);
 // Depth functions that are no minimum: each tile's list in primitive order, folded
 // per pixel (replaces launch_raster and launch_raster_merge); with nanTilesOnly the tiles in which
 // they met a NaN depth (after launch_raster_merge of a general draw).

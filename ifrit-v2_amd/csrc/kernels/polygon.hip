@@ -72,7 +72,7 @@ __device__ __forceinline__ void block_stats(unsigned long long frags, unsigned l
             st.rasterFrags[blockIdx.x] = f;
             st.rasterCovs[blockIdx.x] = f;
         }
-        if ((int)blockIdx.x < st.setupBlocks) st.setupAssembled[blockIdx.x] = 0;
+        if ((int)blockIdx.x < kMadeSums) st.made[blockIdx.x * kMadeStride] = 0;
         if (a) atomicAdd(&ctr->assembled, a);
     }
 }

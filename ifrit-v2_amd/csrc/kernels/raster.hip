@@ -241,6 +241,33 @@ __device__ __forceinline__ void write_pixel(const RasterParams& P, const TriRecs
     if (S == 1 && visClass && won) visClass[C.pix] = class_out(cls, P.tagging);
 }
 
+// A view's outputs: depth per sample and, where wanted, record slots, primitive IDs and
+// (1 sample per pixel) coverage classes.
+// The key holds the primitive, so IDs cost their stores; expanding them from the slots
+// in a pass of its own took 3 us at 256x256 and 6 us at 1080p, and a draw that is not
+// shaded needs no slots.
+struct VisOut {
+    float* depth;
+    uint32_t *slot, *ids;
+    uint8_t* cls;
+};
+template <int S>
+__device__ __forceinline__ VisOut vis_out(const RasterParams& P, const ViewGeom& G, float* depth, uint32_t* slot,
+                                          uint8_t* cls) {
+    const size_t at = G.pixBase * S;
+    return VisOut{depth + at, slot ? slot + at : nullptr, P.ids ? P.ids + at : nullptr, cls ? cls + G.pixBase : nullptr};
+}
+__device__ __forceinline__ void store_ids(uint32_t* to, uint4 v, bool wide) {
+    if (wide) {
+        *reinterpret_cast<uint4*>(to) = v;
+    } else {
+        to[0] = v.x;
+        to[1] = v.y;
+        to[2] = v.z;
+        to[3] = v.w;
+    }
+}
+
 // One tile's outputs staged in LDS in global order (pixel-major, sample-
 // minor) so that they leave with 16-byte stores of consecutive addresses;
 // per-lane stores of one pixel's S samples would touch a partial line per
@@ -304,15 +331,14 @@ __device__ __forceinline__ unsigned pixel_outputs(const RasterParams& P, const T
 template <int S>
 __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
                                             const PixelCtx& C, int t, const unsigned long long* keys, unsigned won,
-                                            TileOut<S>& O, uint8_t* visClass, const float* visDepth,
-                                            const uint32_t* visSlot) {
+                                            TileOut<S>& O, const VisOut& vis) {
     if (!C.inFb) return;
     if (!scissor_pass(P.scissor, C.fpx, C.fpy)) {
         // outside the scissor: the tile's line stores write the pixel's current contents back
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            O.d[t * S + s] = visDepth[C.pix * S + s];
-            O.slot[t * S + s] = visSlot[C.pix * S + s];
+            O.d[t * S + s] = vis.depth[C.pix * S + s];
+            if (vis.slot) O.slot[t * S + s] = vis.slot[C.pix * S + s];
         }
         return;
     }
@@ -324,7 +350,8 @@ __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs
         O.d[t * S + s] = d[s];
         O.slot[t * S + s] = slot[s];
     }
-    if (S == 1 && visClass) visClass[C.pix] = class_out(cls, P.tagging);
+    if (S == 1 && vis.cls) vis.cls[C.pix] = class_out(cls, P.tagging);
+    if (S == 1 && vis.ids) vis.ids[C.pix] = won ? key_tie<S>(keys[0]) >> 2 : 0xffffffffu;
 }
 
 // Outputs of one pixel of a cleared draw straight to memory with 16-byte
@@ -332,19 +359,24 @@ __device__ __forceinline__ void stage_pixel(const RasterParams& P, const TriRecs
 // a row of pixels whole lines).
 template <int S>
 __device__ __forceinline__ void emit_pixel(const RasterParams& P, const TriRecs& recs, const SlotMap& slotOf,
-                                           const PixelCtx& C, const unsigned long long* keys, unsigned won, float* visDepth,
-                                           uint32_t* visSlot) {
+                                           const PixelCtx& C, const unsigned long long* keys, unsigned won,
+                                           const VisOut& vis) {
     static_assert(S % 4 == 0, "whole 16-byte words per pixel");
     if (!C.inFb || !scissor_pass(P.scissor, C.fpx, C.fpy)) return;
     float d[S];
     unsigned slot[S];
     pixel_outputs<S>(P, recs, slotOf, C, keys, won, d, slot);
-    float4* const dd = reinterpret_cast<float4*>(visDepth + C.pix * S);
-    uint4* const ds = reinterpret_cast<uint4*>(visSlot + C.pix * S);
+    float4* const dd = reinterpret_cast<float4*>(vis.depth + C.pix * S);
+    uint4* const ds = reinterpret_cast<uint4*>(vis.slot + C.pix * S);
 #pragma unroll
     for (int v = 0; v < S / 4; v++) {
         dd[v] = make_float4(d[4 * v], d[4 * v + 1], d[4 * v + 2], d[4 * v + 3]);
-        ds[v] = make_uint4(slot[4 * v], slot[4 * v + 1], slot[4 * v + 2], slot[4 * v + 3]);
+        if (vis.slot) ds[v] = make_uint4(slot[4 * v], slot[4 * v + 1], slot[4 * v + 2], slot[4 * v + 3]);
+        if (vis.ids) {
+            auto id = [&](int s) { return (won >> s) & 1u ? key_tie<S>(keys[s]) >> 2 : 0xffffffffu; };
+            store_ids(vis.ids + C.pix * S + 4 * v, make_uint4(id(4 * v), id(4 * v + 1), id(4 * v + 2), id(4 * v + 3)),
+                      P.idsWide != 0);
+        }
     }
 }
 
@@ -354,7 +386,7 @@ __device__ __forceinline__ void emit_pixel(const RasterParams& P, const TriRecs&
 // pixel base is a multiple of 4.
 template <int S, int NT = 256>
 __device__ __forceinline__ void store_tile(int t, const ViewGeom& G, int tx, int ty, const TileOut<S>* O,
-                                           float* visDepth, uint32_t* visSlot) {
+                                           const VisOut& vis) {
     constexpr int perRow = 16 * S / 4;  // float4 per tile row
     const int cols = min(16, G.width - tx * 16), rows = min(16, G.height - ty * 16);
     const bool vec = cols == 16 && (S > 1 || ((G.width & 3) == 0 && (G.pixBase & 3) == 0));
@@ -366,16 +398,16 @@ __device__ __forceinline__ void store_tile(int t, const ViewGeom& G, int tx, int
         const float4 d = *reinterpret_cast<const float4*>(&O->d[l]);
         const uint4 sl = *reinterpret_cast<const uint4*>(&O->slot[l]);
         if (vec) {
-            *reinterpret_cast<float4*>(&visDepth[g]) = d;
-            *reinterpret_cast<uint4*>(&visSlot[g]) = sl;
+            *reinterpret_cast<float4*>(&vis.depth[g]) = d;
+            if (vis.slot) *reinterpret_cast<uint4*>(&vis.slot[g]) = sl;
         } else {
             const float dv[4] = {d.x, d.y, d.z, d.w};
             const unsigned sv[4] = {sl.x, sl.y, sl.z, sl.w};
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if ((q * 4 + e) / S >= cols) continue;
-                visDepth[g + e] = dv[e];
-                visSlot[g + e] = sv[e];
+                vis.depth[g + e] = dv[e];
+                if (vis.slot) vis.slot[g + e] = sv[e];
             }
         }
     }
@@ -386,39 +418,38 @@ __device__ __forceinline__ void store_tile(int t, const ViewGeom& G, int tx, int
 // stores where the tile's rows are whole.
 template <int S, int NT>
 __device__ __forceinline__ void clear_tile(int t, const ViewGeom& G, float clearDepth, const Scissor& sc,
-                                           float* visDepthAll, uint32_t* visSlotAll, uint8_t* visClassAll) {
+                                           bool idsWide, const VisOut& vis) {
     const int tx = G.tile % G.tilesX, ty = G.tile / G.tilesX;
     const int cols = min(16, G.width - tx * 16), rows = min(16, G.height - ty * 16);
     const bool whole = scissor_all(sc, tx * 16, ty * 16, tx * 16 + cols - 1, ty * 16 + rows - 1);
     const bool vec = whole && cols == 16 && (S > 1 || ((G.width & 3) == 0 && (G.pixBase & 3) == 0));
-    float* const visDepth = visDepthAll + G.pixBase * S;
-    uint32_t* const visSlot = visSlotAll + G.pixBase * S;
     constexpr int perRow = 16 * S / 4;  // 16-byte words per tile row
     for (int i = t; i < 64 * S; i += NT) {
         const int row = i / perRow, q = i - row * perRow;
         if (row >= rows) continue;
         const size_t g = ((size_t)(ty * 16 + row) * G.width + tx * 16) * S + q * 4;
         if (vec) {
-            *reinterpret_cast<float4*>(&visDepth[g]) = make_float4(clearDepth, clearDepth, clearDepth, clearDepth);
-            *reinterpret_cast<uint4*>(&visSlot[g]) = make_uint4(~0u, ~0u, ~0u, ~0u);
+            *reinterpret_cast<float4*>(&vis.depth[g]) = make_float4(clearDepth, clearDepth, clearDepth, clearDepth);
+            if (vis.slot) *reinterpret_cast<uint4*>(&vis.slot[g]) = make_uint4(~0u, ~0u, ~0u, ~0u);
+            if (vis.ids) store_ids(&vis.ids[g], make_uint4(~0u, ~0u, ~0u, ~0u), idsWide);
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int col = (q * 4 + e) / S;
                 if (col >= cols) continue;
                 if (!whole && !scissor_pass(sc, (float)(tx * 16 + col), (float)(ty * 16 + row))) continue;
-                visDepth[g + e] = clearDepth;
-                visSlot[g + e] = 0xffffffffu;
+                vis.depth[g + e] = clearDepth;
+                if (vis.slot) vis.slot[g + e] = 0xffffffffu;
+                if (vis.ids) vis.ids[g + e] = 0xffffffffu;
             }
         }
     }
-    if (S == 1 && visClassAll) {
-        uint8_t* const visClass = visClassAll + G.pixBase;
+    if (S == 1 && vis.cls) {
         for (int i = t; i < 256; i += NT) {
             const int row = i >> 4, col = i & 15;
             if (row < rows && col < cols &&
                 (whole || scissor_pass(sc, (float)(tx * 16 + col), (float)(ty * 16 + row))))
-                visClass[(size_t)(ty * 16 + row) * G.width + tx * 16 + col] = 0;
+                vis.cls[(size_t)(ty * 16 + row) * G.width + tx * 16 + col] = 0;
         }
     }
 }
@@ -499,9 +530,11 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             const unsigned e = item - numItems;
             if (e >= numEmptyItems) break;
             if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for (unsigned k = e * KE; k < min(e * KE + KE, numEmpty); k++)
-                clear_tile<S, NT>(t, view_of_tile(V, (int)*(emptyEnd - k)), P.clearDepth, P.scissor, visDepthAll,
-                                  visSlotAll, visClassAll);
+            for (unsigned k = e * KE; k < min(e * KE + KE, numEmpty); k++) {
+                const ViewGeom E = view_of_tile(V, (int)*(emptyEnd - k));
+                clear_tile<S, NT>(t, E, P.clearDepth, P.scissor, P.idsWide != 0,
+                                  vis_out<S>(P, E, visDepthAll, visSlotAll, visClassAll));
+            }
             __syncthreads();  // every lane has read sItem
             continue;
         }
@@ -512,9 +545,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         const int cnt = __builtin_amdgcn_readfirstlane((int)it.z);
         const unsigned pslot = __builtin_amdgcn_readfirstlane(it.w);
         const ViewGeom G_ = view_of_tile(V, tile);
-        float* const visDepth = visDepthAll + G_.pixBase * S;
-        uint32_t* const visSlot = visSlotAll + G_.pixBase * S;
-        uint8_t* const visClass = visClassAll ? visClassAll + G_.pixBase : nullptr;
+        const VisOut vis = vis_out<S>(P, G_, visDepthAll, visSlotAll, visClassAll);
         const SlotMap slotOf{slotOfAll + G_.primBase, waves + (size_t)G_.view * V.waves, G_.slotBase,
                              V.ctr[G_.view].clipIn != 0u};
         const int ttx = G_.tile % G_.tilesX, tty = G_.tile / G_.tilesX;
@@ -528,7 +559,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             for (int s = 0; s < S; s++)
                 sVis[vis_at(s, p)] =
                     G ? general_clear_key(P)
-                      : frag_key(P.clear || !C.inFb ? P.clearDepth : visDepth[C.pix * S + s], 0u);
+                      : frag_key(P.clear || !C.inFb ? P.clearDepth : vis.depth[C.pix * S + s], 0u);
         }
 
         const int cols = min(16, G_.width - tx0), rows = min(16, G_.height - ty0);
@@ -727,7 +758,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                     for (int k = 0; k < PPT; k++) {
                         const int p = t + k * NT;
                         const unsigned won = final_keys<S, G>(P, keys[k]);
-                        emit_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], won, visDepth, visSlot);
+                        emit_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], won, vis);
                     }
                 } else {
                     // every key is in registers: stage the outputs over sVis
@@ -737,18 +768,17 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                     for (int k = 0; k < PPT; k++) {
                         const int p = t + k * NT;
                         const unsigned won = final_keys<S, G>(P, keys[k]);
-                        stage_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), p, keys[k], won, *O, visClass,
-                                       visDepth, visSlot);
+                        stage_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), p, keys[k], won, *O, vis);
                     }
                     __syncthreads();
-                    store_tile<S, NT>(t, G_, ttx, tty, O, visDepth, visSlot);
+                    store_tile<S, NT>(t, G_, ttx, tty, O, vis);
                 }
             } else {
 #pragma unroll
                 for (int k = 0; k < PPT; k++) {
                     const int p = t + k * NT;
-                    write_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], visDepth, visSlot,
-                                   visClass);
+                    write_pixel<S>(P, recs, slotOf, pixel_ctx(G_, p & 15, p >> 4), keys[k], vis.depth, vis.slot,
+                                   vis.cls);
                 }
             }
         }
@@ -763,7 +793,8 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
 }
 
 // Minimum over the parts of every tile whose list was cut, then the outputs
-// (the empty tiles' clear values come from k_raster).
+// (the empty tiles' clear values come from k_raster).  The last workgroup reduces the
+// draw's statistics meanwhile.
 template <int S>
 __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, TriRecs recs,
                                                       const unsigned* __restrict__ slotOfAll,
@@ -771,16 +802,19 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
                                                       const unsigned* __restrict__ binStart,
                                                       const unsigned* __restrict__ binEnd, RasterQueue q,
                                                       float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
-                                                      uint8_t* __restrict__ visClassAll, const DeviceCounters* ctr) {
+                                                      uint8_t* __restrict__ visClassAll, DeviceCounters* ctr, StatPartials st,
+                                                      HostCounters* out) {
+    if (blockIdx.x == gridDim.x - 1u) {
+        finalize_block<256>(st, V, ctr, out);
+        return;
+    }
     const unsigned numMulti = plan_fits(ctr, q) ? ctr->tot[kTotMulti] : 0u;
     const int t = threadIdx.x;
     // tiles whose list was cut into several items: the minimum over their partial blocks
-    for (unsigned m = blockIdx.x; m < numMulti; m += gridDim.x) {
+    for (unsigned m = blockIdx.x; m < numMulti; m += gridDim.x - 1u) {
         const int tile = (int)q.multiList[m];
         const ViewGeom G = view_of_tile(V, tile);
-        float* const visDepth = visDepthAll + G.pixBase * S;
-        uint32_t* const visSlot = visSlotAll + G.pixBase * S;
-        uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
+        const VisOut vis = vis_out<S>(P, G, visDepthAll, visSlotAll, visClassAll);
         const SlotMap slotOf{slotOfAll + G.primBase, waves + (size_t)G.view * V.waves, G.slotBase,
                              V.ctr[G.view].clipIn != 0u};
         const PixelCtx C = pixel_ctx(G, t & 15, t >> 4);
@@ -798,16 +832,16 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
         if (P.clear) {
             const unsigned won = P.general ? final_keys<S, true>(P, keys) : final_keys<S, false>(P, keys);
             if constexpr (S > 1) {
-                emit_pixel<S>(P, recs, slotOf, C, keys, won, visDepth, visSlot);
+                emit_pixel<S>(P, recs, slotOf, C, keys, won, vis);
             } else {
                 __shared__ TileOut<S> O;  // output staging at 1 sample per pixel
                 __syncthreads();          // the previous tile's staging has been stored
-                stage_pixel<S>(P, recs, slotOf, C, t, keys, won, O, visClass, visDepth, visSlot);
+                stage_pixel<S>(P, recs, slotOf, C, t, keys, won, O, vis);
                 __syncthreads();
-                store_tile<S>(t, G, C.tx, C.ty, &O, visDepth, visSlot);
+                store_tile<S>(t, G, C.tx, C.ty, &O, vis);
             }
         } else {
-            write_pixel<S>(P, recs, slotOf, C, keys, visDepth, visSlot, visClass);
+            write_pixel<S>(P, recs, slotOf, C, keys, vis.depth, vis.slot, vis.cls);
         }
     }
 }
@@ -853,18 +887,16 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
         }
         const ViewGeom G = view_of_tile(V, tile);
         const PixelCtx C = pixel_ctx(G, quarter_x(t), quarter_y(t));
-        float* const visDepth = visDepthAll + G.pixBase * S;
-        uint32_t* const visSlot = visSlotAll + G.pixBase * S;
-        uint8_t* const visClass = visClassAll ? visClassAll + G.pixBase : nullptr;
+        const VisOut vis = vis_out<S>(P, G, visDepthAll, visSlotAll, visClassAll);
         float dep[S];
         unsigned slot[S];
         unsigned cls = 0;
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            dep[s] = P.clear || !C.inFb ? P.clearDepth : visDepth[C.pix * S + s];
-            slot[s] = P.clear || !C.inFb ? 0xffffffffu : visSlot[C.pix * S + s];
+            dep[s] = P.clear || !C.inFb ? P.clearDepth : vis.depth[C.pix * S + s];
+            slot[s] = P.clear || !C.inFb ? 0xffffffffu : vis.slot[C.pix * S + s];
         }
-        if (!P.clear && S == 1 && visClass && C.inFb) cls = visClass[C.pix];
+        if (!P.clear && S == 1 && vis.cls && C.inFb) cls = vis.cls[C.pix];
         for_each_ordered<S>(
             recs, B.list, start, cnt, G.slotBase, ntri, C, P.tagging, L,
             [&](const TriRec& R, unsigned sl, unsigned c) {
@@ -898,10 +930,12 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
         if (C.inFb && scissor_pass(P.scissor, C.fpx, C.fpy)) {
 #pragma unroll
             for (int s = 0; s < S; s++) {
-                visDepth[C.pix * S + s] = dep[s];
-                visSlot[C.pix * S + s] = slot[s];
+                vis.depth[C.pix * S + s] = dep[s];
+                if (vis.slot) vis.slot[C.pix * S + s] = slot[s];
+                if (vis.ids)
+                    vis.ids[C.pix * S + s] = slot[s] == 0xffffffffu ? slot[s] : __float_as_uint(recs.q2[slot[s]].y) >> 2;
             }
-            if (S == 1 && visClass) visClass[C.pix] = (uint8_t)cls;
+            if (S == 1 && vis.cls) vis.cls[C.pix] = (uint8_t)cls;
         }
         if (nanTile) {
             __syncthreads();  // every thread has read the mark
@@ -1010,12 +1044,13 @@ void launch_raster_ordered(const RasterParams& p, const Views& views, int sample
 
 void launch_raster_merge(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                          const BinBufs& bins, const RasterQueue& q, float* visDepth, uint32_t* visSlot,
-                         uint8_t* visClass, int tiles, DeviceCounters* ctr, hipStream_t s) {
-    // a workgroup per tile at most
-    const int grid = std::max(1, std::min(2 * q.mergeGrid, tiles));
+                         uint8_t* visClass, int tiles, DeviceCounters* ctr, StatPartials st, HostCounters* out,
+                         hipStream_t s) {
+    // a workgroup per tile at most, and one for the statistics
+    const int grid = std::max(1, std::min(2 * q.mergeGrid, tiles)) + 1;
 #define IFRIT_MERGE_LAUNCH(SN)                                                                                     \
     hipLaunchKernelGGL(k_raster_merge<SN>, dim3(grid), dim3(256), 0, s, p, views, recs, slotOf, bins.waves,       \
-                       bins.start, bins.cursor, q, visDepth, visSlot, visClass, ctr)
+                       bins.start, bins.cursor, q, visDepth, visSlot, visClass, ctr, st, out)
     switch (samples) {
         case 1: IFRIT_MERGE_LAUNCH(1); break;
         case 4: IFRIT_MERGE_LAUNCH(4); break;
