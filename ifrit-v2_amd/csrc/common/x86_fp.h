@@ -61,27 +61,35 @@ IFX_HD float u2f(uint32_t u) { return __builtin_bit_cast(float, u); }
 // give signed zero, NaNs come back quieted.
 // Without branches: the table's entry for the mantissa with 127 - e added to its
 // exponent, replaced where that leaves the normal range.
-IFX_HD float rcp_ps(float x, int model) {
+// In three steps, so that a caller can have several lookups in flight.
+struct RcpTable {
+    const uint32_t* entries;
+    uint32_t shift, mask;
+};
+IFX_HD RcpTable rcp_table(int model) {
+    const bool amd = model == kRcpAmd;
+#if defined(__HIP_DEVICE_COMPILE__)
+    return RcpTable{amd ? kRcpTableAmd : kRcpTable, amd ? 11u : 12u, amd ? 0xfffu : 0x7ffu};
+#else
+    return RcpTable{amd ? kRcpTableAmdHost : kRcpTableHost, amd ? 11u : 12u, amd ? 0xfffu : 0x7ffu};
+#endif
+}
+IFX_HD uint32_t rcp_entry(float x, const RcpTable& tab) { return tab.entries[(f2u(x) >> tab.shift) & tab.mask]; }
+IFX_HD float rcp_ps(float x, uint32_t entry) {
     const uint32_t b = f2u(x);
     const uint32_t sign = b & 0x80000000u;
     const int32_t e = (int32_t)((b >> 23) & 0xffu);
-    const bool amd = model == kRcpAmd;
-    const uint32_t idx = (b >> (amd ? 11 : 12)) & (amd ? 0xfffu : 0x7ffu);
-#if defined(__HIP_DEVICE_COMPILE__)
-    const uint32_t* tab = amd ? kRcpTableAmd : kRcpTable;
-#else
-    const uint32_t* tab = amd ? kRcpTableAmdHost : kRcpTableHost;
-#endif
-    const int32_t t = (int32_t)tab[idx] + ((127 - e) * 0x800000);  // exponents 126 or 127 in the table
+    const int32_t t = (int32_t)entry + ((127 - e) * 0x800000);  // exponents 126 or 127 in the table
     uint32_t r = t < 0x800000 ? 0u : (uint32_t)t;                  // sub-normal results flush to zero
     r = e == 0 ? 0x7f800000u : r;
     r = e == 255 ? ((b & 0x7fffffu) ? (b & 0x7fffffffu) | 0x400000u : 0u) : r;
     return u2f(sign | r);
 }
+IFX_HD float rcp_ps(float x, int model) { return rcp_ps(x, rcp_entry(x, rcp_table(model))); }
 
 // ApproxReciprocalNR256: r = rcp(x); (r + r) - x * (r * r).
-IFX_HD float rcp_nr_ps(float x, int model) {
-    float r = rcp_ps(x, model);
+IFX_HD float rcp_nr_ps(float x, uint32_t entry) {
+    float r = rcp_ps(x, entry);
     float rr = r * r;
     float muls = x * rr;
     float twice = r + r;

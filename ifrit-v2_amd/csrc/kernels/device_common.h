@@ -162,6 +162,27 @@ __device__ __forceinline__ unsigned long long frag_key(float d, unsigned tie) {
     return ((unsigned long long)order_key(d) << 32) | tie;
 }
 
+// A view at a uniform index, in the constant address space: no kernel that reads the
+// table writes it, which the compiler cannot see of a plain pointer beside atomics and
+// stores, so that it loads the matrix into every lane.
+typedef const __attribute__((address_space(4))) ViewDesc UniformView;
+__device__ __forceinline__ const UniformView& uniform_view(const ViewDesc* d) { return *(UniformView*)d; }
+// Words at a uniform address that no kernel reading them writes, and entry i of a map
+// of views (two bytes each; a word of it lies in the map's allocation, whose size is a
+// multiple of four bytes).
+__device__ __forceinline__ unsigned uniform_word(const unsigned* p) {
+    return *(const __attribute__((address_space(4))) unsigned*)p;
+}
+__device__ __forceinline__ uint4 uniform_words(const uint4* p) {
+    typedef unsigned Words __attribute__((ext_vector_type(4)));
+    const Words w = *(const __attribute__((address_space(4))) Words*)p;
+    return make_uint4(w.x, w.y, w.z, w.w);
+}
+__device__ __forceinline__ unsigned uniform_view_of(const unsigned short* map, unsigned i) {
+    i = (unsigned)__builtin_amdgcn_readfirstlane((int)i);
+    return (uniform_word(reinterpret_cast<const unsigned*>(map) + (i >> 1)) >> (16u * (i & 1u))) & 0xffffu;
+}
+
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
 
 // Wave-aggregated counter increment: every active lane adds one to

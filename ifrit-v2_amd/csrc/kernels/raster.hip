@@ -477,6 +477,8 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 // keys' LDS allows four).  Windows from pixel boxes, one lane per entry, instead of block
 // tests of every entry by two: 105 -> 84 us there, and 78 us with fewer registers; 4.2M
 // half-pixel triangles at 4 samples 327 -> 213 us, 34 views at 1 sample 525 -> 355 us.
+// Items and views through the scalar cache and a pass's entries loaded during the one
+// before: 351 -> 330 us at the 34 views, 215 -> 207 and 81 -> 79 us at the others.
 template <int S, int NT, bool G = false>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S == 8 ? 4 : 5, 8)))
 k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slotOfAll,
@@ -525,13 +527,13 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
         asm volatile("" : "+v"(t));
         if (t == 0) sItem = claimed;
         __syncthreads();
-        const unsigned item = sItem * kItemStreams + stream;
+        const unsigned item = (unsigned)__builtin_amdgcn_readfirstlane((int)sItem) * kItemStreams + stream;
         if (item >= numItems) {
             const unsigned e = item - numItems;
             if (e >= numEmptyItems) break;
             if (t == 0) claimed = __hip_atomic_fetch_add(head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             for (unsigned k = e * KE; k < min(e * KE + KE, numEmpty); k++) {
-                const ViewGeom E = view_of_tile(V, (int)*(emptyEnd - k));
+                const ViewGeom E = view_of_tile(V, (int)uniform_word(emptyEnd - k));
                 clear_tile<S, NT>(t, E, P.clearDepth, P.scissor, P.idsWide != 0,
                                   vis_out<S>(P, E, visDepthAll, visSlotAll, visClassAll));
             }
@@ -539,15 +541,15 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             continue;
         }
         // long items from the front of the array, then short ones from its back
-        const uint4 it = q.items[item < numLong ? item : q.itemCap - 1u - (item - numLong)];
-        const int tile = __builtin_amdgcn_readfirstlane((int)it.x);
-        const unsigned first = __builtin_amdgcn_readfirstlane(it.y);
-        const int cnt = __builtin_amdgcn_readfirstlane((int)it.z);
-        const unsigned pslot = __builtin_amdgcn_readfirstlane(it.w);
+        const uint4 it = uniform_words(q.items + (item < numLong ? item : q.itemCap - 1u - (item - numLong)));
+        const int tile = (int)it.x, cnt = (int)it.z;
+        const unsigned first = it.y, pslot = it.w;
+        // a pass's entries are loaded during the one before, the first pass's before the view is known
+        unsigned ent = t < cnt && t < PASS ? binList[first + t] : 0u;
         const ViewGeom G_ = view_of_tile(V, tile);
         const VisOut vis = vis_out<S>(P, G_, visDepthAll, visSlotAll, visClassAll);
         const SlotMap slotOf{slotOfAll + G_.primBase, waves + (size_t)G_.view * V.waves, G_.slotBase,
-                             V.ctr[G_.view].clipIn != 0u};
+                             uniform_word(&V.ctr[G_.view].clipIn) != 0u};
         const int ttx = G_.tile % G_.tilesX, tty = G_.tile / G_.tilesX;
         const int tx0 = ttx * 16, ty0 = tty * 16;
 
@@ -622,7 +624,6 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
             unsigned n = 0, blocks = 0;
             int bx0 = 0, by0 = 0, wcols = 0;
             if (t < pc) {
-                const unsigned ent = binList[first + pb + t];
                 const TriRec R = load_rec(recs, ent & 0x7fffffffu);
                 sRec[t] = R;
                 const Edges E = load_edges(R);
@@ -651,6 +652,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                 sRec[t].q2.z = __uint_as_float(full ? 0x80000000u
                                                     : (unsigned)(x0 | (y0 << 4) | (max(x1, 0) << 8) | (max(y1, 0) << 12)));
             }
+            if (t < PASS && pb + PASS + t < cnt) ent = binList[first + pb + PASS + t];
             unsigned TP;
             int pp = (int)scan_nt<NT>(t, n, sWave, TP);
             if (blocks) {
@@ -816,7 +818,7 @@ __global__ void __launch_bounds__(256) k_raster_merge(RasterParams P, Views V, T
         const ViewGeom G = view_of_tile(V, tile);
         const VisOut vis = vis_out<S>(P, G, visDepthAll, visSlotAll, visClassAll);
         const SlotMap slotOf{slotOfAll + G.primBase, waves + (size_t)G.view * V.waves, G.slotBase,
-                             V.ctr[G.view].clipIn != 0u};
+                             uniform_word(&V.ctr[G.view].clipIn) != 0u};
         const PixelCtx C = pixel_ctx(G, t & 15, t >> 4);
         const unsigned total = binEnd[tile] - binStart[tile];
         const unsigned nparts = (total + (1u << q.partShift) - 1u) >> q.partShift;

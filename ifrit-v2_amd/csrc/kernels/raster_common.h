@@ -63,7 +63,8 @@ struct ViewGeom {
 };
 
 __device__ __forceinline__ ViewGeom view_of_tile(const Views& V, int gtile) {
-    const ViewDesc& D = V.desc[V.tileView[gtile]];
+    const unsigned view = uniform_view_of(V.tileView, (unsigned)gtile);
+    const UniformView& D = uniform_view(V.desc + view);
     ViewGeom G;
     G.width = D.width;
     G.height = D.height;
@@ -72,7 +73,7 @@ __device__ __forceinline__ ViewGeom view_of_tile(const Views& V, int gtile) {
     G.pixBase = (size_t)D.pixBase;
     G.primBase = D.primBase;
     G.slotBase = D.slotBase;
-    G.view = V.tileView[gtile];
+    G.view = (int)view;
     return G;
 }
 

@@ -940,8 +940,8 @@ __device__ __forceinline__ void shade_tiles(const ShadeParams& P, const Views& V
     const int g = (int)(blockIdx.x >> 3);
     const int tile = (g / kShadeRun) * (8 * kShadeRun) + (int)(blockIdx.x & 7u) * kShadeRun + g % kShadeRun;
     if (tile >= tiles) return;
-    const unsigned view = V.shadeView[tile];
-    const ViewDesc& D = V.desc[view];
+    const unsigned view = dev::uniform_view_of(V.shadeView, (unsigned)tile);
+    const dev::UniformView& D = dev::uniform_view(V.desc + view);
     const float4* const bary = baryAll + view_bary(V, view, P.ntri);
     const int width = D.width, height = D.height;
     const int local = tile - (int)D.shadeBase, perRow = (width + T - 1) / T;
@@ -1057,7 +1057,7 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
     int tile;
     unsigned start, cnt;
     while (order.next(q, bins, tiles, &sItem, tile, start, cnt)) {
-        const ViewDesc& D = V.desc[V.tileView[tile]];
+        const dev::UniformView& D = dev::uniform_view(V.desc + dev::uniform_view_of(V.tileView, (unsigned)tile));
         const rc::ViewGeom G = rc::view_of_tile(V, tile);
         const float4* const bary = baryAll + view_bary(V, (unsigned)G.view, P.ntri);
         const rc::PixelCtx C = rc::pixel_ctx(G, rc::quarter_x(t), rc::quarter_y(t));
