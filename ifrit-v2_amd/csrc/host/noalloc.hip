@@ -136,7 +136,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
                             &bary_, &binFront_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_,
                             &ctr_, &groupBounds_, &clipList_, &statPart_, &items_, &tilePartial_,
                             &multiList_, &partials_, &visDepth_, &visSlot_, &visClass_, &rgba8_, &rgba32f_,
-                            &texDesc_, &viewDev_, &tileView_, &shadeView_, &viewCtr_, &swapped_};
+                            &texDesc_, &viewDev_, &tileView_, &order_, &viewCtr_, &swapped_};
     constexpr size_t kBufs = sizeof(bufs) / sizeof(bufs[0]);
     struct Restore {
         TileRasterRenderer& r;
@@ -202,7 +202,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     bigCap_ = std::max(1024u, (unsigned)(ntri / 16));
     const int tilesX = (width_ + kTile - 1) / kTile, tilesY = (height_ + kTile - 1) / kTile;
     totalTiles_ = (unsigned)(tilesX * tilesY);
-    shadeTiles_ = shade ? (unsigned)(((width_ + shadeTile_ - 1) / shadeTile_) * ((height_ + shadeTile_ - 1) / shadeTile_)) : 0u;
+    shadeTiles_ = shade ? totalTiles_ : 0u;
     totalPixels_ = ((size_t)width_ * height_ + 63) & ~(size_t)63;
     itemCap_ = totalTiles_ + binCap_ / part + 1u;
     partialCap_ = std::max(256u, binCap_ / (8u * part));
@@ -231,7 +231,6 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     put(ctr_, sizeof(DeviceCounters));
     put(viewCtr_, sizeof(ViewCounters));
     put(tileView_, std::max<size_t>(1, tiles) * 2);
-    put(shadeView_, std::max<size_t>(1, shadeTiles_) * 2);
     put(binCount_, tiles * 8);
     const size_t zeroed = A.used;
     put(viewDev_, sizeof(ViewDesc));
@@ -256,7 +255,10 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     put(binCursor_, tiles * 4);
     put(binList_, (size_t)binCap_ * 4);
     put(visSlot_, px * samples_ * 4);
-    put(visClass_, px);
+    // the order takes what the coverage classes, which such a draw does not keep, and a map of
+    // shading tiles took
+    const size_t shadeMap = shade ? (size_t)((width_ + shadeTile_ - 1) / shadeTile_) * ((height_ + shadeTile_ - 1) / shadeTile_) : 1;
+    put(order_, std::max(tiles * 8, px + 2 * shadeMap));
     if (!A.fits())
         return setError("iftrDrawNoAlloc: the draw needs " + std::to_string(A.used) + " bytes of scratch; the "
                         "no-allocation entry point holds " + std::to_string((size_t)IFHIP_NOALLOC_SCRATCH_BYTES));

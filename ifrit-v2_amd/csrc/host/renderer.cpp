@@ -66,7 +66,7 @@ TileRasterRenderer::~TileRasterRenderer() {
     for (DevBuf* b : {&vtx_, &idx_, &clip_, &recs_[0], &recs_[1], &recs_[2], &recs_[3], &recs_[4], &recs_[5], &bary_, &binFront_, &slotOf_, &binCount_, &binStart_, &binCursor_, &binList_,
                       &ctr_, &clipList_, &statPart_, &items_, &tilePartial_, &multiList_, &partials_, &visId_, &visDepth_, &visSlot_, &visClass_, &rgba8_, &rgba32f_, &texDesc_, &nnParams_, &nnGrads_, &nnM_, &nnV_,
                       &nnPacked_, &nnQinfo_, &lat32_, &latGrad_, &latM_, &latV_, &lat16_, &nnData_, &nnFeat_, &nnCount_,
-                      &nnLoss_, &nnEvalIn_, &nnEvalOut_, &nnGradPart_, &viewDev_, &tileView_, &shadeView_,
+                      &nnLoss_, &nnEvalIn_, &nnEvalOut_, &nnGradPart_, &viewDev_, &tileView_, &order_,
                       &groupBounds_, &swapped_, &scissorDev_,
                       &viewCtr_, &digest_, &polyKeys_, &meshVtx_, &meshIdx_})
         b->release();
@@ -811,7 +811,7 @@ bool TileRasterRenderer::prepare(int indexCount) {
                  clipList_.ensure((size_t)clipCap_ * 4 * nv) &&
                  statPart_.ensure((2 * (size_t)rasterGrid() + 2) * 8) &&
                  items_.ensure((size_t)itemCap_ * 16) && tilePartial_.ensure(tiles * 4) &&
-                 multiList_.ensure(tiles * 4) && partials_.ensure((size_t)partialCap_ * 256 * samples_ * 8) &&
+                 multiList_.ensure(tiles * 4) && order_.ensure(tiles * 8) && partials_.ensure((size_t)partialCap_ * 256 * samples_ * 8) &&
                  ensureZeroed(binCount_, tiles * 8) && binStart_.ensure(tiles * 4) && binCursor_.ensure(tiles * 4) &&
                  binList_.ensure((size_t)binCap_ * 4) &&
                  visId_.ensure(ps * 4) && visDepth_.ensure(ps * 4) && visSlot_.ensure(ps * 4) &&
@@ -897,9 +897,7 @@ bool TileRasterRenderer::layoutViews(int ntri) {
         D.invH = 1.0f / (float)h.height;
         D.tileBase = tiles;
         tiles += (unsigned)(D.tilesX * D.tilesY);
-        D.shadeBase = shade;
-        if (h.shade)
-            shade += (unsigned)(((h.width + shadeTile_ - 1) / shadeTile_) * ((h.height + shadeTile_ - 1) / shadeTile_));
+        if (h.shade) shade += (unsigned)(D.tilesX * D.tilesY);
         D.slotBase = (unsigned)v * sv;
         D.primBase = (unsigned)v * (unsigned)ntri;
         D.pixBase = pix;
@@ -908,7 +906,6 @@ bool TileRasterRenderer::layoutViews(int ntri) {
         layout.push_back(h.height);
         layout.push_back(h.shade);
     }
-    layout.push_back(shadeTile_);
     totalTiles_ = tiles;
     shadeTiles_ = shade;
     totalPixels_ = pix;
@@ -924,21 +921,14 @@ bool TileRasterRenderer::layoutViews(int ntri) {
         viewDesc_ = d;
     }
     if (layout != viewLayout_) {
-        std::vector<unsigned short> tv(std::max(1u, tiles)), sh(std::max(1u, shade));
+        std::vector<unsigned short> tv(std::max(1u, tiles));
         for (size_t v = 0; v < d.size(); v++) {
             const unsigned n = (unsigned)(d[v].tilesX * d[v].tilesY);
             std::fill(tv.begin() + d[v].tileBase, tv.begin() + d[v].tileBase + n, (unsigned short)v);
-            if (hv[v].shade) {
-                const unsigned m = (unsigned)(((hv[v].width + shadeTile_ - 1) / shadeTile_) *
-                                              ((hv[v].height + shadeTile_ - 1) / shadeTile_));
-                std::fill(sh.begin() + d[v].shadeBase, sh.begin() + d[v].shadeBase + m, (unsigned short)v);
-            }
         }
-        if (!tileView_.ensure(tv.size() * 2) || !shadeView_.ensure(sh.size() * 2))
-            return setError("hipMalloc view maps"), false;
+        if (!tileView_.ensure(tv.size() * 2)) return setError("hipMalloc view maps"), false;
         if (!ok(hipStreamSynchronize(stream_), "view maps") ||
-            !ok(hipMemcpy(tileView_.ptr, tv.data(), tv.size() * 2, hipMemcpyHostToDevice), "view maps") ||
-            !ok(hipMemcpy(shadeView_.ptr, sh.data(), sh.size() * 2, hipMemcpyHostToDevice), "view maps"))
+            !ok(hipMemcpy(tileView_.ptr, tv.data(), tv.size() * 2, hipMemcpyHostToDevice), "view maps"))
             return false;
         viewLayout_ = layout;
     }
@@ -949,7 +939,6 @@ Views TileRasterRenderer::deviceViews() const {
     Views V{};
     V.desc = viewDev_.as<ViewDesc>();
     V.tileView = tileView_.as<unsigned short>();
-    V.shadeView = shadeView_.as<unsigned short>();
     V.ctr = viewCtr_.as<ViewCounters>();
     V.count = (int)viewDesc_.size();
     V.slotsPerView = (unsigned)curTris_ + clipCap_;
@@ -1009,6 +998,15 @@ BinBufs TileRasterRenderer::binBufs() const {
 TriRecs TileRasterRenderer::recPtrs() const {
     return TriRecs{recs_[0].as<float4>(), recs_[1].as<float4>(), recs_[2].as<float4>(),
                    recs_[3].as<float4>(), recs_[4].as<float4>(), recs_[5].as<float4>()};
+}
+
+// planned: the tile plan of the draw lists the tiles.
+ShadeOrder TileRasterRenderer::shadeOrder(bool planned) const {
+    const bool shades = fsBound_ && fs_.desc.kind != IFHIP_FS_DEPTH_ONLY && !blend_.blendEnable;
+    const unsigned* const a = order_.as<unsigned>();
+    return ShadeOrder{planned ? a : nullptr, a + totalTiles_,
+                      reinterpret_cast<const uint4*>(ctr_.as<DeviceCounters>()->order), (int)totalTiles_,
+                      shades ? (int)shadeTiles_ : 0};
 }
 
 StatPartials TileRasterRenderer::statPtrs() const {
@@ -1135,9 +1133,11 @@ void TileRasterRenderer::enqueue(bool clear) {
     launch_geometry(sp, V, vin, idx_.as<int>(), recPtrs(), bary_.as<float4>(), bins, slotOf_.as<unsigned>(),
                     clipList_.as<unsigned>(), ctr_.as<DeviceCounters>(), s);
     mark(2);
+    const ShadeOrder order = shadeOrder(true);
     RasterQueue q{items_.as<uint4>(), tilePartial_.as<int>(), multiList_.as<unsigned>(),
                   partials_.as<unsigned long long>(), itemCap_, partialCap_, binCap_, rasterGrid(),
-                  numCUs_ * rasterGroupsPerCU_, partShift_, samples_ == 1 ? tileThreads_ : 256};
+                  numCUs_ * rasterGroupsPerCU_, order.shaded > 0 ? order_.as<unsigned>() : nullptr,
+                  order_.as<unsigned>() + tiles, samples_ == 8 ? 1 : 0, partShift_, samples_ == 1 ? tileThreads_ : 256};
     BinParams bp{};
     bp.tiles = tiles;
     scatterShape(&bp.grid, &bp.regions);
@@ -1200,10 +1200,11 @@ void TileRasterRenderer::enqueue(bool clear) {
         mark(4);
     }
     mark(5);
-    if (fsBound_ && fs_.desc.kind != IFHIP_FS_DEPTH_ONLY && shadeTiles_ > 0 && !blend_.blendEnable) {
+    if (order.shaded > 0) {
         const bool wantFloat = batch_.empty() && ((fb_ && !fb_->color.empty() && fb_->color[0]) || floatOut_);
-        const ShadeParams sh = shadeParams(wantFloat);
-        launch_shade(sh, V, (int)shadeTiles_, recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),
+        ShadeParams sh = shadeParams(wantFloat);
+        sh.cleared = clear ? 1 : 0;
+        launch_shade(sh, V, order, recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),
                      vtx_.as<float>(), idx_.as<int>(), texDesc_.as<TexDesc>(), texPool_, rgba8_.as<uchar4>(),
                      wantFloat ? rgba32f_.as<float4>() : nullptr, s);
     }
@@ -1241,7 +1242,8 @@ void TileRasterRenderer::enqueuePolygons(bool clear, const Views& V) {
         ShadeParams sh = shadeParams(wantFloat);
         sh.ntri = 0;  // every record carries its own vertex weights (bx, by)
         sh.swapped = nullptr;
-        launch_shade(sh, V, (int)shadeTiles_, recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),
+        sh.cleared = clear ? 1 : 0;
+        launch_shade(sh, V, shadeOrder(false), recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),
                      vtx_.as<float>(), idx_.as<int>(), texDesc_.as<TexDesc>(), texPool_, rgba8_.as<uchar4>(),
                      wantFloat ? rgba32f_.as<float4>() : nullptr, s);
     }

@@ -210,6 +210,7 @@ private:
     Views deviceViews() const;
     ShadeParams shadeParams(bool writeFloat) const;
     bool finish(bool clear, int indexCount);
+    ShadeOrder shadeOrder(bool planned) const;
     bool generalKeys(bool clear) const;
     bool drawsKeys(bool clear) const;
     void copyOutToHost();
@@ -268,7 +269,7 @@ private:
     bool reducePending_ = false;       // the last draw left its statistics to be reduced
     uint32_t* ids_ = nullptr;          // where the current draw writes primitive IDs itself
     bool keepSlots_ = true;            // whether the current draw's record slots and classes are read later
-    DevBuf viewDev_, tileView_, shadeView_, viewCtr_, digest_;
+    DevBuf viewDev_, tileView_, order_, viewCtr_, digest_;
 
     // launch parameters (IfritTuning) and graph replay
     int partShift_ = kRasterPartShift;

@@ -27,26 +27,27 @@ using dev::load_edges;
 
 // ---------------------------------------------------------------------------
 // Raster planning over the tiles of all views, in one launch: each workgroup
-// scans six quantities of its 256 tiles and takes its range of each with one
+// scans its quantities over its 256 tiles and takes its range of each with one
 // atomic on the draw's totals.  The workgroups' ranges come in any order, but
 // every tile's list is contiguous, the lists are disjoint, and a workgroup's
 // tiles stay together.  A tile's list is cut into items of at most 1 <<
 // partShift entries; items of more than kRasterPass entries are listed from
 // the front of the item array and the others from its back, so that the queue
 // hands out the long ones first.  Tiles with several items get a partial key
-// block per item and go to the front of multiList; empty tiles go to its back.
+// block per item and go to the front of multiList; empty tiles go to its back.  The
+// tiles of shaded views are also listed by the length of their lists (ShadeOrder).
 //
 // The plan is also where a draw's live counters end: it publishes the draw's
 // own and leaves the tile counts and the live counters at zero, so that the
 // next draw needs no clearing launch.
 // ---------------------------------------------------------------------------
-constexpr int kPlanQ = kTotCount;
+constexpr int kPlanQ = kTotCount + 2;  // PlanTotal, then the classes of ShadeOrder, two to a word
 
 struct TilePlan {
     unsigned q[kPlanQ];
 };
 
-__device__ __forceinline__ TilePlan tile_plan(unsigned c, bool valid, int sh) {
+__device__ __forceinline__ TilePlan tile_plan(unsigned c, bool valid, int cls, int sh) {
     TilePlan w;
     const unsigned part = 1u << sh;
     const unsigned p = valid ? (c + part - 1u) >> sh : 0u;
@@ -58,11 +59,13 @@ __device__ __forceinline__ TilePlan tile_plan(unsigned c, bool valid, int sh) {
     w.q[kTotPartials] = p > 1u ? p : 0u;
     w.q[kTotMulti] = p > 1u ? 1u : 0u;
     w.q[kTotEmpty] = valid && p == 0u ? 1u : 0u;
+    w.q[kTotCount] = cls < 2 ? 1u << (16 * cls) : 0u;
+    w.q[kTotCount + 1] = cls == 2 || cls == 3 ? 1u << (16 * (cls - 2)) : 0u;
     return w;
 }
 
 // Exclusive scan of kPlanQ values over a 256-thread workgroup; every thread must call it.
-__device__ __forceinline__ void scan256x6(unsigned* v, unsigned (*sWave)[4], unsigned* total) {
+__device__ __forceinline__ void plan_scan(unsigned* v, unsigned (*sWave)[4], unsigned* total) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < kPlanQ; k++) {
@@ -86,7 +89,8 @@ __global__ void __launch_bounds__(kPlanTiles) k_plan(uint2* __restrict__ cnt, un
                                                      DeviceCounters* ctr) {
     static_assert(kPlanTiles == 256, "one tile per thread");
     __shared__ unsigned sWave[kPlanQ][4];
-    __shared__ unsigned sBase[kPlanQ];
+    __shared__ unsigned sBase[kTotCount];
+    __shared__ unsigned long long sOrder[2];
     const int t = threadIdx.x, tile = blockIdx.x * kPlanTiles + t;
     if (blockIdx.x == 0) {
         // publish the draw's counters and clear the live ones
@@ -114,19 +118,31 @@ __global__ void __launch_bounds__(kPlanTiles) k_plan(uint2* __restrict__ cnt, un
         cnt[tile] = make_uint2(0u, 0u);
     }
     const unsigned total = c.x + c.y;
-    const TilePlan w = tile_plan(total, tile < n, q.partShift);
+    // the tile's class in the shading order, 4 where it is not shaded
+    int cls = 4;
+    if (q.orderA && tile < n && (V.count == 1 || V.desc[V.tileView[tile]].shade != 0))
+        cls = total == 0u ? 3 : !q.orderByLength || total <= (unsigned)kRasterPass ? 2 : total <= 4u * kRasterPass ? 1 : 0;
+    const TilePlan w = tile_plan(total, tile < n, cls, q.partShift);
     unsigned v[kPlanQ], sum[kPlanQ];
 #pragma unroll
     for (int k = 0; k < kPlanQ; k++) v[k] = w.q[k];
-    scan256x6(v, sWave, sum);
+    plan_scan(v, sWave, sum);
     // one lane per quantity, so that the atomics' round trips overlap
 #pragma unroll
     for (int k = 0; k < kPlanQ; k++)
-        if (t == k) sBase[k] = sum[k] ? atomicAdd(&ctr->tot[k], sum[k]) : 0u;
+        if (t == k && k < kTotCount) sBase[k] = sum[k] ? atomicAdd(&ctr->tot[k], sum[k]) : 0u;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const unsigned s = sum[kTotCount + k];
+        if (t == kTotCount + k)
+            sOrder[k] = s ? atomicAdd(reinterpret_cast<unsigned long long*>(ctr->order) + k,
+                                      ((unsigned long long)(s >> 16) << 32) | (s & 0xffffu))
+                          : 0ull;
+    }
     __syncthreads();
     if (tile >= n) return;
 #pragma unroll
-    for (int k = 0; k < kPlanQ; k++) v[k] += sBase[k];
+    for (int k = 0; k < kTotCount; k++) v[k] += sBase[k];
     const unsigned part = 1u << q.partShift;
     const unsigned st = v[kTotEntries], p = w.q[kTotLong] + w.q[kTotShort];
     start[tile] = st;
@@ -142,6 +158,12 @@ __global__ void __launch_bounds__(kPlanTiles) k_plan(uint2* __restrict__ cnt, un
     }
     if (p > 1u) q.multiList[v[kTotMulti]] = (unsigned)tile;
     if (p == 0u) q.multiList[(unsigned)n - 1u - v[kTotEmpty]] = (unsigned)tile;
+    if (cls < 4) {
+        // a and b from the front, b and a from the back
+        const unsigned at = (unsigned)(sOrder[cls >> 1] >> (32 * (cls & 1))) +
+                            ((v[kTotCount + (cls >> 1)] >> (16 * (cls & 1))) & 0xffffu);
+        (cls == 0 || cls == 3 ? q.orderA : q.orderB)[cls < 2 ? at : (unsigned)n - 1u - at] = (unsigned)tile;
+    }
     q.tilePartial[tile] = p > 1u ? (int)v[kTotPartials] : -1;
 }
 

@@ -6,7 +6,7 @@
 // view, S samples):
 //   views       ViewDesc[N]               per-view camera, size and bases
 //   tileView    ushort[tiles]             view of each 16x16 tile (tiles of all views)
-//   shadeView   ushort[shadeTiles]        view of each shading tile
+//   order       uint[2][tiles]            the shaded views' tiles, longest lists first (ShadeOrder)
 //   clip        float4[N][V]              vertex stage output (point and line modes; triangle draws
 //                                         transform in the geometry kernel)
 //   recs        TriRecs, N * SV slots     assembled triangles; in view v, slot v*SV + prim
@@ -59,7 +59,6 @@ struct ViewDesc {
     int width, height, tilesX, tilesY;
     float invW, invH;            // 1 / width, 1 / height (TileRasterRenderer.cpp:59-60)
     unsigned tileBase;           // first 16x16 tile
-    unsigned shadeBase;          // first shading tile (shaded views only)
     unsigned slotBase;           // first record slot (v * SV)
     unsigned primBase;           // first slotOf entry (v * T)
     unsigned long long pixBase;  // first pixel of the view's outputs
@@ -105,7 +104,6 @@ __host__ __device__ inline unsigned geom_waves(int ntri) {
 struct Views {
     const ViewDesc* desc;
     const unsigned short* tileView;   // view of each 16x16 tile
-    const unsigned short* shadeView;  // view of each shading tile
     ViewCounters* ctr;
     int count;
     unsigned slotsPerView;            // SV = T + clipCap
@@ -235,8 +233,9 @@ struct ShadeParams {
     float lightColor[4][4];
     int writeFloat;          // also write RGBA32F
     int ntri;                // view-local slots >= ntri are clip fans with their own bx, by
-    int shadeTile;           // pixels per side of a shading tile (8, 16 or 32): one wave shades
+    int shadeTile;           // side of a square of as many pixels as one wave shades (8, 16 or 32),
                              // its 8x8 sub-tiles in turn
+    int cleared;             // the draw cleared its targets
     NeuralShadeParams neural;  // programs 4 (neural material) and 5 (training features)
     const unsigned char* swapped;  // per record slot: vertices 0 and 2 exchanged by setup (null: none)
     float clearColor[4];     // colour of samples no triangle covers (the resolve weighs them)
@@ -292,6 +291,7 @@ struct DeviceCounters {
     unsigned bigCount;
     unsigned clipMax;    // largest per-view fan or clip count so far (sizes clipCap on overflow)
     unsigned long long assembled;
+    alignas(16) unsigned order[4];  // tiles in ShadeOrder's classes
     unsigned tot[8];     // PlanTotal: list entries, items of more than kRasterPass entries (front of the
                          // item array), other items, partial blocks, tiles cut into parts, empty tiles
     struct alignas(128) Live {
@@ -329,8 +329,29 @@ struct RasterQueue {
     unsigned itemCap, partialCap, binCap;
     int grid;         // raster workgroups
     int mergeGrid;    // half the merge workgroups
+    unsigned *orderA, *orderB;  // ShadeOrder's arrays, null where nothing is shaded
+    int orderByLength;          // classes 0 and 1 are used
     int partShift;
     int tileThreads;  // threads per tile at 1 sample per pixel: 64 or 256
+};
+
+// The order in which tiles are shaded: those whose lists are empty (class 3) last and,
+// at 8 samples, those of more than 4 kRasterPass entries (0) and of more than
+// kRasterPass (1) before the others (2), so that none of them is started last.  Class 0
+// fills `a` from the front and class 3 from its back, classes 1 and 2 `b`; count[] tells
+// how many each holds.  a is null where the tiles are taken as they are numbered
+// (point and line modes).
+//
+// List lengths order the work only where a pixel can hold many triangles; at one
+// sample it holds one and its cost is its texture taps, and the neighbours that no
+// longer follow each other cost the caches.  By length or not, in us: 8 samples,
+// 1920x1080: 107 or 118; 4 samples, 1009x767: 31 or 30; 1 sample: 92 or 92 (layered),
+// 73 or 72 (neural), 34 views 109 or 103.
+struct ShadeOrder {
+    const unsigned *a, *b;
+    const uint4* count;
+    int tiles;   // tiles of all views: entries of a and of b
+    int shaded;  // tiles of shaded views
 };
 
 // Launch wrappers.  launch_vertex (point and line modes) writes every view's
@@ -367,7 +388,7 @@ void launch_raster_ordered(const RasterParams& p, const Views& views, int sample
 // triangle * 3 + its point or edge.
 void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32_t* visId, hipStream_t s,
                          bool polygon = false);
-void launch_shade(const ShadeParams& p, const Views& views, int shadeTiles, TriRecs recs, const float4* bary, const uint32_t* visSlot,
+void launch_shade(const ShadeParams& p, const Views& views, const ShadeOrder& order, TriRecs recs, const float4* bary, const uint32_t* visSlot,
                   const float* vtx, const int* idx, const TexDesc* tex, const uint8_t* texPool, uchar4* rgba8,
                   float4* rgba32f, hipStream_t s);
 

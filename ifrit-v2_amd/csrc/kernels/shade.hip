@@ -920,47 +920,86 @@ __device__ __forceinline__ void shade_subtile(const ShadeParams& P, float3 cam, 
     if (rgba32f) rgba32f[pix] = r;
 }
 
-// One wave per shading tile of 8N x 8N pixels (N = 1, 2 or 4: P.shadeTile is
-// 8N), its 8x8 sub-tiles in row order.  Workgroups go to the XCDs in turn;
-// an XCD takes runs of kShadeRun consecutive tiles (texture and vertex reuse
-// in its L2), the runs of the eight XCDs interleaved, so that every XCD
-// shades a share of every part of the frame (one band per XCD leaves the
-// XCDs of the busy bands last to finish).  Tiles of all shaded views are
-// numbered one after another.
+// Clear colour of a tile no triangle is listed for, by one wave: what shade_subtile
+// writes where a pixel holds no fragment.
+template <int S, bool LAYERED>
+__device__ __forceinline__ void shade_empty(const ShadeParams& P, int width, int height, int ox, int oy, size_t pixBase,
+                                            uchar4* __restrict__ rgba8, float4* __restrict__ rgba32f) {
+    const float n = (float)S, inv = 1.0f / (float)S;
+    const float4 r = make_float4(P.clearColor[0] * n * inv, P.clearColor[1] * n * inv, P.clearColor[2] * n * inv,
+                                 P.clearColor[3] * n * inv);
+    const uchar4 c = make_uchar4((unsigned char)floorf(r.x * 255.0f + 0.5f), (unsigned char)floorf(r.y * 255.0f + 0.5f),
+                                 (unsigned char)floorf(r.z * 255.0f + 0.5f), (unsigned char)floorf(r.w * 255.0f + 0.5f));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int px = ox + ((int)threadIdx.x & 15), py = oy + 4 * k + ((int)threadIdx.x >> 4);
+        if (px >= width || py >= height) continue;
+        const size_t pix = pixBase + (size_t)py * width + px;
+        if (LAYERED && P.program == 5 && S == 1) P.neural.featOut[4 * pix + 1] = make_float4(0, 0, 0, 0);
+        if (!rc::scissor_pass(P.scissor, (float)px, (float)py)) continue;
+        rgba8[pix] = c;
+        if (rgba32f) rgba32f[pix] = r;
+    }
+}
+
+// One wave per 8x8 sub-tile of a 16x16 tile (N = 1), per tile (2) or per four tiles (4;
+// P.shadeTile is 8N), a wave per tile where a cleared draw's list is empty.  Tiles come
+// in ShadeOrder: in the order of the frame a wave whose pixels hold many triangles or
+// taps could start last, and the kernel waited for it alone (1920x1080, 8 samples,
+// 1.3M triangles: every wave had started after 84 us, the last ended after 122).
+// Workgroups go to the XCDs in turn; an XCD takes runs of kShadeRun consecutive
+// sub-tiles (texture and vertex reuse in its L2), the runs of the eight XCDs
+// interleaved, so that every XCD shades a share of every part of the frame (one
+// band per XCD leaves the XCDs of the busy bands last to finish).
 constexpr int kShadeRun = 64;
 
 template <int S, bool NEURAL, bool FP8, int N, bool LAYERED, bool GENERIC = false>
-__device__ __forceinline__ void shade_tiles(const ShadeParams& P, const Views& V, const TriRecs& recs,
-                                            const float4* __restrict__ baryAll,
+__device__ __forceinline__ void shade_tiles(const ShadeParams& P, const Views& V, const ShadeOrder& O,
+                                            const TriRecs& recs, const float4* __restrict__ baryAll,
                                             const uint32_t* __restrict__ visSlot, const float* __restrict__ vtx,
                                             const int* __restrict__ idx, const TexDesc* __restrict__ tex,
                                             const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8,
-                                            float4* __restrict__ rgba32f, int tiles) {
-    constexpr int T = 8 * N;
-    const int g = (int)(blockIdx.x >> 3);
-    const int tile = (g / kShadeRun) * (8 * kShadeRun) + (int)(blockIdx.x & 7u) * kShadeRun + g % kShadeRun;
-    if (tile >= tiles) return;
-    const unsigned view = dev::uniform_view_of(V.shadeView, (unsigned)tile);
-    const dev::UniformView& D = dev::uniform_view(V.desc + view);
-    const float4* const bary = baryAll + view_bary(V, view, P.ntri);
-    const int width = D.width, height = D.height;
-    const int local = tile - (int)D.shadeBase, perRow = (width + T - 1) / T;
-    const int ox0 = (local % perRow) * T, oy0 = (local / perRow) * T;
-    const size_t pb = (size_t)D.pixBase;
-    const float3 cam = make_float3(D.camera[0], D.camera[1], D.camera[2]);
-    const unsigned fanStart = D.slotBase + (unsigned)P.ntri;
-    if constexpr (N == 1) {
-        shade_subtile<S, NEURAL, FP8, LAYERED, GENERIC>(P, cam, width, height, fanStart, ox0, oy0, pb, recs, bary,
-                                                        visSlot + pb * S,
-                                      vtx, idx, tex, pool, rgba8 + pb, rgba32f ? rgba32f + pb : nullptr);
-    } else {
+                                            float4* __restrict__ rgba32f) {
+    const unsigned g = blockIdx.x >> 3;
+    const unsigned index = (g / kShadeRun) * (8 * kShadeRun) + (blockIdx.x & 7u) * kShadeRun + g % kShadeRun;
+    uint4 c = make_uint4(0u, 0u, (unsigned)O.tiles, 0u);
+    if (O.a) c = dev::uniform_words(O.count);
+    const unsigned listed = c.x + c.y + c.z, end = listed + c.w, busy = P.cleared ? listed : end;
+    unsigned pos, last;  // positions in the order
+    if constexpr (N == 1)
+        pos = index < 4u * busy ? index >> 2 : index - 3u * busy;
+    else
+        pos = N == 4 ? 4u * index : index;
+    last = min(N == 4 ? pos + 4u : pos + 1u, end);
 #pragma unroll 1
-        for (int k = 0; k < N * N; k++) {
-            const int ox = ox0 + (k % N) * 8, oy = oy0 + (k / N) * 8;
+    for (; pos < last; pos++) {
+        unsigned tile = pos;
+        if (O.a)
+            tile = dev::uniform_word(pos < c.x               ? O.a + pos
+                                     : pos < c.x + c.y       ? O.b + (pos - c.x)
+                                     : pos < listed          ? O.b + ((unsigned)O.tiles - 1u - (pos - c.x - c.y))
+                                                             : O.a + ((unsigned)O.tiles - 1u - (pos - listed)));
+        const unsigned view = V.count == 1 ? 0u : dev::uniform_view_of(V.tileView, tile);
+        const dev::UniformView& D = dev::uniform_view(V.desc + view);
+        if (!D.shade) continue;
+        const int width = D.width, height = D.height;
+        const unsigned local = tile - D.tileBase;
+        const int tx = (int)(local % (unsigned)D.tilesX) * 16, ty = (int)(local / (unsigned)D.tilesX) * 16;
+        const size_t pb = (size_t)D.pixBase;
+        if (pos >= busy) {
+            shade_empty<S, LAYERED>(P, width, height, tx, ty, pb, rgba8, rgba32f);
+            continue;
+        }
+        const float4* const bary = baryAll + view_bary(V, view, P.ntri);
+        const float3 cam = make_float3(D.camera[0], D.camera[1], D.camera[2]);
+        const unsigned fanStart = D.slotBase + (unsigned)P.ntri;
+#pragma unroll 1
+        for (unsigned k = N == 1 ? index & 3u : 0u; k < 4u; k += N == 1 ? 4u : 1u) {
+            const int ox = tx + (int)(k & 1u) * 8, oy = ty + (int)(k >> 1) * 8;
             if (ox >= width || oy >= height) continue;
             shade_subtile<S, NEURAL, FP8, LAYERED, GENERIC>(P, cam, width, height, fanStart, ox, oy, pb, recs, bary,
-                                                            visSlot + pb * S,
-                                          vtx, idx, tex, pool, rgba8 + pb, rgba32f ? rgba32f + pb : nullptr);
+                                                            visSlot + pb * S, vtx, idx, tex, pool, rgba8 + pb,
+                                                            rgba32f ? rgba32f + pb : nullptr);
         }
     }
 }
@@ -1119,10 +1158,10 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
 // per lane at once needs more registers: at four waves it is slower.
 template <int S, int N>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8)))
-k_shade(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ bary, const uint32_t* __restrict__ visSlot,
+k_shade(ShadeParams P, Views V, ShadeOrder O, TriRecs recs, const float4* __restrict__ bary, const uint32_t* __restrict__ visSlot,
         const float* __restrict__ vtx, const int* __restrict__ idx, const TexDesc* __restrict__ tex,
-        const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8, float4* __restrict__ rgba32f, int tiles) {
-    shade_tiles<S, false, false, N, false>(P, V, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f, tiles);
+        const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8, float4* __restrict__ rgba32f) {
+    shade_tiles<S, false, false, N, false>(P, V, O, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f);
 }
 
 // The single-texture and cube-map programs under a sampler other than
@@ -1130,33 +1169,33 @@ k_shade(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ bary, c
 // variant of k_shade, so that the default sampler's kernel carries none of it.
 template <int S, int N>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_shade_sampled(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ bary,
+k_shade_sampled(ShadeParams P, Views V, ShadeOrder O, TriRecs recs, const float4* __restrict__ bary,
                 const uint32_t* __restrict__ visSlot, const float* __restrict__ vtx, const int* __restrict__ idx,
                 const TexDesc* __restrict__ tex, const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8,
-                float4* __restrict__ rgba32f, int tiles) {
-    shade_tiles<S, false, false, N, false, true>(P, V, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f, tiles);
+                float4* __restrict__ rgba32f) {
+    shade_tiles<S, false, false, N, false, true>(P, V, O, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f);
 }
 
 // Layered GGX (programs 3 and 5): four waves per SIMD (at most 128 VGPRs), as
 // the neural program.
 template <int S, int N>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_shade_layered(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ bary,
+k_shade_layered(ShadeParams P, Views V, ShadeOrder O, TriRecs recs, const float4* __restrict__ bary,
                 const uint32_t* __restrict__ visSlot, const float* __restrict__ vtx, const int* __restrict__ idx,
                 const TexDesc* __restrict__ tex, const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8,
-                float4* __restrict__ rgba32f, int tiles) {
-    shade_tiles<S, false, false, N, true>(P, V, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f, tiles);
+                float4* __restrict__ rgba32f) {
+    shade_tiles<S, false, false, N, true>(P, V, O, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f);
 }
 
 // The neural material, held to four waves per SIMD like the other programs so
 // that the latent fetches stay overlapped.
 template <int S, bool FP8, int N>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_shade_neural(ShadeParams P, Views V, TriRecs recs, const float4* __restrict__ bary,
+k_shade_neural(ShadeParams P, Views V, ShadeOrder O, TriRecs recs, const float4* __restrict__ bary,
                const uint32_t* __restrict__ visSlot, const float* __restrict__ vtx, const int* __restrict__ idx,
                const TexDesc* __restrict__ tex, const uint8_t* __restrict__ pool, uchar4* __restrict__ rgba8,
-               float4* __restrict__ rgba32f, int tiles) {
-    shade_tiles<S, true, FP8, N, false>(P, V, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f, tiles);
+               float4* __restrict__ rgba32f) {
+    shade_tiles<S, true, FP8, N, false>(P, V, O, recs, bary, visSlot, vtx, idx, tex, pool, rgba8, rgba32f);
 }
 
 }  // namespace
@@ -1177,14 +1216,16 @@ void launch_blend_ordered(const ShadeParams& p, const BlendCoefs& b, int depthFu
 #undef IFRIT_BLEND_LAUNCH
 }
 
-void launch_shade(const ShadeParams& p, const Views& views, int shadeTiles, TriRecs recs, const float4* bary,
+void launch_shade(const ShadeParams& p, const Views& views, const ShadeOrder& order, TriRecs recs, const float4* bary,
                   const uint32_t* visSlot, const float* vtx, const int* idx, const TexDesc* tex,
                   const uint8_t* texPool, uchar4* rgba8, float4* rgba32f, hipStream_t s) {
-    if (shadeTiles <= 0) return;
-    // runs of kShadeRun tiles per XCD: the grid covers whole rounds of eight runs
-    const int perXcd = ((shadeTiles + 7) / 8 + kShadeRun - 1) / kShadeRun * kShadeRun;
+    if (order.shaded <= 0) return;
+    // runs of kShadeRun waves per XCD: the grid covers whole rounds of eight runs.  How many tiles are
+    // empty is not known here: the waves beyond the order's end have nothing to do
+    const int waves = p.shadeTile == 32 ? (order.shaded + 3) / 4 : p.shadeTile == 16 ? order.shaded : 4 * order.shaded;
+    const int perXcd = ((waves + 7) / 8 + kShadeRun - 1) / kShadeRun * kShadeRun;
     const dim3 grid(8 * perXcd);
-#define IFRIT_ARGS p, views, recs, bary, visSlot, vtx, idx, tex, texPool, rgba8, rgba32f, shadeTiles
+#define IFRIT_ARGS p, views, order, recs, bary, visSlot, vtx, idx, tex, texPool, rgba8, rgba32f
 #define IFRIT_SHADE_N(SN, NN)                                                                                      \
     do {                                                                                                            \
         if (p.program == 3 || p.program == 5)                                                                       \
