@@ -1137,7 +1137,8 @@ void TileRasterRenderer::enqueue(bool clear) {
     RasterQueue q{items_.as<uint4>(), tilePartial_.as<int>(), multiList_.as<unsigned>(),
                   partials_.as<unsigned long long>(), itemCap_, partialCap_, binCap_, rasterGrid(),
                   numCUs_ * rasterGroupsPerCU_, order.shaded > 0 ? order_.as<unsigned>() : nullptr,
-                  order_.as<unsigned>() + tiles, samples_ == 8 ? 1 : 0, partShift_, samples_ == 1 ? tileThreads_ : 256};
+                  order_.as<unsigned>() + tiles, samples_ == 8 ? 1 : 0, partShift_, samples_ == 1 ? tileThreads_ : 256,
+                  (size_t)curTris_ * viewDesc_.size() <= (size_t)rasterGrid() * kRasterPass ? 1 : 0};
     BinParams bp{};
     bp.tiles = tiles;
     scatterShape(&bp.grid, &bp.regions);

@@ -333,6 +333,8 @@ struct RasterQueue {
     int orderByLength;          // classes 0 and 1 are used
     int partShift;
     int tileThreads;  // threads per tile at 1 sample per pixel: 64 or 256
+    int wide;         // the raster takes passes of 2 kRasterPass entries: no more triangles than one
+                      // pass of kRasterPass per workgroup
 };
 
 // The order in which tiles are shaded: those whose lists are empty (class 3) last and,

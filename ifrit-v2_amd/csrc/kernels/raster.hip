@@ -33,7 +33,7 @@
 // Scheduling.  A tile's list is cut into parts of at most 1 << partShift entries and
 // all parts form one work queue that a persistent grid drains, so a few
 // tiles holding thousands of sub-pixel triangles do not serialise on one
-// compute unit.  A part goes through LDS in passes of kPass entries, all
+// compute unit.  A part goes through LDS in passes, all
 // merging into the tile's keys.  Each part rasterises into LDS; a tile with one part writes
 // its outputs from LDS, each part of a longer list stores its LDS keys to a
 // private partial block and a second kernel takes the minimum over the parts
@@ -53,8 +53,6 @@ namespace {
 
 using namespace dev;
 using namespace rc;
-
-constexpr int kPass = kRasterPass;  // the most list entries per pass through LDS
 
 // inside() with the three edge results combined by bitwise and: the same
 // arithmetic, and the compiler keeps the sample loop free of branches.
@@ -465,7 +463,7 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 
 // NT threads per tile: 256 (one pixel per thread) or, at 1 sample per pixel,
 // 64 (one wave per tile, four pixels per lane: more tiles in flight per
-// compute unit, for many small tiles).  Passes hold NT / 2 entries.  G: the
+// compute unit, for many small tiles).  Passes hold NT / 2 entries, WIDE ones NT.  G: the
 // general keys of a cleared draw with another depth function than LESS, which
 // also marks the tiles that met a NaN depth (nanTile): in those the function's
 // result depends on the order after all.
@@ -479,24 +477,28 @@ __device__ __forceinline__ int vis_at(int s, int p) { return s * kVisStride + p;
 // half-pixel triangles at 4 samples 327 -> 213 us, 34 views at 1 sample 525 -> 355 us.
 // Items and views through the scalar cache and a pass's entries loaded during the one
 // before: 351 -> 330 us at the 34 views, 215 -> 207 and 81 -> 79 us at the others.
-template <int S, int NT, bool G = false>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S == 8 ? 4 : 5, 8)))
+// WIDE is for draws that leave the chip idle (RasterQueue::wide), where the passes of
+// the longest list are what is waited for: 15 -> 11.5 us for a 256x256 target, 26 -> 22
+// at 1009x767 with 4 samples; their LDS leaves three workgroups per compute unit, and
+// with 1.3M triangles it costs 48 -> 56 us (1 sample) and 79 -> 90 us (8).
+template <int S, int NT, bool WIDE, bool G>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : S == 8 ? 4 : 5, 8)))
 k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slotOfAll,
          const WaveInfo* __restrict__ waves, const unsigned* __restrict__ binList, RasterQueue q,
          const unsigned* __restrict__ emptyEnd, float* __restrict__ visDepthAll, uint32_t* __restrict__ visSlotAll,
          uint8_t* __restrict__ visClassAll, StatPartials st, DeviceCounters* ctr, unsigned* __restrict__ nanTile) {
-    constexpr int PASS = NT / 2;            // list entries per pass through LDS
+    constexpr int PASS = WIDE ? NT : NT / 2;  // list entries per pass through LDS
     constexpr int UNITS = NT * 8;           // units expanded into LDS per round
     constexpr int PAIRS = 16 * PASS;        // (entry, window) pairs of a pass
     using Unit = typename std::conditional<S == 1, unsigned, unsigned short>::type;
     constexpr int PPT = 256 / NT;           // tile pixels per thread
-    static_assert(PASS <= kPass, "pairs and units encode the entry in 7 bits");
+    static_assert(PASS <= 256, "pairs and units encode the entry in 8 bits");
     // key of sample s of tile pixel p at vis_at(s, p)
     __shared__ unsigned long long sVis[S * kVisStride];
     static_assert(sizeof(TileOut<S>) <= sizeof(sVis), "output staging reuses sVis");
     __shared__ TriRec sRec[PASS];            // q2.z: bit 31 when the tile is accepted, else the pixel box
     __shared__ Unit sUnit[UNITS];            // entry << 8 | tile pixel, and << 2 | class at 1 sample
-    __shared__ unsigned short sPair[PAIRS];  // entry << 9 | window row << 5 | column << 1 | a tile's block
+    __shared__ unsigned short sPair[PAIRS];  // entry << 8 | window row << 4 | column
     __shared__ unsigned sWave[4];
     __shared__ unsigned sItem;
 
@@ -659,12 +661,12 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                 while (blocks) {
                     const int q = __ffs(blocks) - 1;
                     blocks &= blocks - 1u;
-                    sPair[pp++] = (unsigned short)((t << 9) | ((q >> 2) << 7) | ((q & 3) << 3) | 1);
+                    sPair[pp++] = (unsigned short)((t << 8) | ((q >> 2) << 6) | ((q & 3) << 2));
                 }
             } else {
                 for (int k = 0; k < (int)n; k++) {
                     const int wx = bx0 + 4 * few_col(k, wcols), wy = by0 + 4 * few_row(k, wcols);
-                    sPair[pp++] = (unsigned short)((t << 9) | (wy << 5) | (wx << 1));
+                    sPair[pp++] = (unsigned short)((t << 8) | (wy << 4) | wx);
                 }
             }
             __syncthreads();
@@ -675,9 +677,9 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                 bool acc = false;
                 if (p0 + t < TP) {
                     const unsigned pr = sPair[p0 + t];
-                    pe = (int)(pr >> 9);
-                    wx = (int)((pr >> 1) & 15u);
-                    wy = (int)((pr >> 5) & 15u);
+                    pe = (int)(pr >> 8);
+                    wx = (int)(pr & 15u);
+                    wy = (int)((pr >> 4) & 15u);
                     const unsigned bits = __float_as_uint(sRec[pe].q2.z);
                     acc = (bits >> 31) != 0u;  // the tile, or below the block, is accepted
                     // up to the frame's and the box's last column and row
@@ -688,7 +690,7 @@ k_raster(RasterParams P, Views V, TriRecs recs, const unsigned* __restrict__ slo
                         const Edges E = load_edges(sRec[pe]);
                         const float fx = (float)(tx0 + wx), fy = (float)(ty0 + wy);
                         if constexpr (S == 1) {
-                            if (pr & 1u) acc = block_accepted(E, fx, fy);
+                            if (((wx | wy) & 3) == 0) acc = block_accepted(E, fx, fy);
                             const unsigned in = window_inside(E, fx, fy);
                             window_classes(in, wx, wy, groups, quads);
                             pm &= in;
@@ -875,13 +877,21 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
     const int t = threadIdx.x;
     unsigned long long frags = 0, covs = 0;
     OrderedTiles T(q, ctr, nanTile == nullptr);
-    int tile = (int)blockIdx.x - (int)gridDim.x;
+    // with nanTile: the marks of up to 64 of the workgroup's tiles at a time (a bit each)
+    unsigned long long marked = 0;
+    int tile = 0, round = 0, left = 0;
     for (;;) {
         unsigned start, cnt;
         if (nanTile) {
-            tile += gridDim.x;
-            if (tile >= tiles) break;
-            if (nanTile[2 * tile] == 0u) continue;
+            while (!marked) {
+                if (left >= tiles) return;
+                const int mine = (int)blockIdx.x + (64 * round + (t & 63)) * (int)gridDim.x;
+                marked = __ballot(mine < tiles && nanTile[2 * mine] != 0u);
+                __syncthreads();  // every wave has read the marks before the first is cleared
+                left = (int)blockIdx.x + 64 * ++round * (int)gridDim.x;
+            }
+            tile = (int)blockIdx.x + (64 * (round - 1) + __ffsll(marked) - 1) * (int)gridDim.x;
+            marked &= marked - 1ull;
             start = B.start[tile];
             cnt = start >= P.binCap ? 0u : min(B.cursor[tile] - start, P.binCap - start);
         } else if (!T.next(q, B, tiles, &sItem, tile, start, cnt)) {
@@ -939,10 +949,7 @@ __global__ void __launch_bounds__(256) k_raster_ordered(RasterParams P, Views V,
             }
             if (S == 1 && vis.cls) vis.cls[C.pix] = (uint8_t)cls;
         }
-        if (nanTile) {
-            __syncthreads();  // every thread has read the mark
-            if (t == 0) nanTile[2 * tile] = 0u;
-        }
+        if (nanTile && t == 0) nanTile[2 * tile] = 0u;
     }
     if (nanTile) return;  // the key raster has counted
     const unsigned long long tf = block_sum256(frags);
@@ -999,33 +1006,42 @@ void launch_slot_to_prim(const uint32_t* visSlot, TriRecs recs, size_t n, uint32
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                    const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
                    uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s) {
-#define IFRIT_RASTER_LAUNCH(...)                                                                                   \
-    hipLaunchKernelGGL((k_raster<__VA_ARGS__>), dim3(q.grid), dim3(q.tileThreads), 0, s, p, views, recs, slotOf,  \
+#define IFRIT_RASTER_LAUNCH_G(SN, NT, WIDE, G)                                                                     \
+    hipLaunchKernelGGL((k_raster<SN, NT, WIDE, G>), dim3(q.grid), dim3(NT), 0, s, p, views, recs, slotOf,          \
                        bins.waves, bins.list, q, q.multiList + tiles - 1, visDepth, visSlot, visClass, st, ctr,   \
                        bins.cnt)
-    if (p.general) {
-        switch (samples) {
-            case 1:
-                if (q.tileThreads == 64)
-                    IFRIT_RASTER_LAUNCH(1, 64, true);
-                else
-                    IFRIT_RASTER_LAUNCH(1, 256, true);
-                break;
-            case 4: IFRIT_RASTER_LAUNCH(4, 256, true); break;
-            default: IFRIT_RASTER_LAUNCH(8, 256, true); break;
-        }
+#define IFRIT_RASTER_LAUNCH(SN, NT, WIDE)                                                                          \
+    do {                                                                                                           \
+        if (p.general)                                                                                             \
+            IFRIT_RASTER_LAUNCH_G(SN, NT, WIDE, true);                                                             \
+        else                                                                                                       \
+            IFRIT_RASTER_LAUNCH_G(SN, NT, WIDE, false);                                                            \
+    } while (0)
+    if (samples == 1 && q.tileThreads == 64) {
+        IFRIT_RASTER_LAUNCH(1, 64, false);
         return;
     }
     switch (samples) {
         case 1:
-            if (q.tileThreads == 64)
-                IFRIT_RASTER_LAUNCH(1, 64);
+            if (q.wide)
+                IFRIT_RASTER_LAUNCH(1, 256, true);
             else
-                IFRIT_RASTER_LAUNCH(1, 256);
+                IFRIT_RASTER_LAUNCH(1, 256, false);
             break;
-        case 4: IFRIT_RASTER_LAUNCH(4, 256); break;
-        default: IFRIT_RASTER_LAUNCH(8, 256); break;
+        case 4:
+            if (q.wide)
+                IFRIT_RASTER_LAUNCH(4, 256, true);
+            else
+                IFRIT_RASTER_LAUNCH(4, 256, false);
+            break;
+        default:
+            if (q.wide)
+                IFRIT_RASTER_LAUNCH(8, 256, true);
+            else
+                IFRIT_RASTER_LAUNCH(8, 256, false);
+            break;
     }
+#undef IFRIT_RASTER_LAUNCH_G
 #undef IFRIT_RASTER_LAUNCH
 }
 
@@ -1034,7 +1050,7 @@ void launch_raster_ordered(const RasterParams& p, const Views& views, int sample
                            uint8_t* visClass, StatPartials st, bool nanTilesOnly, DeviceCounters* ctr,
                            hipStream_t s) {
 #define IFRIT_ORDERED_LAUNCH(SN)                                                                                  \
-    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(q.grid), dim3(256), 0, s, p, views, recs, bins, q, tiles, p.ntri,  \
+    hipLaunchKernelGGL(k_raster_ordered<SN>, dim3(nanTilesOnly ? (q.grid + 1) / 2 : q.grid), dim3(256), 0, s, p, views, recs, bins, q, tiles, p.ntri,  \
                        visDepth, visSlot, visClass, st, nanTilesOnly ? bins.cnt : nullptr, ctr)
     switch (samples) {
         case 1: IFRIT_ORDERED_LAUNCH(1); break;
