@@ -41,14 +41,12 @@ def log(msg):
 
 
 def algorithmic_bytes(scene, stage: str) -> float:
-    """Compulsory HBM bytes of one launch of each stage: positions in and clip positions out, indices and
-    clip positions in, per-sample depth and ID out, RGBA8 out plus one texel per pixel with its mips."""
+    """Compulsory HBM bytes of one launch of each stage: positions and indices in (the vertex transform is
+    part of setup), per-sample depth and ID out, RGBA8 out plus one texel per pixel with its mips."""
     W, H, S = scene.width, scene.height, scene.samples
     V, T = scene.vertices.shape[0], scene.num_triangles
-    if stage == "vertex":
-        return V * 12 + V * 16            # positions in, clip positions out
     if stage == "setup":
-        return T * 12 + 3 * T * 16        # indices and clip positions in
+        return V * 12 + T * 12            # positions and indices in
     if stage == "raster":
         return W * H * S * 8              # per-sample depth + primitive id out
     if stage == "shade":
@@ -66,10 +64,10 @@ def frame_bytes(scene) -> float:
     return V * scene.stride * 4 + 12 * T + W * H * S * 8 + 4 * W * H + tau
 
 
-# kernels of each timed stage (the raster stage's outputs are written by both
-# k_raster and, for tiles whose list was cut into items, k_raster_merge)
-STAGE_KERNELS = {"vertex": ["k_vertex"], "setup": ["k_setup", "k_clip"],
-                 "bin": ["k_bin_small", "k_bin_big_count", "k_plan_sums", "k_plan_scan", "k_plan_write"],
+# kernels of each timed stage (the vertex stage has one of its own only in the point
+# and line modes; the raster stage's outputs are written by both k_raster and, for
+# tiles whose list was cut into items, k_raster_merge)
+STAGE_KERNELS = {"vertex": [], "setup": ["k_geometry", "k_clip"], "bin": ["k_plan", "k_scatter"],
                  "raster": ["k_raster", "k_raster_merge"], "shade": ["k_shade"]}
 
 

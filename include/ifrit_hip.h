@@ -404,8 +404,8 @@ typedef struct {
     int64_t coveredSamples;
     uint32_t status;       /* overflow bits, 0 when the frame is complete */
     uint32_t retries;      /* frames re-run with larger buffers */
-    float stageMs[8];      /* vertex (and counter reset), setup (clip, cull), bin, raster, raster merge,
-                              shade, (unused), (unused) */
+    float stageMs[8];      /* vertex (point and line modes; triangles are transformed in setup), setup
+                              (clip, cull), bin, raster, raster merge, shade, (unused), (unused) */
 } IfritFrameStats;
 
 void iftrGetFrameStats(IfritRendererHandle* h, IfritFrameStats* out);
