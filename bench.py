@@ -67,7 +67,7 @@ def frame_bytes(scene) -> float:
 # kernels of each timed stage (the vertex stage has one of its own only in the point
 # and line modes; the raster stage's outputs are written by both k_raster and, for
 # tiles whose list was cut into items, k_raster_merge)
-STAGE_KERNELS = {"vertex": [], "setup": ["k_geometry"], "bin": ["k_clip_plan", "k_scatter"],
+STAGE_KERNELS = {"vertex": [], "setup": ["k_geometry", "k_clip"], "bin": ["k_plan", "k_scatter"],
                  "raster": ["k_raster", "k_raster_merge"], "shade": ["k_shade"]}
 
 

@@ -1133,8 +1133,8 @@ void TileRasterRenderer::enqueue(bool clear) {
     sp.bigCap = bigCap_;
     sp.bigThreshold = bigThreshold_;
     const BinBufs bins = binBufs();
-    launch_geometry(sp, V, vin, idx_.as<int>(), recPtrs(), bins, clipList_.as<unsigned>(),
-                    ctr_.as<DeviceCounters>(), s);
+    launch_geometry(sp, V, vin, idx_.as<int>(), recPtrs(), bary_.as<float4>(), bins, slotOf_.as<unsigned>(),
+                    clipList_.as<unsigned>(), ctr_.as<DeviceCounters>(), s);
     mark(2);
     const ShadeOrder order = shadeOrder(true);
     RasterQueue q{items_.as<uint4>(), tilePartial_.as<int>(), multiList_.as<unsigned>(),
@@ -1143,13 +1143,12 @@ void TileRasterRenderer::enqueue(bool clear) {
                   order_.as<unsigned>() + tiles, samples_ == 8 ? 1 : 0, partShift_, samples_ == 1 ? tileThreads_ : 256,
                   (size_t)curTris_ * viewDesc_.size() <= (size_t)rasterGrid() * kRasterPass ? 1 : 0};
     BinParams bp{};
+    bp.tiles = tiles;
     scatterShape(&bp.grid, &bp.regions);
     bp.ntri = curTris_;
     bp.clipCap = clipCap_;
     bp.binCap = binCap_;
     bp.bigCap = bigCap_;
-    launch_clip_plan(sp, V, vin, idx_.as<int>(), recPtrs(), bary_.as<float4>(), bins, slotOf_.as<unsigned>(),
-                     clipList_.as<unsigned>(), q, tiles, ctr_.as<DeviceCounters>(), s);
     launch_bin(bp, V, recPtrs(), bins, q, statPtrs(), ctr_.as<DeviceCounters>(), s);
     mark(3);
     RasterParams rp{};

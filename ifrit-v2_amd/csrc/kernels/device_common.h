@@ -278,8 +278,8 @@ __device__ __forceinline__ void bin_lanes(const Edges& E, int4 b, unsigned tileB
 constexpr unsigned kBigParts = 32;
 template <bool SCATTER>
 __device__ __forceinline__ void bin_big(unsigned nbig, const Views& V, const TriRecs& recs, const BinBufs& B,
-                                        unsigned binCap, unsigned part, unsigned parts) {
-    for (unsigned u = part; u < nbig * kBigParts; u += parts) {
+                                        unsigned binCap) {
+    for (unsigned u = blockIdx.x; u < nbig * kBigParts; u += gridDim.x) {
         const uint4 g = B.big[u / kBigParts];
         const int4 b = unpack_box(make_uint2(g.y, g.z));
         const int w = b.z - b.x + 1, area = w * (b.w - b.y + 1);

@@ -173,6 +173,7 @@ constexpr int kMadeSums = 64, kMadeStride = 16;
 constexpr int kGroupTris = kGeomBlock;
 
 struct BinParams {
+    int tiles;          // tiles of all views
     int grid;           // workgroups of the scatter launch
     int regions;        // geometry waves a scatter wave takes at a time (1 .. 64)
     int ntri;
@@ -295,10 +296,7 @@ struct DeviceCounters {
                          // item array), other items, partial blocks, tiles cut into parts, empty tiles
     struct alignas(128) Live {
         unsigned status, bigCount, clipMax, fans;  // fans: fan triangles assembled
-        unsigned left;                             // 1: the geometry kernel left triangles to clip or count
     } live;
-    // shares of k_clip_plan's clipping taken, and those done
-    alignas(128) unsigned clipTaken, clipDone;
     alignas(128) unsigned itemHeads[kItemStreams][32];  // next item of each stream, one 128-byte line each
 };
 
@@ -365,15 +363,13 @@ void launch_vertex(const VertexInput& in, int nverts, const Views& views, float4
 void launch_group_bounds(const float* vtx, int stride, int nverts, const int* idx, int ntri, float4* bounds,
                          hipStream_t s);
 void launch_reset(const Views& views, DeviceCounters* ctr, hipStream_t s);
-// Vertex transform, triangle setup and the bin counts.
+// Vertex transform, triangle setup and the bin counts, then the triangles that
+// cross w = 0 and those deferred by the bin count.
 void launch_geometry(const SetupParams& p, const Views& views, const VertexInput& in, const int* idx, TriRecs recs,
-                     const BinBufs& bins, unsigned* clipList, DeviceCounters* ctr, hipStream_t s);
-// The triangles that cross w = 0 and those deferred by the bin count, then the tile plan.
-void launch_clip_plan(const SetupParams& p, const Views& views, const VertexInput& in, const int* idx, TriRecs recs,
-                      float4* bary, const BinBufs& bins, unsigned* slotOf, const unsigned* clipList,
-                      const RasterQueue& q, int tiles, DeviceCounters* ctr, hipStream_t s);
+                     float4* bary, const BinBufs& bins, unsigned* slotOf, unsigned* clipList, DeviceCounters* ctr,
+                     hipStream_t s);
 void launch_finalize(StatPartials st, const Views& views, DeviceCounters* ctr, HostCounters* out, hipStream_t s);
-// The scatter into the tile lists.
+// The tile plan and the scatter into the tile lists.
 void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
                 StatPartials st, DeviceCounters* ctr, hipStream_t s);
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
