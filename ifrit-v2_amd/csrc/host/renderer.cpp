@@ -1068,6 +1068,7 @@ ShadeParams TileRasterRenderer::shadeParams(bool writeFloat) const {
     std::memcpy(sh.lightColor, d.lightColor, sizeof(sh.lightColor));
     sh.writeFloat = writeFloat ? 1 : 0;
     sh.ntri = curTris_;
+    sh.fanCap = clipCap_;
     sh.shadeTile = shadeTile_;
     sh.neural = neuralShadeParams();
     sh.swapped = needSwapFlags() ? swapped_.as<unsigned char>() : nullptr;
@@ -1245,6 +1246,8 @@ void TileRasterRenderer::enqueuePolygons(bool clear, const Views& V) {
         const bool wantFloat = (fb_ && !fb_->color.empty() && fb_->color[0]) || floatOut_;
         ShadeParams sh = shadeParams(wantFloat);
         sh.ntri = 0;  // every record carries its own vertex weights (bx, by)
+        sh.fanCap = (unsigned)curIdx_;
+        sh.ownWeights = 1;
         sh.swapped = nullptr;
         sh.cleared = clear ? 1 : 0;
         launch_shade(sh, V, shadeOrder(false), recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),

@@ -233,6 +233,8 @@ struct ShadeParams {
     float lightColor[4][4];
     int writeFloat;          // also write RGBA32F
     int ntri;                // view-local slots >= ntri are clip fans with their own bx, by
+    unsigned fanCap;         // fans per view that `bary` holds, or slots in the point and line modes
+    int ownWeights;          // point and line modes: every slot of the draw has its bx, by
     int shadeTile;           // side of a square of as many pixels as one wave shades (8, 16 or 32),
                              // its 8x8 sub-tiles in turn
     int cleared;             // the draw cleared its targets

@@ -1,0 +1,92 @@
+"""Colours of pixels that keep a record of an earlier, larger draw.
+
+Draws without clear shade every pixel again, those they leave alone by the slot of
+the draw that won them: 12k triangles and then two, or a few lines, over them (slots
+beyond the second draw's records and beyond every clip fan it reserves, 4096 at the
+least), and a textured scene followed by its own first triangles, of which none
+passes.  Flat colours follow the primitive IDs (at most 16 roundings, as in the
+shading-order tests); the textured frame must not change by a bit.
+"""
+import numpy as np
+import pytest
+
+from ifrit_hip import scenes
+from oracle import oracle as O
+
+from test_gpu_shade_order import _flat, _scene
+
+pytestmark = pytest.mark.gpu
+
+EYE = np.eye(4, dtype=np.float32)
+BLACK = np.zeros(4)
+
+
+def _overlay():
+    clip = np.array([[-0.9, -0.8, 0.05, 1], [0.7, -0.5, 0.05, 1], [-0.2, 0.9, 0.05, 1],
+                     [0.9, 0.8, 0.04, 1], [-0.6, 0.7, 0.04, 1], [0.1, -0.9, 0.04, 1]], np.float32)
+    return clip, np.array([0, 1, 2, 2, 1, 0, 3, 4, 5, 5, 4, 3], np.int32)
+
+
+def _bind(r, W, H, samples, clip, idx):
+    r.bind_geometry(clip, idx, EYE, clip_passthrough=True)
+    r.bind_fragment_program(scenes.Scene("t", W, H, samples, clip, idx, EYE, program=scenes.PROGRAM_FLAT))
+
+
+@pytest.mark.parametrize("samples", [1, 4])
+def test_small_draw_over_a_large_one(renderer_factory, samples):
+    r = renderer_factory()
+    r.set_float_output(True)
+    W, H = 320, 201
+    clip, idx = _scene(np.random.default_rng(samples), W, H, 5600)
+    over, oi = _overlay()
+    f = O.Frame().render(W, H, samples, clip, idx)
+    g = O.Frame().render(W, H, samples, over, oi, clear=False, depth_in=f.depth)
+    r.set_target(W, H, samples)
+    _bind(r, W, H, samples, clip, idx)
+    r.draw()
+    _bind(r, W, H, samples, over, oi)
+    print(f"[kept slots s={samples}]", flush=True)
+    r.draw(clear=False)
+    ids = np.where(g.ids != 0xFFFFFFFF, g.ids, f.ids)
+    assert (g.ids != 0xFFFFFFFF).any() and (f.ids[g.ids == 0xFFFFFFFF] > 5000).any()
+    assert np.array_equal(r.visibility()[0], ids)
+    want = _flat(ids.reshape(H, W, samples), BLACK).mean(2)
+    assert np.abs(r.color_f32().reshape(H, W, 4) - want).max() < 1e-6
+
+
+def test_lines_over_a_large_draw(renderer_factory):
+    r = renderer_factory()
+    r.set_float_output(True)
+    W, H = 320, 201
+    clip, idx = _scene(np.random.default_rng(7), W, H, 5600)
+    clip[:36, 0] = 3.0  # the slots that the lines' records take hold no pixel
+    over, oi = _overlay()
+    f = O.Frame().render(W, H, 1, clip, idx)
+    g = O.Frame().render_polygons(W, H, over, oi, 1, clear=False, depth_in=f.depth)
+    r.set_target(W, H, 1)
+    _bind(r, W, H, 1, clip, idx)
+    r.draw()
+    r.set_polygon_mode(1)
+    _bind(r, W, H, 1, over, oi)
+    print("[kept slots, lines]", flush=True)
+    r.draw(clear=False)
+    line = g.ids != 0xFFFFFFFF
+    assert line.any() and (f.ids[~line & (f.ids != 0xFFFFFFFF)] > 5000).any()
+    want = _flat(np.where(line, g.ids // 3, f.ids).reshape(H, W), BLACK)
+    assert np.abs(r.color_f32().reshape(H, W, 4) - want).max() < 1e-6
+
+
+@pytest.mark.parametrize("samples", [1, 4])
+def test_first_triangles_of_a_textured_scene(renderer_factory, samples):
+    s = scenes.config2(200, 150, samples, spheres=8, tex_size=64)
+    assert s.num_triangles == 40960
+    r = renderer_factory()
+    r.set_float_output(True)
+    r.load_scene(s)
+    assert r.draw()["clippedTriangles"] == 0
+    before = r.color_f32()
+    r.num_indices = 6
+    print(f"[kept slots, textured s={samples}]", flush=True)
+    st = r.draw(clear=False)
+    assert st["inputTriangles"] == 2
+    assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
