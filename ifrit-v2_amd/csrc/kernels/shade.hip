@@ -682,13 +682,16 @@ __device__ __forceinline__ void shade_subtile(const ShadeParams& P, float3 cam, 
     const int px = ox + (lane & 7);
     const int py = oy + (lane >> 3);
     const bool inFb = px < width && py < height;
+    // outside the scissor a pixel keeps its colour, and the slots of an earlier draw, which this one
+    // may not hold any more
+    const bool drawn = inFb && rc::scissor_pass(P.scissor, (float)px, (float)py);
     const size_t pix = (size_t)py * width + px;
 
     // 1. distinct triangles of the pixel
     unsigned ids[S];
 #pragma unroll
     for (int s = 0; s < S; s++) ids[s] = 0xffffffffu;
-    if (inFb) {
+    if (drawn) {
         if constexpr (S % 4 == 0) {
             // a pixel's samples are contiguous and 16-byte aligned
 #pragma unroll
@@ -934,7 +937,7 @@ __device__ __forceinline__ void shade_subtile(const ShadeParams& P, float3 cam, 
         }
         __syncthreads();
     }
-    if (!inFb || !rc::scissor_pass(P.scissor, (float)px, (float)py)) return;
+    if (!drawn) return;
     const float inv = 1.0f / (float)S;
     const float4 r = make_float4(sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv);
     rgba8[pix] = make_uchar4((unsigned char)floorf(r.x * 255.0f + 0.5f), (unsigned char)floorf(r.y * 255.0f + 0.5f),

@@ -4,7 +4,8 @@ Draws without clear shade every pixel again, those they leave alone by the slot 
 the draw that won them: 12k triangles and then two, or a few lines, over them (slots
 beyond the second draw's records and beyond every clip fan it reserves, 4096 at the
 least), and a textured scene followed by its own first triangles, of which none
-passes.  Flat colours follow the primitive IDs (at most 16 roundings, as in the
+passes; and a scissored draw of a few over 12k, which keeps slots outside its
+rectangle.  Flat colours follow the primitive IDs (at most 16 roundings, as in the
 shading-order tests); the textured frame must not change by a bit.
 """
 import numpy as np
@@ -90,3 +91,30 @@ def test_first_triangles_of_a_textured_scene(renderer_factory, samples):
     st = r.draw(clear=False)
     assert st["inputTriangles"] == 2
     assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
+
+
+@pytest.mark.parametrize("samples", [1, 8])
+@pytest.mark.parametrize("tile", [8, 32])
+def test_scissored_small_draw_over_a_large_one(renderer_factory, tile, samples):
+    s = scenes.config2(200, 150, samples, spheres=8, tex_size=64)
+    r = renderer_factory()
+    r.set_tuning(shadeTile=tile)
+    r.set_float_output(True)
+    r.load_scene(s)
+    r.draw()
+    before = r.color_f32()
+    r.set_clear_values((0.25, 0.5, 0.75, 1.0))
+    r.num_indices = 3 * 2 * 5120  # the first two spheres, one inside the scissor
+    r.draw()
+    alone = r.color_f32()
+    r.set_clear_values()
+    r.num_indices = s.indices.size
+    r.draw()
+    r.set_clear_values((0.25, 0.5, 0.75, 1.0))
+    r.set_scissors([(21.0, 18.0, 102.0, 90.0)])
+    r.num_indices = 3 * 2 * 5120
+    print(f"[kept slots, scissor s={samples} tile={tile}]", flush=True)
+    r.draw()
+    y, x = np.mgrid[:s.height, :s.width]
+    inside = ((x >= 21) & (x <= 123) & (y >= 18) & (y <= 108))[..., None]
+    assert np.array_equal(r.color_f32(), np.where(inside, alone, before))
