@@ -281,8 +281,10 @@ __global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs r
         atomicAdd(&B.made[(blockIdx.x % kMadeSums) * kMadeStride],
                   (unsigned long long)(sMade[0] + sMade[1] + sMade[2] + sMade[3]));
         if (blockIdx.x == 0) {
-            // on a bin or work-list overflow nothing is rasterised (plan_fits); the host grows the
-            // buffers and draws again
+            // on a bin or work-list overflow nothing is rasterised (plan_fits) and nothing shaded, as the
+            // record slots are those of earlier draws; the host grows the buffers and draws again
+            if (!dev::plan_fits(ctr, q))
+                for (int k = 0; k < 4; k++) ctr->order[k] = 0u;
             if (ctr->tot[kTotEntries] > q.binCap) atomicOr(&ctr->status, kStatusBinOverflow);
             if (!dev::plan_items_fit(ctr, q)) atomicOr(&ctr->status, kStatusRasterOverflow);
         }

@@ -5,13 +5,14 @@ the draw that won them: 12k triangles and then two, or a few lines, over them (s
 beyond the second draw's records and beyond every clip fan it reserves, 4096 at the
 least), and a textured scene followed by its own first triangles, of which none
 passes; and a scissored draw of a few over 12k, which keeps slots outside its
-rectangle.  Flat colours follow the primitive IDs (at most 16 roundings, as in the
+rectangle.  A draw whose tile lists do not fit draws nothing and must leave the
+colours alone.  Flat colours follow the primitive IDs (at most 16 roundings, as in the
 shading-order tests); the textured frame must not change by a bit.
 """
 import numpy as np
 import pytest
 
-from ifrit_hip import scenes
+from ifrit_hip import IfritError, scenes
 from oracle import oracle as O
 
 from test_gpu_shade_order import _flat, _scene
@@ -118,3 +119,29 @@ def test_scissored_small_draw_over_a_large_one(renderer_factory, tile, samples):
     y, x = np.mgrid[:s.height, :s.width]
     inside = ((x >= 21) & (x <= 123) & (y >= 18) & (y <= 108))[..., None]
     assert np.array_equal(r.color_f32(), np.where(inside, alone, before))
+
+
+@pytest.mark.parametrize("part", [256, 512])
+@pytest.mark.parametrize("clear", [True, False])
+def test_overflowing_draw_shades_nothing(renderer_factory, clear, part):
+    r = renderer_factory()
+    r.set_tuning(rasterPartEntries=part)
+    W, H = 320, 201
+    small, si = _overlay()
+    large, li = _scene(np.random.default_rng(3), W, H, 5600)
+    r.set_target(W, H, 4)
+    _bind(r, W, H, 4, large, li)
+    r.draw()
+    want = r.color()
+    _bind(r, W, H, 4, small, si)
+    r.draw()
+    before = r.color()
+    _bind(r, W, H, 4, large, li)
+    r.set_tuning(binCapacity=4096)
+    print(f"[kept slots, overflow clear={clear} part={part}]", flush=True)
+    r.draw_async(clear=clear)
+    with pytest.raises(IfritError, match="binning buffers"):
+        r.synchronize()
+    assert np.array_equal(r.color(), before)
+    r.draw()  # the buffers have grown
+    assert np.array_equal(r.color(), want)
