@@ -807,7 +807,8 @@ bool TileRasterRenderer::prepare(int indexCount) {
                  recs_[1].ensure(slots * 16) && recs_[2].ensure(slots * 16) && recs_[3].ensure(slots * 16) &&
                  recs_[4].ensure(slots * 16) && recs_[5].ensure(slots * 16) && bary_.ensure(fans * 32) &&
                  binFront_.ensure(frontBytes()) && slotOf_.ensure((size_t)std::max(1, ntri) * 4 * nv) &&
-                 (!needSwapFlags() || swapped_.ensure(slots)) &&
+                 // a flag for every record that exists: a draw without clear also shades those it keeps
+                 (!needSwapFlags() || ensureZeroed(swapped_, std::max(slots, recs_[0].bytes / 16))) &&
                  clipList_.ensure((size_t)clipCap_ * 4 * nv) &&
                  statPart_.ensure((2 * (size_t)rasterGrid() + 2) * 8) &&
                  items_.ensure((size_t)itemCap_ * 16) && tilePartial_.ensure(tiles * 4) &&

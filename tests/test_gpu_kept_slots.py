@@ -145,3 +145,18 @@ def test_overflowing_draw_shades_nothing(renderer_factory, clear, part):
     assert np.array_equal(r.color(), before)
     r.draw()  # the buffers have grown
     assert np.array_equal(r.color(), want)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_cull_mode_with_swap_flags_after_a_large_draw(renderer_factory, mode):
+    s = scenes.config2(200, 150, 1, spheres=8, tex_size=64)
+    r = renderer_factory()
+    r.set_float_output(True)
+    r.load_scene(s)
+    r.draw()
+    before = r.color_f32()
+    r.set_cull_mode(mode)
+    r.num_indices = 6
+    print(f"[kept slots, cull mode {mode}]", flush=True)
+    r.draw(clear=False)  # behind the sphere's front
+    assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
