@@ -185,6 +185,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
             r.texPool_ = pool;
             r.ids_ = nullptr;
             r.keepSlots_ = true;
+            r.weightBase_ = 0;
         }
     } restore(*this, bufs);
 
@@ -242,6 +243,7 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
     // they are laid out
     const size_t weights = ((size_t)clipCap_ * 32 + 255) & ~(size_t)255;
     put(bary_, weights);
+    weightBase_ = (unsigned)ntri;  // no pixel is shaded that keeps an earlier draw's slot
     put(binFront_, std::max(frontBytes(), (size_t)nverts_ * 16 + slots * 48 + std::max<size_t>(1, groups) - weights));
     put(slotOf_, (size_t)std::max(1, ntri) * 4);
     if (needSwapFlags()) put(swapped_, slots);

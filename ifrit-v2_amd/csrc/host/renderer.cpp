@@ -797,15 +797,15 @@ bool TileRasterRenderer::prepare(int indexCount) {
     partialCap_ = std::max<unsigned>(partialCap_, std::max(256u, binCap_ / (8u * part)));
     // point and line records take one slot per index (3 per triangle)
     const size_t slots = std::max(((size_t)ntri + clipCap_) * nv, polygonMode_ != 0 ? (size_t)indexCount : 0);
-    // vertex weights: of the clip fans, or of every point and line
-    const size_t fans = std::max((size_t)clipCap_ * nv, polygonMode_ != 0 ? (size_t)indexCount : 0);
     const bool wantFloat = batch_.empty() && ((fb_ && !fb_->color.empty() && fb_->color[0]) || floatOut_ ||
                                               blend_.blendEnable);
     // clip positions are kept for the point and line modes only (a host vertex shader uploaded its own)
     bool okAll = (polygonMode_ == 0 || clip_.ensure((size_t)nverts_ * 16 * nv)) &&
                  recs_[0].ensure(slots * 16) &&
                  recs_[1].ensure(slots * 16) && recs_[2].ensure(slots * 16) && recs_[3].ensure(slots * 16) &&
-                 recs_[4].ensure(slots * 16) && recs_[5].ensure(slots * 16) && bary_.ensure(fans * 32) &&
+                 recs_[4].ensure(slots * 16) && recs_[5].ensure(slots * 16) &&
+                 // vertex weights for every record that exists: a draw without clear also shades those it keeps
+                 bary_.ensure(std::max(slots, recs_[0].bytes / 16) * 32) &&
                  binFront_.ensure(frontBytes()) && slotOf_.ensure((size_t)std::max(1, ntri) * 4 * nv) &&
                  // a flag for every record that exists: a draw without clear also shades those it keeps
                  (!needSwapFlags() || ensureZeroed(swapped_, std::max(slots, recs_[0].bytes / 16))) &&
@@ -1069,7 +1069,7 @@ ShadeParams TileRasterRenderer::shadeParams(bool writeFloat) const {
     std::memcpy(sh.lightColor, d.lightColor, sizeof(sh.lightColor));
     sh.writeFloat = writeFloat ? 1 : 0;
     sh.ntri = curTris_;
-    sh.fanCap = clipCap_;
+    sh.weightBase = weightBase_;
     sh.shadeTile = shadeTile_;
     sh.neural = neuralShadeParams();
     sh.swapped = needSwapFlags() ? swapped_.as<unsigned char>() : nullptr;
@@ -1127,6 +1127,7 @@ void TileRasterRenderer::enqueue(bool clear) {
     sp.swapped = needSwapFlags() ? swapped_.as<unsigned char>() : nullptr;
     sp.msaa = samples_ > 1 ? 1 : 0;
     sp.clipCap = clipCap_;
+    sp.weightBase = weightBase_;
     sp.invTileWidth = ifx::rcp_nr_ss(16.0f, rcpModel_);
     sp.rcpModel = rcpModel_;
     // triangle groups outside a view are skipped whole
@@ -1247,8 +1248,6 @@ void TileRasterRenderer::enqueuePolygons(bool clear, const Views& V) {
         const bool wantFloat = (fb_ && !fb_->color.empty() && fb_->color[0]) || floatOut_;
         ShadeParams sh = shadeParams(wantFloat);
         sh.ntri = 0;  // every record carries its own vertex weights (bx, by)
-        sh.fanCap = (unsigned)curIdx_;
-        sh.ownWeights = 1;
         sh.swapped = nullptr;
         sh.cleared = clear ? 1 : 0;
         launch_shade(sh, V, shadeOrder(false), recPtrs(), bary_.as<float4>(), visSlot_.as<uint32_t>(),

@@ -291,6 +291,7 @@ private:
     bool countersDirty_ = false;
     bool ensureZeroed(DevBuf& b, size_t n);
     DevBuf groupBounds_;             // per triangle group: bounds
+    unsigned weightBase_ = 0;        // the slot whose vertex weights bary_ starts with
     DevBuf swapped_;                 // per record slot: set up with vertices 0 and 2 exchanged
     DevBuf polyKeys_;                // point and line modes: per pixel the nearest candidate's key
     static constexpr int kBufferSlots = 64;

@@ -11,8 +11,8 @@
 //                                         transform in the geometry kernel)
 //   recs        TriRecs, N * SV slots     assembled triangles; in view v, slot v*SV + prim
 //                                         for unclipped triangles, v*SV + T + k for clip fans
-//   bary        float4[2 * N * clipCap]   vertex-weight bases bx, by of clip fans (shading only), or of
-//                                         every slot in the point and line modes
+//   bary        float4[2 * slots]         vertex-weight bases bx, by of the slots whose record says that it
+//                                         has its own (kOwnWeights): clip fans, points and lines (shading only)
 //   waves       WaveInfo[N][waves]        per 64 triangles, what the geometry kernel made of them
 //   entry       uint2, uint4[N][64 waves] per triangle, its bin entries or tile rectangle (WaveInfo)
 //   fanBox      uint2[N][clipCap]         tile rectangle of each clip fan
@@ -42,6 +42,10 @@ struct __align__(16) TriRec {
     float4 q0, q1, q2;
     float4 f1, f2, f3;
 };
+
+// The pixel box's high end of a record with vertex weights of its own (clip fans, which no box
+// bounds, points and lines): beyond every target, and no box of an unclipped triangle ends there.
+constexpr unsigned kOwnWeights = 0xfffeffffu;
 
 // Records are stored as six float4 streams (structure of arrays) so that a
 // wave's stores and the tile loader's gathers are 16-byte accesses.
@@ -137,6 +141,7 @@ struct SetupParams {
                              // up with its first and third vertex exchanged (null for back)
     int msaa;           // 1 disables the small-triangle cull
     unsigned clipCap;   // capacity for clip fan triangles and for triangles to clip
+    unsigned weightBase;  // the slot whose vertex weights `bary` starts with
     float invW, invH;   // 1 / width, 1 / height (TileRasterRenderer.cpp:59-60)
     float invTileWidth; // ApproxReciprocal(16.0f) (TileRasterWorker.cpp:499)
     int rcpModel;       // ifx::RcpModel: whose RCPPS the reciprocals of w and of the area reproduce
@@ -233,8 +238,7 @@ struct ShadeParams {
     float lightColor[4][4];
     int writeFloat;          // also write RGBA32F
     int ntri;                // view-local slots >= ntri are clip fans with their own bx, by
-    unsigned fanCap;         // fans per view that `bary` holds, or slots in the point and line modes
-    int ownWeights;          // point and line modes: every slot of the draw has its bx, by
+    unsigned weightBase;     // the slot whose weights `bary` starts with
     int shadeTile;           // side of a square of as many pixels as one wave shades (8, 16 or 32),
                              // its 8x8 sub-tiles in turn
     int cleared;             // the draw cleared its targets

@@ -45,9 +45,9 @@ __device__ __forceinline__ void store_record(TriRecs recs, float4* bary, unsigne
     recs.f1[slot] = f1;
     recs.f2[slot] = f2;
     recs.f3[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    recs.q2[slot] = make_float4(0.0f, __uint_as_float(key), 0.0f, 0.0f);
-    bary[2 * slot] = make_float4(bx[0], bx[1], bx[2], by[0]);
-    bary[2 * slot + 1] = make_float4(by[1], by[2], 0.0f, 0.0f);
+    recs.q2[slot] = make_float4(0.0f, __uint_as_float(key), 0.0f, __uint_as_float(kOwnWeights));
+    bary[2 * (size_t)slot] = make_float4(bx[0], bx[1], bx[2], by[0]);
+    bary[2 * (size_t)slot + 1] = make_float4(by[1], by[2], 0.0f, 0.0f);
 }
 
 // The workgroup's candidate count into the raster partials and its accepted

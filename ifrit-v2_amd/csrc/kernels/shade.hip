@@ -35,43 +35,25 @@ struct ShadeTri {
     int swapped;  // set up with its first and third vertex exchanged (cull modes none and front)
 };
 
-// Vertex weights of the clip fans.  A view's capacity of fans follows the previous view's; in the
-// point and line modes (one view, ntri = 0) every slot of the draw has its own.
-struct FanWeights {
-    const float4* bary;
-    const ViewCounters* ctr;
-    unsigned view;
-};
-
-// How many slots from fanStart on have them.  Pixels that a draw without clear leaves alone keep the
-// slots of earlier draws, which may lie far beyond.
-__device__ __forceinline__ unsigned fan_count(const ShadeParams& P, const FanWeights& F) {
-    return P.ownWeights ? P.fanCap : min(dev::uniform_word(&F.ctr[F.view].fans), P.fanCap);
-}
-
-// The weight bases of a slot's triangle: a fan's own, else (0, 0, 1) and (1, 0, 0) as unclipped
-// triangles have them (TileRasterWorker.cpp:711-712).
-__device__ __forceinline__ void set_weights(const ShadeParams& P, const FanWeights& F, unsigned fanStart, unsigned slot,
-                                            ShadeTri& T) {
-    const unsigned f = slot - fanStart;
-    T.bx[0] = 0.0f; T.bx[1] = 0.0f; T.bx[2] = 1.0f;
-    T.by[0] = 1.0f; T.by[1] = 0.0f; T.by[2] = 0.0f;
-    if (f < fan_count(P, F)) {
-        const float4* const w = F.bary + 2 * ((size_t)F.view * P.fanCap + f);
-        const float4 a = w[0], b = w[1];
-        T.bx[0] = a.x; T.bx[1] = a.y; T.bx[2] = a.z;
-        T.by[0] = a.w; T.by[1] = b.x; T.by[2] = b.y;
-    }
+// The weight bases of a slot's triangle, whose record ends in box `hi`: its own where the record
+// says so, else (0, 0, 1) and (1, 0, 0) as unclipped triangles have them
+// (TileRasterWorker.cpp:711-712).
+__device__ __forceinline__ void set_weights(float hi, const float4& a, const float4& b, ShadeTri& T) {
+    const bool own = __float_as_uint(hi) == kOwnWeights;
+    T.bx[0] = own ? a.x : 0.0f; T.bx[1] = own ? a.y : 0.0f; T.bx[2] = own ? a.z : 1.0f;
+    T.by[0] = own ? a.w : 1.0f; T.by[1] = own ? b.x : 0.0f; T.by[2] = own ? b.y : 0.0f;
 }
 
 // The ntri slots below fanStart (the view's first clip fan slot) are the
 // unclipped triangles, triangle p in slot fanStart - ntri + p: their
 // primitive comes from the slot itself, so the vertex indices can be read in
-// the same round trip as the record.  Any other slot, a fan's or one that an
-// earlier draw left, reads its key first.  The
+// the same round trip as the record.  Any other slot is a fan's, or one that an
+// earlier draw left (a draw without clear shades the pixels that it leaves alone
+// too): it reads its key first, and its weights with it, which exist for every slot
+// that a pixel can hold.  The
 // record's planes are read last: a load still in flight when the two kinds
 // of slot rejoin would otherwise be waited for there.
-__device__ __forceinline__ void load_shade_tri(const ShadeParams& P, const TriRecs& recs, const FanWeights& F,
+__device__ __forceinline__ void load_shade_tri(const ShadeParams& P, const TriRecs& recs, const float4* bary,
                                                unsigned fanStart, unsigned slot, ShadeTri& T) {
     const unsigned ntri = (unsigned)P.ntri, p = slot - (fanStart - ntri);
     if (p < ntri) {
@@ -79,8 +61,10 @@ __device__ __forceinline__ void load_shade_tri(const ShadeParams& P, const TriRe
         T.bx[0] = 0.0f; T.bx[1] = 0.0f; T.bx[2] = 1.0f;
         T.by[0] = 1.0f; T.by[1] = 0.0f; T.by[2] = 0.0f;
     } else {
-        T.prim = (int)(__float_as_uint(recs.q2[slot].y) >> 2);
-        set_weights(P, F, fanStart, slot, T);
+        const float4* const w = bary + 2 * (size_t)(slot - P.weightBase);
+        const float4 q2 = recs.q2[slot], a = w[0], b = w[1];
+        T.prim = (int)(__float_as_uint(q2.y) >> 2);
+        set_weights(q2.w, a, b, T);
     }
     T.swapped = P.swapped ? P.swapped[slot] : 0;
     T.f1 = recs.f1[slot];
@@ -88,11 +72,16 @@ __device__ __forceinline__ void load_shade_tri(const ShadeParams& P, const TriRe
     T.f3 = recs.f3[slot];
 }
 
-// load_shade_tri for a record at hand: the primitive comes from its key.
-__device__ __forceinline__ void record_shade_tri(const ShadeParams& P, const TriRec& R, const FanWeights& F,
+// load_shade_tri for a record of the draw at hand: the primitive comes from its key.
+__device__ __forceinline__ void record_shade_tri(const ShadeParams& P, const TriRec& R, const float4* bary,
                                                  unsigned fanStart, unsigned slot, ShadeTri& T) {
     T.prim = (int)(__float_as_uint(R.q2.y) >> 2);
-    set_weights(P, F, fanStart, slot, T);
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+    if (slot >= fanStart) {
+        a = bary[2 * (size_t)(slot - P.weightBase)];
+        b = bary[2 * (size_t)(slot - P.weightBase) + 1];
+    }
+    set_weights(R.q2.w, a, b, T);
     T.swapped = P.swapped ? P.swapped[slot] : 0;
     T.f1 = R.f1;
     T.f2 = R.f2;
@@ -651,7 +640,7 @@ constexpr int kTapWindow = 128;
 template <int S, bool NEURAL, bool FP8, bool LAYERED, bool GENERIC = false>
 __device__ __forceinline__ void shade_subtile(const ShadeParams& P, float3 cam, int width, int height,
                                               unsigned fanStart, int ox, int oy, size_t pixBase, const TriRecs& recs,
-                                              const FanWeights& fans, const uint32_t* __restrict__ visSlot,
+                                              const float4* __restrict__ bary, const uint32_t* __restrict__ visSlot,
                                               const float* __restrict__ vtx, const int* __restrict__ idx,
                                               const TexDesc* __restrict__ tex, const uint8_t* __restrict__ pool,
                                               uchar4* __restrict__ rgba8, float4* __restrict__ rgba32f) {
@@ -760,7 +749,7 @@ __device__ __forceinline__ void shade_subtile(const ShadeParams& P, float3 cam, 
             const unsigned slot = fSlot[fi];
             const int fl = fPix[fi];
             ShadeTri T;
-            load_shade_tri(P, recs, fans, fanStart, slot, T);
+            load_shade_tri(P, recs, bary, fanStart, slot, T);
             const int qx = ox + (fl & 7), qy = oy + (fl >> 3);
             R = prep_fragment(P, cam, T, vtx, idx, tex, pool, qx, qy, o, NEURAL || LAYERED, GENERIC);
             if (R.mat >= 0) {
@@ -1017,14 +1006,13 @@ __device__ __forceinline__ void shade_tiles(const ShadeParams& P, const Views& V
             shade_empty<S, LAYERED>(P, width, height, tx, ty, pb, rgba8, rgba32f);
             continue;
         }
-        const FanWeights fans{bary, V.ctr, view};
         const float3 cam = make_float3(D.camera[0], D.camera[1], D.camera[2]);
         const unsigned fanStart = D.slotBase + (unsigned)P.ntri;
 #pragma unroll 1
         for (unsigned k = N == 1 ? index & 3u : 0u; k < 4u; k += N == 1 ? 4u : 1u) {
             const int ox = tx + (int)(k & 1u) * 8, oy = ty + (int)(k >> 1) * 8;
             if (ox >= width || oy >= height) continue;
-            shade_subtile<S, NEURAL, FP8, LAYERED, GENERIC>(P, cam, width, height, fanStart, ox, oy, pb, recs, fans,
+            shade_subtile<S, NEURAL, FP8, LAYERED, GENERIC>(P, cam, width, height, fanStart, ox, oy, pb, recs, bary,
                                                             visSlot + pb * S, vtx, idx, tex, pool, rgba8 + pb,
                                                             rgba32f ? rgba32f + pb : nullptr);
         }
@@ -1125,7 +1113,6 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
     while (order.next(q, bins, tiles, &sItem, tile, start, cnt)) {
         const dev::UniformView& D = dev::uniform_view(V.desc + dev::uniform_view_of(V.tileView, (unsigned)tile));
         const rc::ViewGeom G = rc::view_of_tile(V, tile);
-        const FanWeights fans{bary, V.ctr, (unsigned)G.view};
         const rc::PixelCtx C = rc::pixel_ctx(G, rc::quarter_x(t), rc::quarter_y(t));
         const size_t pix = G.pixBase + C.pix;
         const float3 cam = make_float3(D.camera[0], D.camera[1], D.camera[2]);
@@ -1154,7 +1141,7 @@ __global__ void __launch_bounds__(256) k_blend_ordered(ShadeParams P, BlendCoefs
                     src = make_float4(sat(f.x), sat(f.y), sat(f.z), f.w);
                 } else {
                     ShadeTri T;
-                    record_shade_tri(P, R, fans, fanStart, sl, T);
+                    record_shade_tri(P, R, bary, fanStart, sl, T);
                     src = shade_fragment(P, cam, T, vtx, idx, tex, pool, C.px, C.py);
                 }
                 col = blend_pixel(B, src, col);

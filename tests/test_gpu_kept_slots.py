@@ -160,3 +160,20 @@ def test_cull_mode_with_swap_flags_after_a_large_draw(renderer_factory, mode):
     print(f"[kept slots, cull mode {mode}]", flush=True)
     r.draw(clear=False)  # behind the sphere's front
     assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
+
+
+@pytest.mark.parametrize("samples", [1, 4])
+def test_clip_fans_of_a_large_draw(renderer_factory, samples):
+    """The ground crosses w = 0: its pixels keep fans, whose weights the next draw must not lose."""
+    s = scenes.config1(200, 150)
+    s.samples = samples
+    r = renderer_factory()
+    r.set_float_output(True)
+    r.load_scene(s)
+    assert r.draw()["clippedTriangles"] > 0
+    assert (r.visibility()[0] == s.num_triangles - 1).sum() > 1000
+    before = r.color_f32()
+    r.num_indices = 6
+    print(f"[kept slots, fans s={samples}]", flush=True)
+    assert r.draw(clear=False)["clippedTriangles"] == 0
+    assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
