@@ -543,7 +543,8 @@ __device__ __forceinline__ void for_each_ordered(const TriRecs& recs, const unsi
                 const int x0 = max((int)(lo & 0xFFFFu) - tx0, 0), y0 = max((int)(lo >> 16) - ty0, 8 * half);
                 const int x1 = min((int)(hi & 0xFFFFu) - tx0, 15), y1 = min((int)(hi >> 16) - ty0, 8 * half + 7);
                 if (!full && x0 <= x1 && y0 <= y1) {
-                    const bool one = x1 - x0 < 4 && y1 - y0 < 4;  // a window off the blocks' grid
+                    // one window, on the blocks' grid or off it: off it, every block lacks a pixel
+                    const bool one = x1 - x0 < 4 && y1 - y0 < 4;
                     const int gx = one ? x0 : x0 & ~3, gy = one ? y0 : y0 & ~3;
                     const int wcols = (x1 - gx + 4) >> 2, n = wcols * ((y1 - gy + 4) >> 2);
                     big = n > 4;
@@ -556,7 +557,7 @@ __device__ __forceinline__ void for_each_ordered(const TriRecs& recs, const unsi
                             unsigned pm = block_fb_mask(x1 + 1 - wx, y1 + 1 - wy), groups = 0, quads = 0;
                             bool acc = false;
                             if constexpr (S == 1) {
-                                if (!one) acc = block_accepted(E, fx, fy);
+                                if (((wx | wy) & 3) == 0) acc = block_accepted(E, fx, fy);
                                 const unsigned in = window_inside(E, fx, fy);
                                 window_classes(in, wx, wy, groups, quads);
                                 pm &= in;
