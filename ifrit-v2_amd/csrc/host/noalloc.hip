@@ -150,6 +150,9 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
         FrameBuffer* fb;
         bool floatOut;
         uint8_t* pool;
+        // the counters of the draw before, which may not have been asked for yet, once it has ended
+        bool ended = false, pending = false;
+        HostCounters counters;
         Restore(TileRasterRenderer& rr, DevBuf* const* b) : r(rr), bufs(b) {
             for (size_t i = 0; i < kBufs; i++) saved[i] = *bufs[i];
             const unsigned c[5] = {r.clipCap_, r.binCap_, r.bigCap_, r.itemCap_, r.partialCap_};
@@ -186,6 +189,10 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
             r.ids_ = nullptr;
             r.keepSlots_ = true;
             r.weightBase_ = 0;
+            if (ended) {
+                *r.hostCtr_ = counters;
+                r.reducePending_ = pending;
+            }
         }
     } restore(*this, bufs);
 
@@ -277,6 +284,9 @@ void TileRasterRenderer::drawNoAlloc(const IfritNoAllocDraw& d) {
 
     // tables: the view, its tile maps (all view 0), the texture descriptors
     if (!ok(hipStreamSynchronize(stream_), "iftrDrawNoAlloc")) return;
+    restore.counters = *hostCtr_;
+    restore.pending = reducePending_;
+    restore.ended = true;
     std::vector<TexDesc> td(std::max<size_t>(1, textures_.size()));
     texPool_ = nullptr;
     for (const TextureSlot& t : textures_)
