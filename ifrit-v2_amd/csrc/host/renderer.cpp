@@ -1070,6 +1070,9 @@ ShadeParams TileRasterRenderer::shadeParams(bool writeFloat) const {
     sh.writeFloat = writeFloat ? 1 : 0;
     sh.ntri = curTris_;
     sh.weightBase = weightBase_;
+    auto last = [](size_t room) { return (unsigned)std::min<size_t>(std::max<size_t>(room, 1) - 1, 0x7fffffffu); };
+    sh.lastTri = last(idx_.bytes / 12);
+    sh.lastVertex = last(vtx_.bytes / ((size_t)std::max(stride_, 1) * 4));
     sh.shadeTile = shadeTile_;
     sh.neural = neuralShadeParams();
     sh.swapped = needSwapFlags() ? swapped_.as<unsigned char>() : nullptr;

@@ -239,6 +239,7 @@ struct ShadeParams {
     int writeFloat;          // also write RGBA32F
     int ntri;                // view-local slots >= ntri are clip fans with their own bx, by
     unsigned weightBase;     // the slot whose weights `bary` starts with
+    unsigned lastTri, lastVertex;  // the last ones that the index and vertex buffers have room for
     int shadeTile;           // side of a square of as many pixels as one wave shades (8, 16 or 32),
                              // its 8x8 sub-tiles in turn
     int cleared;             // the draw cleared its targets

@@ -452,7 +452,10 @@ __device__ FragPrep prep_fragment(const ShadeParams& P, float3 cam, const ShadeT
     // the planes weigh the vertices in the order setup took them: exchanged triangles
     // take their first and third vertex the other way round (chosen after the loads, so
     // that the index loads need not wait for the flag)
-    const int i0 = idx[3 * T.prim], i1 = idx[3 * T.prim + 1], i2 = idx[3 * T.prim + 2];
+    // a triangle that an earlier draw left may lie beyond this one's buffers
+    const int* const tri = idx + 3 * (size_t)min((unsigned)T.prim, P.lastTri);
+    const unsigned i0 = min((unsigned)tri[0], P.lastVertex), i1 = min((unsigned)tri[1], P.lastVertex),
+                   i2 = min((unsigned)tri[2], P.lastVertex);
     const float* v0 = vtx + (size_t)(T.swapped ? i2 : i0) * P.stride;
     const float* v1 = vtx + (size_t)i1 * P.stride;
     const float* v2 = vtx + (size_t)(T.swapped ? i0 : i2) * P.stride;

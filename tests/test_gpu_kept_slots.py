@@ -177,3 +177,41 @@ def test_clip_fans_of_a_large_draw(renderer_factory, samples):
     print(f"[kept slots, fans s={samples}]", flush=True)
     assert r.draw(clear=False)["clippedTriangles"] == 0
     assert np.array_equal(r.color_f32().view(np.uint32), before.view(np.uint32))
+
+
+@pytest.mark.parametrize("large", ["meshlets", "short records"])
+def test_small_buffers_after_a_large_draw(renderer_factory, large):
+    """Kept triangles and vertices beyond the second draw's buffers: their colour is of no use, but
+    the second draw's own pixels are as when it draws alone."""
+    s = scenes.config2(200, 150, 1, spheres=8, tex_size=64)
+    clip, oi = _overlay()
+    over = np.random.default_rng(1).uniform(0.1, 0.9, (6, 8 if large == "meshlets" else 256)).astype(np.float32)
+    over[:, :4] = clip
+    small = scenes.Scene("t", 200, 150, 1, over, oi, EYE, program=s.program, sampler=s.sampler, lights=s.lights,
+                         textures=s.textures)
+    r = renderer_factory()
+    r.set_float_output(True)
+    if large == "meshlets":
+        recs, loc, vo, io, _ = scenes.build_meshlets(s.vertices, s.indices)
+        r.set_target(200, 150, 1)
+        for t in s.textures:
+            r.add_texture(t)
+        r.bind_fragment_program(small)
+        for slot, a in enumerate((recs, loc, vo, io)):
+            r.create_buffer(slot, a)
+        r.bind_meshlets(s.mvp, recs.shape[1])
+        r.bind_geometry(over, oi, EYE, clip_passthrough=True)
+        r.draw_mesh_tasks(len(vo) - 1)
+    else:
+        r.load_scene(s)
+        r.draw()
+        r.bind_geometry(over, oi, EYE, clip_passthrough=True)
+        r.bind_fragment_program(small)
+    assert (r.visibility()[0] != 0xFFFFFFFF).sum() > 1000
+    print(f"[kept slots, small buffers after {large}]", flush=True)
+    r.draw(clear=False)
+    got = r.color_f32().reshape(-1, 4)
+    r.draw()
+    own = r.visibility()[0] != 0xFFFFFFFF
+    assert 1000 < own.sum() < own.size
+    assert np.array_equal(got[own].view(np.uint32), r.color_f32().reshape(-1, 4)[own].view(np.uint32))
