@@ -51,11 +51,11 @@ void DevBuf::release() {
     bytes = 0;
 }
 
-bool TileRasterRenderer::ensureZeroed(DevBuf& b, size_t n) {
+bool TileRasterRenderer::ensureFilled(DevBuf& b, size_t n, int byte) {
     const void* had = b.ptr;
     const size_t bytes = b.bytes;
     if (!b.ensure(n)) return false;
-    return (b.ptr == had && b.bytes == bytes) || hipMemsetAsync(b.ptr, 0, b.bytes, stream_) == hipSuccess;
+    return (b.ptr == had && b.bytes == bytes) || hipMemsetAsync(b.ptr, byte, b.bytes, stream_) == hipSuccess;
 }
 
 TileRasterRenderer::TileRasterRenderer() {}
@@ -815,7 +815,9 @@ bool TileRasterRenderer::prepare(int indexCount) {
                  multiList_.ensure(tiles * 4) && order_.ensure(tiles * 8) && partials_.ensure((size_t)partialCap_ * 256 * samples_ * 8) &&
                  ensureZeroed(binCount_, tiles * 8) && binStart_.ensure(tiles * 4) && binCursor_.ensure(tiles * 4) &&
                  binList_.ensure((size_t)binCap_ * 4) &&
-                 visId_.ensure(ps * 4) && visDepth_.ensure(ps * 4) && visSlot_.ensure(ps * 4) &&
+                 visId_.ensure(ps * 4) && visDepth_.ensure(ps * 4) &&
+                 // samples that no draw has written hold no slot
+                 ensureFilled(visSlot_, ps * 4, 0xff) &&
                  visClass_.ensure(px) && rgba8_.ensure(px * 4) && (!wantFloat || rgba32f_.ensure(px * 16)) &&
                  (polygonMode_ == 0 || polyKeys_.ensure(px * 8));
     if (!okAll) {

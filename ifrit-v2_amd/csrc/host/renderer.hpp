@@ -289,7 +289,8 @@ private:
     // the tile counts and live counters, zero between draws (the tile plan leaves them so), were
     // left behind by a draw that failed to launch
     bool countersDirty_ = false;
-    bool ensureZeroed(DevBuf& b, size_t n);
+    bool ensureFilled(DevBuf& b, size_t n, int byte);  // fills what it newly allocates
+    bool ensureZeroed(DevBuf& b, size_t n) { return ensureFilled(b, n, 0); }
     DevBuf groupBounds_;             // per triangle group: bounds
     unsigned weightBase_ = 0;        // the slot whose vertex weights bary_ starts with
     DevBuf swapped_;                 // per record slot: set up with vertices 0 and 2 exchanged

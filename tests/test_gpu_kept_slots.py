@@ -215,3 +215,22 @@ def test_small_buffers_after_a_large_draw(renderer_factory, large):
     own = r.visibility()[0] != 0xFFFFFFFF
     assert 1000 < own.sum() < own.size
     assert np.array_equal(got[own].view(np.uint32), r.color_f32().reshape(-1, 4)[own].view(np.uint32))
+
+
+@pytest.mark.parametrize("samples", [1, 4, 8])
+def test_pixels_no_draw_has_written(renderer_factory, samples):
+    """The first draw of a renderer, and one into a larger target, under a scissor."""
+    r = renderer_factory()
+    clip, idx = _overlay()
+    for W, H in [(64, 33), (321, 200)]:
+        r.set_target(W, H, samples)
+        _bind(r, W, H, samples, clip, idx)
+        r.set_scissors([(5.0, 3.0, 31.0, 20.0)])
+        print(f"[no draw yet s={samples} {W}x{H}]", flush=True)
+        r.draw()
+        f = O.Frame().render(W, H, samples, clip, idx)
+        y, x = np.mgrid[:H, :W]
+        inside = np.repeat(((x >= 5) & (x <= 36) & (y >= 3) & (y <= 23)).reshape(-1), samples)
+        ids = r.visibility()[0]
+        assert (ids[~inside] == 0xFFFFFFFF).all()
+        assert np.array_equal(ids[inside], f.ids[inside])
