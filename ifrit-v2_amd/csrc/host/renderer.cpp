@@ -1276,7 +1276,7 @@ std::vector<uint8_t> TileRasterRenderer::graphKey(bool clear) const {
                         nnFallback_[1] ? 1 : 0, (int)textures_.size(), stageTiming_ ? 1 : 0,
                         fb_ && !fb_->color.empty() && fb_->color[0] ? 1 : 0, batch_.empty() ? 1 : 0,
                         floatOut_ ? 1 : 0, blend_.blendEnable ? 1 : 0, cullMode_, deterministic_ ? 1 : 0,
-                        polygonMode_, curIdx_, clipAt_, rcpModel_};
+                        polygonMode_, curIdx_, clipAt_, rcpModel_, tileThreads_};
     put(ints, sizeof(ints));
     // emitted lists swap buffers without reallocating them
     const void* inputs[] = {vtx_.ptr, idx_.ptr};
