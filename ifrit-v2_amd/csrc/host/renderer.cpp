@@ -35,7 +35,8 @@ bool DevBuf::ensure(size_t n) {
     if (n <= bytes && ptr) return true;
     release();
     generation++;
-    size_t cap = std::max<size_t>(n, 256);
+    // whole 16-byte words: the kernels read some maps of two-byte entries by words
+    size_t cap = std::max<size_t>((n + 15) & ~(size_t)15, 256);
     if (hipMalloc(&ptr, cap) != hipSuccess) {
         ptr = nullptr;
         bytes = 0;
