@@ -1158,7 +1158,7 @@ void TileRasterRenderer::enqueue(bool clear) {
     bp.clipCap = clipCap_;
     bp.binCap = binCap_;
     bp.bigCap = bigCap_;
-    launch_bin(bp, V, recPtrs(), bins, q, statPtrs(), ctr_.as<DeviceCounters>(), s);
+    launch_bin(bp, V, recPtrs(), bins, q, ctr_.as<DeviceCounters>(), s);
     mark(3);
     RasterParams rp{};
     rp.depthFunc = depthFunc_;

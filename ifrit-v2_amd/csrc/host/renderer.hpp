@@ -262,7 +262,7 @@ private:
     };
     std::vector<HostView> batch_;
     std::vector<ViewDesc> viewDesc_;        // device table as last uploaded
-    std::vector<int> viewLayout_;           // (width, height, shade) per view + shading tile
+    std::vector<int> viewLayout_;           // (width, height, shade) per view
     unsigned totalTiles_ = 0, shadeTiles_ = 0;
     size_t totalPixels_ = 0;
     HostCounters* hostCtr_ = nullptr;  // pinned: the last finished draw's counters

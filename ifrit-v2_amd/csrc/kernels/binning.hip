@@ -202,7 +202,7 @@ __device__ __forceinline__ Region next_region(const WaveInfo& W, unsigned long l
 //
 // Bound by the latency of the entries, the list starts and the scattered stores.
 __global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs recs, BinBufs B, RasterQueue q,
-                                                 StatPartials st, DeviceCounters* ctr) {
+                                                 DeviceCounters* ctr) {
     __shared__ unsigned sMade[4];
     const int lane = dev::lane_id();
     const unsigned gw = blockIdx.x * 4u + (threadIdx.x >> 6), G = gridDim.x * 4u;
@@ -294,10 +294,10 @@ __global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs r
 }  // namespace
 
 void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
-                StatPartials st, DeviceCounters* ctr, hipStream_t s) {
+                DeviceCounters* ctr, hipStream_t s) {
     hipLaunchKernelGGL(k_plan, dim3((p.tiles + kPlanTiles - 1) / kPlanTiles), dim3(kPlanTiles), 0, s,
                        reinterpret_cast<uint2*>(bins.cnt), bins.start, bins.cursor, p.tiles, views, q, ctr);
-    hipLaunchKernelGGL(k_scatter, dim3(p.grid), dim3(256), 0, s, p, views, recs, bins, q, st, ctr);
+    hipLaunchKernelGGL(k_scatter, dim3(p.grid), dim3(256), 0, s, p, views, recs, bins, q, ctr);
 }
 
 }  // namespace ifrit_hip

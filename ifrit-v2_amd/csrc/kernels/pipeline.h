@@ -378,7 +378,7 @@ void launch_geometry(const SetupParams& p, const Views& views, const VertexInput
 void launch_finalize(StatPartials st, const Views& views, DeviceCounters* ctr, HostCounters* out, hipStream_t s);
 // The tile plan and the scatter into the tile lists.
 void launch_bin(const BinParams& p, const Views& views, TriRecs recs, const BinBufs& bins, const RasterQueue& q,
-                StatPartials st, DeviceCounters* ctr, hipStream_t s);
+                DeviceCounters* ctr, hipStream_t s);
 void launch_raster(const RasterParams& p, const Views& views, int samples, TriRecs recs, const unsigned* slotOf,
                    const BinBufs& bins, const RasterQueue& q, int tiles, float* visDepth, uint32_t* visSlot,
                    uint8_t* visClass, StatPartials st, DeviceCounters* ctr, hipStream_t s);

@@ -420,8 +420,6 @@ __device__ __forceinline__ float3 ggx_light(float3 n, float3 V, float3 L, float4
     return make_float3((alb.x * diff + spec) * ndl, (alb.y * diff + spec) * ndl, (alb.z * diff + spec) * ndl);
 }
 
-// frame = false for callers that never run the programs from 3 on (layered GGX
-// and the neural material): their shading-frame paths then fold away.
 // Flat colour: bytes 0-2 of a hash of the primitive; the translucent flat colour also
 // takes alpha = (64 + (byte 3 & 127)) / 255.
 __device__ __forceinline__ float4 flat_color(int program, int prim) {
@@ -431,6 +429,8 @@ __device__ __forceinline__ float4 flat_color(int program, int prim) {
                        program == 6 ? (float)(64u + ((h >> 24) & 0x7fu)) * (1.0f / 255.0f) : 1.0f);
 }
 
+// frame = false for callers that never run the programs from 3 on (layered GGX
+// and the neural material): their shading-frame paths then fold away.
 __device__ FragPrep prep_fragment(const ShadeParams& P, float3 cam, const ShadeTri& T, const float* vtx,
                                   const int* idx, const TexDesc* tex, const uint8_t* pool, int px, int py, float o,
                                   bool frame, bool generic = false) {

@@ -519,8 +519,8 @@ uint64_t iftrGetDigest(IfritRendererHandle* h);
    iftrDrawLegacy for the bound single target (iftrSetRenderTarget or iftrBindFrameBuffer size,
    MSAA sample count, GPU vertex and fragment programs, textures, depth function), from the
    caller's device-resident vertices and indices into the caller's device outputs.  It calls no
-   hipMalloc or hipFree: every intermediate buffer (clip positions, triangle records, bins, raster
-   queue, counters, the per-sample record slots) is carved out of one static device array of
+   hipMalloc or hipFree: every intermediate buffer (triangle records, bins, raster queue, counters,
+   the per-sample record slots) is carved out of one static device array of
    IFHIP_NOALLOC_SCRATCH_BYTES per GPU, which the library holds from iftrInit until the process
    ends.  A draw whose buffers do not fit is refused with an error (iftrGetLastError) before any
    launch; 1920x1080 at 1 sample with 128K triangles, or 1024x1024 at 4 samples with 64K
