@@ -353,9 +353,11 @@ struct RasterQueue {
 //
 // List lengths order the work only where a pixel can hold many triangles; at one
 // sample it holds one and its cost is its texture taps, and the neighbours that no
-// longer follow each other cost the caches.  By length or not, in us: 8 samples,
-// 1920x1080: 107 or 118; 4 samples, 1009x767: 31 or 30; 1 sample: 92 or 92 (layered),
-// 73 or 72 (neural), 34 views 109 or 103.
+// longer follow each other cost the caches.  By length or not, in us, for 1.3M
+// triangles at 1920x1080, the same at 640x480, 4.2M half-pixel ones, and 82k at 1280x720:
+// 8 samples 107 or 114, 59 or 64, 36 or 40, 41 or 42; 4 samples 81 or 84, 41 or 42, 27 or
+// 28, 29 or 29; 1 sample 55 or 54, 24 or 24, 25 or 25, 18 or 18, and 34 views 109 or 103.
+// The gain follows the length of the lists; at 4 samples the line leaves some of it.
 struct ShadeOrder {
     const unsigned *a, *b;
     const uint4* count;
