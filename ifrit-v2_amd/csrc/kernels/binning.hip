@@ -261,7 +261,7 @@ __global__ void __launch_bounds__(256) k_scatter(BinParams P, Views V, TriRecs r
     const unsigned per = max(1u, G / (unsigned)V.count);
     for (unsigned k = gw; k < per * (unsigned)V.count; k += G) {
         const unsigned v = k / per;
-        const unsigned n = min(V.ctr[v].fans, P.clipCap), each = min(64u, (n + per - 1u) / per);
+        const unsigned n = fan_extent(V.ctr[v].clipIn, V.ctr[v].fans, P.clipCap), each = min(64u, (n + per - 1u) / per);
         for (unsigned i0 = (k % per) * each; i0 < n; i0 += per * each) {
             const ViewDesc& D = V.desc[v];
             const unsigned i = i0 + (unsigned)lane, slot = D.slotBase + (unsigned)P.ntri + i;

@@ -73,9 +73,9 @@ struct ViewDesc {
 // the tile plan moves them to the last two, which later kernels read, and
 // leaves zeros for the next draw.
 struct ViewCounters {
-    unsigned fanLive;   // clip fan slots taken so far
+    unsigned fanLive;   // clip fans so far
     unsigned clipLive;  // triangles found to cross w = 0 so far
-    unsigned fans;      // clip fan slots of the draw
+    unsigned fans;      // clip fans of the draw
     unsigned clipIn;    // triangles of the draw crossing w = 0
     unsigned pad[28];
 };
@@ -173,6 +173,21 @@ struct BinBufs {
 };
 // The scatter's workgroups add to as many sums as spread their atomics, a 128-byte line each.
 constexpr int kMadeSums = 64, kMadeStride = 16;
+
+// Slots of the clip fans.  Where a view has few triangles to clip, each takes as many slots as it can
+// have fans, in the order of the triangles, so that the same triangles leave their fans in the same
+// slots: a pixel that a later draw without clear leaves alone keeps its slot.  Ranking one
+// against all others costs n^2 / 64 comparisons a view; above kClipRanked, or where the capacity is
+// short, the fans take slots as they come.
+constexpr unsigned kFanSlots = 3;  // at most three vertices kept and two made, for edges that change sign
+constexpr unsigned kClipRanked = 4096;
+__host__ __device__ inline bool clips_ranked(unsigned clips, unsigned clipCap) {
+    return clips <= kClipRanked && kFanSlots * clips <= clipCap;
+}
+// Clip slots of a view that may hold a fan.
+__host__ __device__ inline unsigned fan_extent(unsigned clips, unsigned fans, unsigned clipCap) {
+    return clips_ranked(clips, clipCap) ? kFanSlots * clips : fans < clipCap ? fans : clipCap;
+}
 
 // Triangles per culling group (one workgroup of the geometry kernel).
 constexpr int kGroupTris = kGeomBlock;

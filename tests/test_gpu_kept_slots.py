@@ -234,3 +234,32 @@ def test_pixels_no_draw_has_written(renderer_factory, samples):
         ids = r.visibility()[0]
         assert (ids[~inside] == 0xFFFFFFFF).all()
         assert np.array_equal(ids[inside], f.ids[inside])
+
+
+@pytest.mark.parametrize("samples", [1, 4])
+@pytest.mark.parametrize("n", [1, 63, 130, 1365])
+def test_same_fans_keep_their_slots(renderer_factory, n, samples):
+    """n triangles across w = 0 among as many others, drawn again without clear: nothing passes, and
+    primitive IDs and colours must not change (1365: as many as the smallest capacity ranks)."""
+    rng = np.random.default_rng(n)
+    W, H = 200, 150
+    xyz = np.concatenate([rng.uniform(-1, 1, (2 * n, 3, 2)), rng.uniform(0.2, 0.8, (2 * n, 3, 1))], -1)
+    w = rng.uniform(0.5, 2.0, (2 * n, 3, 1))
+    w[::2, 0] *= -1.0  # one corner of every other one behind the eye
+    v = np.concatenate([xyz * np.abs(w), w, rng.uniform(-1, 1, (2 * n, 3, 8))], -1).reshape(-1, 12).astype(np.float32)
+    i = np.arange(6 * n, dtype=np.int32).reshape(-1, 3)
+    idx = np.ascontiguousarray(np.where(rng.random((2 * n, 1)) < 0.5, i, i[:, ::-1])).reshape(-1)
+    r = renderer_factory()
+    r.set_float_output(True)
+    r.set_cull_mode(0)
+    r.set_target(W, H, samples)
+    r.bind_geometry(v, idx, EYE, clip_passthrough=True)
+    r.bind_fragment_program(scenes.Scene("t", W, H, samples, v, idx, EYE, program=scenes.PROGRAM_NORMAL_LAMBERT,
+                                         lights=[((0.3, 0.5, 0.8, 0.0), (1.0, 0.9, 0.8, 0.0))]))
+    assert r.draw()["clippedTriangles"] >= n
+    ids, color = r.visibility()[0], r.color_f32()
+    for k in range(3):
+        print(f"[kept slots, same fans n={n} s={samples} {k}]", flush=True)
+        r.draw(clear=False)
+        assert np.array_equal(r.visibility()[0], ids)
+        assert np.array_equal(r.color_f32().view(np.uint32), color.view(np.uint32))
