@@ -817,10 +817,10 @@ bool TileRasterRenderer::prepare(int indexCount) {
                  ensureZeroed(binCount_, tiles * 8) && binStart_.ensure(tiles * 4) && binCursor_.ensure(tiles * 4) &&
                  binList_.ensure((size_t)binCap_ * 4) &&
                  visId_.ensure(ps * 4) && visDepth_.ensure(ps * 4) &&
-                 // samples that no draw has written hold no slot
-                 ensureFilled(visSlot_, ps * 4, 0xff) &&
                  visClass_.ensure(px) && rgba8_.ensure(px * 4) && (!wantFloat || rgba32f_.ensure(px * 16)) &&
-                 (polygonMode_ == 0 || polyKeys_.ensure(px * 8));
+                 (polygonMode_ == 0 || polyKeys_.ensure(px * 8)) &&
+                 // samples that no draw has written hold no slot (last: freeing a buffer waits for the fill)
+                 ensureFilled(visSlot_, ps * 4, 0xff);
     if (!okAll) {
         setError("device allocation failed");
         return false;
