@@ -476,8 +476,8 @@ struct LdsRec : TriRec {
 // result depends on the order after all.
 //
 // Bound by the latency of an item's chain (claim, item, view, list entries,
-// records, then the window and unit rounds) and by VALU issue: 68 % of its
-// cycles at 1920x1080, 8 samples, 1.3M triangles, 45 % at 1 sample.  Held to the
+// records, then the window and unit rounds) and by VALU issue: 69 % of its
+// cycles at 1920x1080, 8 samples, 1.3M triangles, 46 % at 1 sample.  Held to the
 // registers of five workgroups per compute unit at 1 and 4 samples (at 8 the
 // keys' LDS allows four).  Windows from pixel boxes, one lane per entry, instead of block
 // tests of every entry by two: 105 -> 84 us there, and 78 us with fewer registers; 4.2M
